@@ -431,24 +431,6 @@ __global__ void __launch_bounds__(kBlock) dga_inject_kernel(
     if (threadIdx.x == 0) poy_part[blockIdx.x] = s;
 }
 
-// Second Poynting partial after the E update: 0.5*U_new*fb on h-source edges.
-template <typename T>
-__global__ void __launch_bounds__(kBlock) dga_poynting_kernel(
-    int32_t n_inj, const int32_t* __restrict__ inj_edge, const int8_t* __restrict__ inj_kind,
-    const int32_t* __restrict__ inj_tb, const int32_t* __restrict__ inj_te, const int32_t* __restrict__ term_src,
-    const double* __restrict__ term_w, const double* __restrict__ carr_step, const T* __restrict__ U,
-    double* __restrict__ poy_part) {
-    __shared__ double red[kBlock / kWave];
-    const int32_t i = blockIdx.x * kBlock + threadIdx.x;
-    double poy = 0;
-    if (i < n_inj && inj_kind[i] == 0) {
-        const double v = source_value(inj_tb[i], inj_te[i], term_src, term_w, carr_step);
-        poy = 0.5 * (double)U[inj_edge[i]] * v;
-    }
-    const double s = block_sum(poy, red);
-    if (threadIdx.x == 0) poy_part[blockIdx.x] = s;
-}
-
 // ---- lossy dga: fractional unknowns (D:883-920, tf_dga_frac)
 // Sources of a lossy dga step. h edges as in dga_inject_kernel (curl_f and
 // the first Poynting partial); the other kinds write their value into the
@@ -486,16 +468,18 @@ __global__ void __launch_bounds__(kBlock) frac_inject_kernel(
     if (threadIdx.x == 0) poy_part[blockIdx.x] = s;
 }
 
-// out[i] = X[a[i]] (+ X[b[i]] when b[i] >= 0): U = Mu U_frac, F = Tf F_frac
-// (rows of one or two unit entries).
+// out[e] = X[a[e]] (+ X[b[e]] when b[e] >= 0) for the n entities of list
+// (null: every entity): U = Mu U_frac, F = Tf F_frac (rows of one or two unit
+// entries).
 template <typename T>
-__global__ void __launch_bounds__(kBlock) frac_gather_kernel(int32_t n, const int32_t* __restrict__ a,
+__global__ void __launch_bounds__(kBlock) frac_gather_kernel(int32_t n, const int32_t* __restrict__ list,
+                                                             const int32_t* __restrict__ a,
                                                              const int32_t* __restrict__ b, const T* __restrict__ X,
                                                              T* __restrict__ out) {
     const int32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
-    const int32_t j = b[i];
-    out[i] = j >= 0 ? (T)((double)X[a[i]] + (double)X[j]) : X[a[i]];
+    const int32_t e = list ? list[i] : i, j = b[e];
+    out[e] = j >= 0 ? (T)((double)X[a[e]] + (double)X[j]) : X[a[e]];
 }
 
 // Source work taken by workgroups appended to dga_curl_kernel's grid (after

@@ -160,19 +160,21 @@ __device__ __forceinline__ int lane_id() { return threadIdx.x & (kWave - 1); }
 struct SliceRange {
     int s, end, step;
 };
-__device__ __forceinline__ SliceRange block_slices(int nslices, int band) {
+__device__ __forceinline__ SliceRange block_slices_of(int nslices, int band, int b, int g) {
     const int wpb = (int)(blockDim.x / kWave), w = (int)(threadIdx.x / kWave);
     if (band) {
-        const int g = (int)gridDim.x, b = (int)blockIdx.x;
         const int nx = g < kXcd ? g : kXcd, x = b % nx, i = b / nx;
         const int bx = g / nx + (x < g % nx ? 1 : 0);  // workgroups of part x
         const int x0 = (int)((int64_t)nslices * x / nx), x1 = (int)((int64_t)nslices * (x + 1) / nx);
         return SliceRange{x0 + i * wpb + w, x1, bx * wpb};
     }
-    const int lb = xcd_block();
-    const int s0 = (int)((int64_t)nslices * lb / gridDim.x);
-    const int s1 = (int)((int64_t)nslices * (lb + 1) / gridDim.x);
+    const int lb = xcd_block_of(b, g);
+    const int s0 = (int)((int64_t)nslices * lb / g);
+    const int s1 = (int)((int64_t)nslices * (lb + 1) / g);
     return SliceRange{s0 + w, s1, wpb};
+}
+__device__ __forceinline__ SliceRange block_slices(int nslices, int band) {
+    return block_slices_of(nslices, band, (int)blockIdx.x, (int)gridDim.x);
 }
 
 #define TF_FOR_SLICES(m)                                                               \
@@ -366,21 +368,79 @@ __global__ void __launch_bounds__(kBlock) sell_h_kernel(SellView<T> m, const int
     }
 }
 
+// Rows of K too long for one lane (create_tet: more than kLongRow entries),
+// taken out of the SELL matrix: row[i] holds entries ptr[i] .. ptr[i + 1) of
+// col / val; mask has one 64-bit word per slice, bit l set for a long row.
+template <typename T>
+struct LongRows {
+    int32_t n = 0;
+    const int32_t* row = nullptr;
+    const int32_t* ptr = nullptr;
+    const int32_t* col = nullptr;
+    const T* val = nullptr;
+    const uint64_t* mask = nullptr;
+};
+
 // Lossy dga, one fractional row r per lane (D:888-890, D:916-919):
 // Y[r] = (R X)[r] + sdt (K v)[r], K the row of H / Mp / Mq (N / Tr / Ts)
 // applied to curl_f (curl_u), R the row's old entries (the identity, P_p
 // or R_r, a node-star Q or tet S block) applied to the old U_frac (F_frac);
-// sdt = dt for U, -dt for F. K and R have the same rows.
+// sdt = dt for U, -dt for F. K and R have the same rows. row_out[r] >= 0:
+// the edge whose only entry is r, so out[row_out[r]] = Y[r] as well.
+//
+// The first lr.n workgroups take one long row each: the reference's mirror
+// entries of mixed-class pairs all land in row 0 of H and of Mp (about 5,000
+// entries at 24^3, against 27 in every other row), and as two lanes of the
+// slice loop they were the whole kernel's critical path (168 us at 24^3 in
+// fp64; with a workgroup per long row 14 us, bound by the gather latency of
+// the ordinary rows' two products). Sums of long rows run in fp64.
 template <typename T, int NB, bool W = false>
 __global__ void __launch_bounds__(kBlock) sell_frac_kernel(SellView<T> K, SellView<T> R, const T* __restrict__ v,
-                                                           const T* __restrict__ X, T* __restrict__ Y, double sdt) {
+                                                           const T* __restrict__ X, T* __restrict__ Y, double sdt,
+                                                           LongRows<T> lr, const int32_t* __restrict__ row_out,
+                                                           T* __restrict__ out) {
     const int lane = lane_id();
-    TF_FOR_SLICES(K) {
-        const int s = sr_.s;
+    if ((int)blockIdx.x < lr.n) {
+        __shared__ double red[kBlock / kWave];
+        const int32_t r = lr.row[blockIdx.x], e1 = lr.ptr[blockIdx.x + 1];
+        double kv = 0;
+        constexpr int U = 8;  // entries a thread keeps in flight
+        for (int32_t k = lr.ptr[blockIdx.x] + (int32_t)threadIdx.x; k < e1; k += U * kBlock) {
+            int32_t ci[U];
+            T vi[U], gi[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int32_t q = min(k + u * kBlock, e1 - 1);  // clamped: inside the row
+                ci[u] = lr.col[q];
+                vi[u] = lr.val[q];
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) gi[u] = v[ci[u]];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (k + u * kBlock < e1) kv += (double)vi[u] * (double)gi[u];
+        }
+        kv = block_sum(kv, red);
+        if (threadIdx.x < kWave) {
+            const double rx = sell_dot<T, NB, W>(R, r / kSlice, r % kSlice, [&](int32_t j) { return X[j]; });
+            if (threadIdx.x == 0) {
+                Y[r] = (T)(rx + sdt * kv);
+                if (row_out && row_out[r] >= 0) out[row_out[r]] = (T)(rx + sdt * kv);
+            }
+        }
+        return;
+    }
+    for (SliceRange sr = block_slices_of(K.nslices, K.band, (int)blockIdx.x - lr.n, (int)gridDim.x - lr.n);
+         sr.s < sr.end; sr.s += sr.step) {
+        const int s = sr.s;
         const double kv = sell_dot<T, NB, W>(K, s, lane, [&](int32_t j) { return v[j]; });
         const double rx = sell_dot<T, NB, W>(R, s, lane, [&](int32_t j) { return X[j]; });
         const int32_t r = s * kSlice + lane;
-        if (r < K.nrows) Y[r] = (T)(rx + sdt * kv);
+        if (r < K.nrows && !(lr.n && (lr.mask[s] >> lane & 1))) {
+            const T y = (T)(rx + sdt * kv);
+            Y[r] = y;
+            if (row_out && row_out[r] >= 0) out[row_out[r]] = y;
+        }
     }
 }
 

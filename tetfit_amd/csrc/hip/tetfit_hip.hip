@@ -46,6 +46,11 @@ static_assert(kCgPartA <= kMaxPart && kCgPartB <= kMaxPart && kCgPartC <= kMaxPa
 // within windows of this many rows, so the 64 rows of a slice pad little.
 constexpr int kSigma = 1024;
 constexpr int kSpmvCap = 8192;   // blocks of the other SELL kernels
+// Rows of a lossy dga operator with more entries than this leave the SELL
+// matrix and take a workgroup each (LongRows): tet rows hold 7-27 entries, a
+// lane walks about 0.3 us per batch of 8, so 128 entries cost a lane about as
+// much as the launch itself.
+constexpr int kLongRow = 128;
 
 // Carrier of Source::Compute in long double (Source.hpp:316-327); 0 for t<0.
 double carrier_value(const tf_source& s, double t) {
@@ -250,6 +255,18 @@ struct tf_ctx {
     DevBuf mu_a, mu_b, tf_a, tf_b, fslot, uf[2], ff[2];
     int fcur = 0;
     int32_t nU = 0, nF = 0, q0 = 0, q1 = 0;
+    // long rows of Ku / Kf (LongRows); edge (face) whose only entry is the
+    // row (u_out, f_out: -1 none) and the entities with other rows (u_two,
+    // f_two: gathered after the update); f_plain: Rf = I and Tf a permutation,
+    // F then steps in place with N = Kf's rows in face order (fKf)
+    struct Long {
+        int32_t n = 0;
+        DevBuf row, ptr, col, val, mask;
+    };
+    Long lu, lf;
+    DevBuf u_out, f_out, u_two, f_two;
+    int32_t n_u_two = 0, n_f_two = 0;
+    bool f_plain = false;
     std::vector<int32_t> h_mu_a, h_mu_b, h_tf_a, h_tf_b;
     DevBuf loss_part;            // per step and block: U_old.SigMat U_old partials of a run
     int64_t loss_cap = 0;
@@ -344,6 +361,7 @@ struct tf_ctx {
         DevBuf carr, poy;
     };
     StepGraph sg;
+    int sg_fcur = 0;  // lossy dga: fcur when sg was captured
     bool use_graphs = true;
 
     // profiling
@@ -375,7 +393,8 @@ size_t tf_ctx::device_bytes() const {
                            &h_edge, &curl_f, &curl_u, &free_edge, &edge_row, &dir_edge, &dir_new, &fb, &pre, &x, &r, &rs0, &rs1, &z,
                            &p0, &p1, &q, &r0, &hx1, &hx2, &dx, &rr0part, &cg_part, &cg_state, &inj_edge, &inj_kind, &inj_tb, &inj_te,
                            &term_src, &term_w, &carr, &probes, &samples, &eser, &epart, &poy, &row_dt_h, &row_dt_f,
-                           &mu_a, &mu_b, &tf_a, &tf_b, &fslot, &row_dt_cg, &bt_inst, &bt_s0, &bt_s1, &bt_w0, &bt_w1, &uf[0], &uf[1], &ff[0], &ff[1], &U_older, &fw, &fw2};
+                           &mu_a, &mu_b, &tf_a, &tf_b, &fslot, &row_dt_cg, &bt_inst, &bt_s0, &bt_s1, &bt_w0, &bt_w1, &uf[0], &uf[1], &ff[0], &ff[1], &u_out, &f_out, &u_two, &f_two,
+                           &lu.row, &lu.ptr, &lu.col, &lu.val, &lu.mask, &lf.row, &lf.ptr, &lf.col, &lf.val, &lf.mask, &U_older, &fw, &fw2};
     for (auto b : all) s += b->bytes;
     const Csr32* cs[] = {&Ct};
     for (auto c : cs) s += c->ptr.bytes + c->col.bytes + c->val.bytes + c->sg.bytes;
@@ -422,8 +441,9 @@ std::vector<int64_t> sell_layout(const tf_csr& c) {
     return sptr;
 }
 
+// windows: whether the four-window column form may be used.
 template <class T>
-void upload_sell(Sell& d, const tf_csr& c, bool values) {
+void upload_sell(Sell& d, const tf_csr& c, bool values, bool windows = true) {
     d.nrows = c.nrows;
     d.nnz = c.nnz;
     d.nslices = (c.nrows + kSlice - 1) / kSlice;
@@ -434,7 +454,8 @@ void upload_sell(Sell& d, const tf_csr& c, bool values) {
     std::vector<int32_t> col(d.entries, 0);
     std::vector<T> val(values ? d.entries : 0, (T)0);
     std::vector<int8_t> sg(values ? 0 : d.entries, 0);
-    for (int32_t s = 0; s < d.nslices; ++s) {
+    par_chunks(d.nslices, 1024, [&](int64_t lo, int64_t hi) {
+      for (int32_t s = (int32_t)lo; s < (int32_t)hi; ++s) {
         const int64_t w = (sptr[s + 1] - sptr[s]) / kSlice;
         // rows without entries (and lanes past the last row) pad with a column
         // the slice already uses, so that padding does not widen its span
@@ -457,7 +478,8 @@ void upload_sell(Sell& d, const tf_csr& c, bool values) {
                 }
             }
         }
-    }
+      }
+    });
     upload(d.sptr, sptr);
     upload(d.col, col);
     if (values) upload(d.val, val);
@@ -475,49 +497,60 @@ void upload_sell(Sell& d, const tf_csr& c, bool values) {
     const bool force32 = env_on("TETFIT_SELL_COL32");
     std::vector<int32_t> cb(std::max(d.nslices, 1), 0);
     bool fits = !force32 && !env_on("TETFIT_SELL_WIN");
-    for (int32_t s = 0; s < d.nslices && fits; ++s) {
-        int32_t lo = INT32_MAX, hi = 0;
-        for (int64_t o = sptr[s]; o < sptr[s + 1]; ++o) { lo = std::min(lo, col[o]); hi = std::max(hi, col[o]); }
-        if (sptr[s + 1] == sptr[s]) lo = hi = 0;
-        cb[s] = lo;
-        fits = (int64_t)hi - lo <= 65535;
-    }
+    std::atomic<bool> ok{fits};
+    par_chunks(d.nslices, 1024, [&](int64_t s0, int64_t s1) {
+        for (int64_t s = s0; s < s1 && ok; ++s) {
+            int32_t lo = INT32_MAX, hi = 0;
+            for (int64_t o = sptr[s]; o < sptr[s + 1]; ++o) { lo = std::min(lo, col[o]); hi = std::max(hi, col[o]); }
+            if (sptr[s + 1] == sptr[s]) lo = hi = 0;
+            cb[s] = lo;
+            if ((int64_t)hi - lo > 65535) ok = false;
+        }
+    });
+    fits = ok;
     std::vector<uint16_t> c16;
     if (fits) {
         c16.assign(std::max<int64_t>(d.entries, 1), 0);
         for (int32_t s = 0; s < d.nslices; ++s)
             for (int64_t o = sptr[s]; o < sptr[s + 1]; ++o) c16[o] = (uint16_t)(col[o] - cb[s]);
-    } else if (!force32) {
+    } else if (!force32 && windows) {
         // windows: greedy over the slice's sorted columns, each window opening
         // at the smallest column not yet covered
         cb.assign(4 * std::max(d.nslices, 1), 0);
         std::vector<uint8_t> nwin(std::max(d.nslices, 1), 0);
-        fits = true;
-        std::vector<int32_t> cs;
-        for (int32_t s = 0; s < d.nslices && fits; ++s) {
-            cs.assign(col.begin() + sptr[s], col.begin() + sptr[s + 1]);
-            std::sort(cs.begin(), cs.end());
-            int nw = 0;
-            for (size_t k = 0; k < cs.size();) {
-                if (nw == 4) { fits = false; break; }
-                const int32_t b = cs[k];
-                cb[4 * s + nw++] = b;
-                while (k < cs.size() && (int64_t)cs[k] - b <= 16383) ++k;
+        ok = true;
+        par_chunks(d.nslices, 1024, [&](int64_t lo, int64_t hi) {
+            std::vector<int32_t> cs;
+            for (int64_t s = lo; s < hi && ok; ++s) {
+                cs.assign(col.begin() + sptr[s], col.begin() + sptr[s + 1]);
+                std::sort(cs.begin(), cs.end());
+                int nw = 0;
+                for (size_t k = 0; k < cs.size();) {
+                    if (nw == 4) { ok = false; break; }
+                    const int32_t b = cs[k];
+                    cb[4 * s + nw++] = b;
+                    while (k < cs.size() && (int64_t)cs[k] - b <= 16383) ++k;
+                }
+                nwin[s] = (uint8_t)nw;
             }
-            nwin[s] = (uint8_t)nw;
-        }
+        });
+        fits = ok;
         if (fits) {
             c16.assign(std::max<int64_t>(d.entries, 1), 0);
-            for (int32_t s = 0; s < d.nslices; ++s)
-                for (int64_t o = sptr[s]; o < sptr[s + 1]; ++o) {
-                    // the last opened window whose base is <= the column; the
-                    // windows are disjoint and cover every column of the slice
-                    int w = nwin[s] - 1;
-                    while (w > 0 && cb[4 * s + w] > col[o]) --w;
-                    const int64_t off = (int64_t)col[o] - cb[4 * s + w];
-                    if (off < 0 || off > 16383) throw std::logic_error("SELL column window");
-                    c16[o] = (uint16_t)(w << 14 | off);
-                }
+            ok = true;
+            par_chunks(d.nslices, 1024, [&](int64_t lo, int64_t hi) {
+                for (int64_t s = lo; s < hi; ++s)
+                    for (int64_t o = sptr[s]; o < sptr[s + 1]; ++o) {
+                        // the last opened window whose base is <= the column; the
+                        // windows are disjoint and cover every column of the slice
+                        int w = nwin[s] - 1;
+                        while (w > 0 && cb[4 * s + w] > col[o]) --w;
+                        const int64_t off = (int64_t)col[o] - cb[4 * s + w];
+                        if (off < 0 || off > 16383) ok = false;
+                        c16[o] = (uint16_t)(w << 14 | off);
+                    }
+            });
+            if (!ok) throw std::logic_error("SELL column window");
             d.cwin = true;
         }
     }
@@ -1045,6 +1078,77 @@ void residual_operator(const tf_dga_ops& d, double dt, const std::vector<int32_t
     o.v.val = o.val.data();
 }
 
+// Uploads a K operator of lossy dga: rows of more than kLongRow entries into
+// l, the others into the SELL matrix d (where a long row is empty).
+template <class T>
+void upload_frac_k(Sell& d, tf_ctx::Long& l, const tf_csr& k) {
+    std::vector<int32_t> row, ptr(1, 0), col;
+    std::vector<T> val;
+    CsrBuf o;
+    o.rp.assign(1, 0);
+    o.rp.reserve((size_t)k.nrows + 1);
+    o.col.reserve(k.nnz);
+    o.val.reserve(k.nnz);
+    for (int32_t r = 0; r < k.nrows; ++r) {
+        const int64_t b = k.rowptr[r], e = k.rowptr[r + 1];
+        if (e - b > kLongRow) {
+            if ((int64_t)col.size() + (e - b) > INT32_MAX) throw std::runtime_error("fractional operator too large");
+            row.push_back(r);
+            col.insert(col.end(), k.col + b, k.col + e);
+            for (int64_t q = b; q < e; ++q) val.push_back((T)k.val[q]);
+            ptr.push_back((int32_t)col.size());
+        } else {
+            o.col.insert(o.col.end(), k.col + b, k.col + e);
+            o.val.insert(o.val.end(), k.val + b, k.val + e);
+        }
+        o.rp.push_back((int64_t)o.col.size());
+    }
+    o.v = k;
+    o.v.nnz = o.rp.back();
+    o.v.rowptr = o.rp.data();
+    o.v.col = o.col.data();
+    o.v.val = o.val.data();
+    // windowed columns bring the wide-mesh kernels with their non-temporal
+    // loads, which only an operator beyond the 256 MB Infinity Cache gains
+    // from (24^3, 27 MB: sell_frac 15.5 us windowed, 14.3 us with int32 columns)
+    const bool big = k.nnz * (int64_t)(sizeof(T) + 4) > ((int64_t)256 << 20);
+    const char* win = std::getenv("TETFIT_SELL_WIN");
+    upload_sell<T>(d, o.v, true, big || (win && *win && std::strcmp(win, "0") != 0));
+    l.n = (int32_t)row.size();
+    if (!l.n) return;
+    std::vector<uint64_t> mask(std::max(d.nslices, 1), 0);
+    for (int32_t r : row) mask[r / kSlice] |= (uint64_t)1 << (r % kSlice);
+    upload(l.row, row);
+    upload(l.ptr, ptr);
+    upload(l.col, col);
+    upload(l.val, val);
+    upload(l.mask, mask);
+}
+template <class T>
+LongRows<T> long_rows(const tf_ctx::Long& l) {
+    return LongRows<T>{l.n,           l.row.as<int32_t>(), l.ptr.as<int32_t>(),
+                       l.col.as<int32_t>(), l.val.as<T>(),  l.mask.as<uint64_t>()};
+}
+
+// Where the update of nx fractional rows writes the entities' values: out[r]
+// = the entity whose only entry is r and which no other entity reads (-1:
+// none); the others are listed in `two` and gathered afterwards.
+void frac_outputs(int32_t nx, const std::vector<int32_t>& a, const std::vector<int32_t>& b, DevBuf& out, DevBuf& two,
+                  int32_t& n_two) {
+    std::vector<int32_t> uses(std::max(nx, 1), 0), o(std::max(nx, 1), -1), t;
+    for (size_t e = 0; e < a.size(); ++e) {
+        ++uses[a[e]];
+        if (b[e] >= 0) ++uses[b[e]];
+    }
+    for (size_t e = 0; e < a.size(); ++e) {
+        if (b[e] < 0 && uses[a[e]] == 1) o[a[e]] = (int32_t)e;
+        else t.push_back((int32_t)e);
+    }
+    n_two = (int32_t)t.size();
+    upload(out, o);
+    upload(two, t);
+}
+
 template <class T>
 void create_tet(tf_ctx* c, const tf_problem* p, const std::vector<int32_t>* batch_rows) {
     const tf_dga_ops& d = p->dga;
@@ -1076,10 +1180,8 @@ void create_tet(tf_ctx* c, const tf_problem* p, const std::vector<int32_t>* batc
         c->q1 = c->q0 + fr.q_size;
         if (fr.Ru.nrows != c->nU || fr.Rf.nrows != c->nF || fr.Mu.nrows != E || fr.Tf.nrows != F)
             throw std::runtime_error("inconsistent fractional operators");
-        upload_sell<T>(c->fKu, fr.Ku, true);
+        upload_frac_k<T>(c->fKu, c->lu, fr.Ku);
         upload_sell<T>(c->fRu, fr.Ru, true);
-        upload_sell<T>(c->fKf, fr.Kf, true);
-        upload_sell<T>(c->fRf, fr.Rf, true);
         auto two = [](const tf_csr& m, int32_t ncols, std::vector<int32_t>& a, std::vector<int32_t>& b) {
             a.assign(m.nrows, -1);
             b.assign(m.nrows, -1);
@@ -1098,8 +1200,29 @@ void create_tet(tf_ctx* c, const tf_problem* p, const std::vector<int32_t>* batc
         two(fr.Tf, c->nF, c->h_tf_a, c->h_tf_b);
         upload(c->mu_a, c->h_mu_a);
         upload(c->mu_b, c->h_mu_b);
-        upload(c->tf_a, c->h_tf_a);
-        upload(c->tf_b, c->h_tf_b);
+        frac_outputs(c->nU, c->h_mu_a, c->h_mu_b, c->u_out, c->u_two, c->n_u_two);
+        // without magnetic loss F_frac is F in another order: Rf the identity
+        // and Tf a permutation
+        std::vector<uint8_t> seen(std::max(c->nF, 1), 0);
+        c->f_plain = c->nF == F && fr.Rf.nnz == F;
+        for (int32_t f = 0; f < F && c->f_plain; ++f) {
+            const int32_t a = c->h_tf_a[f];
+            c->f_plain = c->h_tf_b[f] < 0 && !seen[a] && fr.Rf.rowptr[f] == f && fr.Rf.col[f] == f && fr.Rf.val[f] == 1.0;
+            seen[a] = 1;
+        }
+        for (int32_t r = 0; r < fr.Kf.nrows && c->f_plain; ++r)
+            c->f_plain = fr.Kf.rowptr[r + 1] - fr.Kf.rowptr[r] <= kLongRow;
+        if (c->f_plain) {
+            CsrBuf nb;
+            select_rows(fr.Kf, c->h_tf_a.data(), F, nullptr, nb);
+            upload_sell<T>(c->fKf, nb.v, true);
+        } else {
+            upload_frac_k<T>(c->fKf, c->lf, fr.Kf);
+            upload_sell<T>(c->fRf, fr.Rf, true);
+            upload(c->tf_a, c->h_tf_a);
+            upload(c->tf_b, c->h_tf_b);
+            frac_outputs(c->nF, c->h_tf_a, c->h_tf_b, c->f_out, c->f_two, c->n_f_two);
+        }
         std::vector<int32_t> sl(fr.slot, fr.slot + E);
         for (int32_t v : sl)
             if (v < -1 || v >= c->nU) throw std::runtime_error("fractional slot out of range");
@@ -1110,7 +1233,7 @@ void create_tet(tf_ctx* c, const tf_problem* p, const std::vector<int32_t>* batc
             if (d.edge_class[e] == 4 && sl[e] >= 0) u0[sl[e]] = (T)c->h_fixed_value[e];
         for (int k = 0; k < 2; ++k) {
             upload(c->uf[k], u0);
-            zero_field<T>(c->ff[k], std::max(c->nF, 1), c->stream);
+            if (!c->f_plain) zero_field<T>(c->ff[k], std::max(c->nF, 1), c->stream);
         }
         c->fcur = 0;
     } else if (p->method == TF_METHOD_DGA) {
@@ -1496,12 +1619,12 @@ bool graph_steps(const tf_ctx* c) {
 }
 
 // Captures kGraphSteps calls of step(local step, carrier row, Poynting slot)
-// into the context's graph (once), then runs steps [k0, k0 + m) of the
-// current tf_run in chunks of kGraphSteps by replay; per_step = Poynting
+// into the context's graph (once), then runs steps [first_k, first_k + m) of
+// the current tf_run in chunks of kGraphSteps by replay; per_step = Poynting
 // partials per step. Returns the number of steps run (a multiple of
 // kGraphSteps); the caller runs the rest with ordinary launches.
 template <class Step>
-int64_t run_graph_chunks(tf_ctx* c, int64_t m, int per_step, Step step) {
+int64_t run_graph_chunks(tf_ctx* c, int64_t first_k, int64_t m, int per_step, Step step) {
     const int64_t chunks = m / kGraphSteps;
     if (chunks == 0) return 0;
     const size_t ns = std::max<size_t>(c->src.size(), 1);
@@ -1522,7 +1645,7 @@ int64_t run_graph_chunks(tf_ctx* c, int64_t m, int per_step, Step step) {
         TF_HIP(hipGraphInstantiate(&c->sg.exec, c->sg.graph, nullptr, nullptr, 0));
     }
     for (int64_t q = 0; q < chunks; ++q) {
-        const int64_t k0 = q * kGraphSteps;
+        const int64_t k0 = first_k + q * kGraphSteps;
         // carrier rows k0 .. k0 + kGraphSteps of this run (row 0 = the step before)
         TF_HIP(hipMemcpyAsync(c->sg.carr.p, c->carr.as<double>() + (size_t)k0 * ns,
                               (kGraphSteps + 1) * ns * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
@@ -1563,7 +1686,7 @@ void run_fit(tf_ctx* c, int64_t first, int64_t n, tf_stats* st) {
                      c->fit_grid ? c->fh_code.as<uint16_t>() : nullptr, c->grid, c->U.as<T>(), c->Fv.as<T>(),
                      c->B.as<T>(), c->dt);
     };
-    const int64_t g = graph_steps(c) ? run_graph_chunks(c, n, sp_blocks, [&](int, const double* cs, double* poy) {
+    const int64_t g = graph_steps(c) ? run_graph_chunks(c, 0, n, sp_blocks, [&](int, const double* cs, double* poy) {
         step(cs, poy);
     }) : 0;
     for (int64_t k = g; k < n; ++k) {
@@ -1588,86 +1711,6 @@ void run_fit(tf_ctx* c, int64_t first, int64_t n, tf_stats* st) {
     st->steps_done += n;
 }
 
-// Lossy dga (D:810-939 with edge classes 2/3 and face classes 2/3): one
-// step is curl_f = Ct F with the h sources, the boundary values and e
-// sources into U_frac, U_frac' = Ru U_frac + dt Ku curl_f, U = Mu U_frac',
-// the Poynting partials, curl_u = C U with the B update, F_frac' = Rf F_frac
-// - dt Kf curl_u, F = Tf F_frac'; the two U_frac (F_frac) buffers swap
-// roles every step. Launched from the host step by step (no graph).
-template <class T>
-void run_dga_frac(tf_ctx* c, int64_t first, int64_t n, tf_stats* st) {
-    const int inj_blocks = c->n_inj ? blocks_for(c->n_inj) : 0;
-    const size_t ns = std::max<size_t>(c->src.size(), 1);
-    if (inj_blocks && c->poy_cap < 2 * n * inj_blocks) {
-        c->poy.alloc(2 * n * inj_blocks * sizeof(double));
-        c->poy_cap = 2 * n * inj_blocks;
-    }
-    auto inject = [&](const double* cs, double* poy, int init) {
-        if (!c->n_inj) return;
-        launch_timed(c, "frac_inject_kernel", frac_inject_kernel<T>, inj_blocks, c->n_inj, c->inj_edge.as<int32_t>(),
-                     c->inj_kind.as<int8_t>(), c->inj_tb.as<int32_t>(), c->inj_te.as<int32_t>(),
-                     c->term_src.as<int32_t>(), c->term_w.as<double>(), cs, c->curl_f.as<T>(),
-                     (const T*)c->U.as<T>(), c->uf[c->fcur].as<T>(), c->fslot.as<int32_t>(),
-                     c->mu_a.as<int32_t>(), c->mu_b.as<int32_t>(), c->q0, c->q1, poy, init);
-    };
-    auto gather_u = [&]() {
-        launch_timed(c, "frac_gather_kernel", frac_gather_kernel<T>, blocks_for(c->E), c->E, c->mu_a.as<int32_t>(),
-                     c->mu_b.as<int32_t>(), (const T*)c->uf[c->fcur].as<T>(), c->U.as<T>());
-    };
-    if (!c->initial_done && first == 1) {
-        // the pass before the loop (D:726-790), then the export at t = 0
-        inject(c->carr.as<double>(), c->poy.as<double>(), 1);
-        gather_u();
-        if (want_sample(c, 0, 0.0)) sample<T>(c, 0.0);
-    }
-    c->initial_done = true;
-    const int gb_ct = tuned_blocks(c, TK_CT, c->sCt, kSpmvCap);
-    const int gb_u = sell_blocks(c->fKu, kSpmvCap), gb_f = sell_blocks(c->fKf, kSpmvCap);
-    for (int64_t k = 0; k < n; ++k) {
-        const int64_t i = first + k;
-        const double t = (double)i * c->dt;
-        const double* cs = c->carr.as<double>() + (k + 1) * ns;
-        double* poy = c->poy.as<double>() + 2 * k * inj_blocks;
-        TF_LAUNCH_TIMED(c, "sell_ct_kernel", c->tune[TK_CT].unroll, sell_ct_kernel, T, gb_ct,
-                        tuned_view(c, TK_CT, c->sCt.signs()), c->Fv.as<T>(), c->curl_f.as<T>());
-        inject(cs, poy, 0);
-        const int nx = c->fcur ^ 1;
-        if (c->nU > 0)
-            TF_LAUNCH_TIMED(c, "sell_frac_kernel", 8, sell_frac_kernel, T, gb_u, c->fKu.vals<T>(), c->fRu.vals<T>(),
-                            (const T*)c->curl_f.as<T>(), (const T*)c->uf[c->fcur].as<T>(), c->uf[nx].as<T>(), c->dt);
-        launch_timed(c, "frac_gather_kernel", frac_gather_kernel<T>, blocks_for(c->E), c->E, c->mu_a.as<int32_t>(),
-                     c->mu_b.as<int32_t>(), (const T*)c->uf[nx].as<T>(), c->U.as<T>());
-        if (c->n_inj)
-            launch_timed(c, "dga_poynting_kernel", dga_poynting_kernel<T>, inj_blocks, c->n_inj,
-                         c->inj_edge.as<int32_t>(), c->inj_kind.as<int8_t>(), c->inj_tb.as<int32_t>(),
-                         c->inj_te.as<int32_t>(), c->term_src.as<int32_t>(), c->term_w.as<double>(), cs,
-                         (const T*)c->U.as<T>(), poy + inj_blocks);
-        launch_timed(c, "dga_curl_kernel", dga_curl_kernel<T>, blocks_for(c->F), c->F, c->c_col.as<int32_t>(),
-                     c->c_fixed_signs ? nullptr : c->c_sg.as<int8_t>(), (const T*)c->U.as<T>(), c->curl_u.as<T>(),
-                     c->B.as<T>(), c->dt, (const double*)nullptr, (const CgState*)nullptr, CurlSources<T>{});
-        if (c->nF > 0)
-            TF_LAUNCH_TIMED(c, "sell_frac_kernel", 8, sell_frac_kernel, T, gb_f, c->fKf.vals<T>(), c->fRf.vals<T>(),
-                            (const T*)c->curl_u.as<T>(), (const T*)c->ff[c->fcur].as<T>(), c->ff[nx].as<T>(), -c->dt);
-        launch_timed(c, "frac_gather_kernel", frac_gather_kernel<T>, blocks_for(c->F), c->F, c->tf_a.as<int32_t>(),
-                     c->tf_b.as<int32_t>(), (const T*)c->ff[nx].as<T>(), c->Fv.as<T>());
-        c->fcur = nx;
-        if (want_sample(c, i, t)) sample<T>(c, t);
-        if (c->profiling && (k & 63) == 63) ev_flush(c);
-    }
-    TF_HIP(hipGetLastError());
-    std::vector<double> part((size_t)2 * n * std::max(inj_blocks, 1), 0.0);
-    if (inj_blocks)
-        TF_HIP(hipMemcpyAsync(part.data(), c->poy.p, 2 * n * inj_blocks * sizeof(double), hipMemcpyDeviceToHost,
-                              c->stream));
-    TF_HIP(hipStreamSynchronize(c->stream));
-    for (int64_t k = 0; k < n; ++k) {
-        double sum = 0;
-        for (int b = 0; b < 2 * inj_blocks; ++b) sum += part[2 * k * inj_blocks + b];
-        c->poynting.push_back(sum);
-    }
-    st->steps_done += n;
-}
-
 // The context's injection items as dga_curl_kernel's appended source work
 // (mode 1: dga second Poynting half; mode 2: gfdtd / fem sources).
 template <class T>
@@ -1688,6 +1731,100 @@ CurlSources<T> curl_sources(tf_ctx* c, int mode, const double* carr_step, const 
     s.delta = c->fem ? 1 : 0;
     s.poy_part = poy;
     return s;
+}
+
+// Lossy dga (D:810-939 with edge classes 2/3 and face classes 2/3): one
+// step is curl_f = Ct F with the h sources, the boundary values and e
+// sources into U_frac, U_frac' = Ru U_frac + dt Ku curl_f with U = Mu U_frac'
+// (written by the update for the edges of one entry, gathered after it for
+// the others), curl_u = C U with the B update and the second Poynting half,
+// F_frac' = Rf F_frac - dt Kf curl_u, F = Tf F_frac' (in place when F_frac is
+// F in another order, f_plain); the two U_frac (F_frac) buffers swap roles
+// every step.
+template <class T>
+void run_dga_frac(tf_ctx* c, int64_t first, int64_t n, tf_stats* st) {
+    const int inj_blocks = c->n_inj ? blocks_for(c->n_inj) : 0;
+    const size_t ns = std::max<size_t>(c->src.size(), 1);
+    if (inj_blocks && c->poy_cap < 2 * n * inj_blocks) {
+        c->poy.alloc(2 * n * inj_blocks * sizeof(double));
+        c->poy_cap = 2 * n * inj_blocks;
+    }
+    auto inject = [&](const double* cs, double* poy, int init) {
+        if (!c->n_inj) return;
+        launch_timed(c, "frac_inject_kernel", frac_inject_kernel<T>, inj_blocks, c->n_inj, c->inj_edge.as<int32_t>(),
+                     c->inj_kind.as<int8_t>(), c->inj_tb.as<int32_t>(), c->inj_te.as<int32_t>(),
+                     c->term_src.as<int32_t>(), c->term_w.as<double>(), cs, c->curl_f.as<T>(),
+                     (const T*)c->U.as<T>(), c->uf[c->fcur].as<T>(), c->fslot.as<int32_t>(),
+                     c->mu_a.as<int32_t>(), c->mu_b.as<int32_t>(), c->q0, c->q1, poy, init);
+    };
+    auto gather = [&](int32_t cnt, const DevBuf* list, const DevBuf& a, const DevBuf& b, const DevBuf& x, DevBuf& out) {
+        if (cnt <= 0) return;
+        launch_timed(c, "frac_gather_kernel", frac_gather_kernel<T>, blocks_for(cnt), cnt,
+                     list ? (const int32_t*)list->as<int32_t>() : (const int32_t*)nullptr, a.as<int32_t>(),
+                     b.as<int32_t>(), (const T*)x.as<T>(), out.as<T>());
+    };
+    if (!c->initial_done && first == 1) {
+        // the pass before the loop (D:726-790), then the export at t = 0
+        inject(c->carr.as<double>(), c->poy.as<double>(), 1);
+        gather(c->E, nullptr, c->mu_a, c->mu_b, c->uf[c->fcur], c->U);
+        if (want_sample(c, 0, 0.0)) sample<T>(c, 0.0);
+    }
+    c->initial_done = true;
+    const int gb_ct = tuned_blocks(c, TK_CT, c->sCt, kSpmvCap);
+    const int gb_u = sell_blocks(c->fKu, kSpmvCap) + c->lu.n, gb_f = sell_blocks(c->fKf, kSpmvCap) + c->lf.n;
+    auto step = [&](const double* cs, double* poy) {
+        TF_LAUNCH_TIMED(c, "sell_ct_kernel", c->tune[TK_CT].unroll, sell_ct_kernel, T, gb_ct,
+                        tuned_view(c, TK_CT, c->sCt.signs()), c->Fv.as<T>(), c->curl_f.as<T>());
+        inject(cs, poy, 0);
+        const int nx = c->fcur ^ 1;
+        if (c->nU > 0)
+            TF_LAUNCH_TIMED(c, "sell_frac_kernel", 8, sell_frac_kernel, T, gb_u, c->fKu.vals<T>(), c->fRu.vals<T>(),
+                            (const T*)c->curl_f.as<T>(), (const T*)c->uf[c->fcur].as<T>(), c->uf[nx].as<T>(), c->dt,
+                            long_rows<T>(c->lu), (const int32_t*)c->u_out.as<int32_t>(), c->U.as<T>());
+        gather(c->n_u_two, &c->u_two, c->mu_a, c->mu_b, c->uf[nx], c->U);
+        const CurlSources<T> py = c->n_inj ? curl_sources<T>(c, 1, cs, nullptr, poy + inj_blocks) : CurlSources<T>{};
+        launch_timed(c, "dga_curl_kernel", dga_curl_kernel<T>, blocks_for(c->F) + inj_blocks, c->F,
+                     c->c_col.as<int32_t>(), c->c_fixed_signs ? nullptr : c->c_sg.as<int8_t>(), (const T*)c->U.as<T>(),
+                     c->curl_u.as<T>(), c->B.as<T>(), c->dt, (const double*)nullptr, (const CgState*)nullptr, py);
+        if (c->f_plain) {
+            TF_LAUNCH_TIMED(c, "sell_n_kernel", 8, sell_n_kernel, T, gb_f, c->fKf.vals<T>(), c->curl_u.as<T>(),
+                            c->Fv.as<T>(), c->dt, 0, nullptr, nullptr);
+        } else if (c->nF > 0) {
+            TF_LAUNCH_TIMED(c, "sell_frac_kernel", 8, sell_frac_kernel, T, gb_f, c->fKf.vals<T>(), c->fRf.vals<T>(),
+                            (const T*)c->curl_u.as<T>(), (const T*)c->ff[c->fcur].as<T>(), c->ff[nx].as<T>(), -c->dt,
+                            long_rows<T>(c->lf), (const int32_t*)c->f_out.as<int32_t>(), c->Fv.as<T>());
+            gather(c->n_f_two, &c->f_two, c->tf_a, c->tf_b, c->ff[nx], c->Fv);
+        }
+        c->fcur = nx;
+    };
+    // a captured chunk is an even number of steps that start at one of the
+    // two buffers: a run that starts at the other one steps once from the host
+    int64_t h = 0;
+    auto host_step = [&](int64_t k) {
+        const int64_t i = first + k;
+        const double t = (double)i * c->dt;
+        step(c->carr.as<double>() + (k + 1) * ns, c->poy.as<double>() + 2 * k * inj_blocks);
+        if (want_sample(c, i, t)) sample<T>(c, t);
+        if (c->profiling && (k & 63) == 63) ev_flush(c);
+    };
+    if (graph_steps(c)) {
+        if (c->sg.exec && c->sg_fcur != c->fcur && n > 0) host_step(h++);
+        if (!c->sg.exec) c->sg_fcur = c->fcur;
+        h += run_graph_chunks(c, h, n - h, 2 * inj_blocks, [&](int, const double* cs, double* poy) { step(cs, poy); });
+    }
+    for (; h < n; ++h) host_step(h);
+    TF_HIP(hipGetLastError());
+    std::vector<double> part((size_t)2 * n * std::max(inj_blocks, 1), 0.0);
+    if (inj_blocks)
+        TF_HIP(hipMemcpyAsync(part.data(), c->poy.p, 2 * n * inj_blocks * sizeof(double), hipMemcpyDeviceToHost,
+                              c->stream));
+    TF_HIP(hipStreamSynchronize(c->stream));
+    for (int64_t k = 0; k < n; ++k) {
+        double sum = 0;
+        for (int b = 0; b < 2 * inj_blocks; ++b) sum += part[2 * k * inj_blocks + b];
+        c->poynting.push_back(sum);
+    }
+    st->steps_done += n;
 }
 
 template <class T>
@@ -1744,7 +1881,7 @@ void run_dga(tf_ctx* c, int64_t first, int64_t n, tf_stats* st) {
         TF_LAUNCH_TIMED(c, "sell_n_kernel", c->tune[TK_N].unroll, sell_n_kernel, T, gb_n,
                         tuned_view(c, TK_N, c->N.vals<T>()), c->curl_u.as<T>(), c->Fv.as<T>(), c->dt, 0, fdt, nullptr);
     };
-    const int64_t g = graph_steps(c) ? run_graph_chunks(c, n, per_step, [&](int, const double* cs, double* poy) {
+    const int64_t g = graph_steps(c) ? run_graph_chunks(c, 0, n, per_step, [&](int, const double* cs, double* poy) {
         step(cs, poy);
     }) : 0;
     for (int64_t k = g; k < n; ++k) {
@@ -3547,7 +3684,7 @@ tf_status tf_write_state(tf_ctx* c, const double* U, const double* F, const doub
                 wr(dst, v.data(), (int64_t)v.size());
             };
             split(c->uf[c->fcur], c->nU, U, c->E, c->h_mu_a, c->h_mu_b);
-            split(c->ff[c->fcur], c->nF, F, c->F, c->h_tf_a, c->h_tf_b);
+            if (!c->f_plain) split(c->ff[c->fcur], c->nF, F, c->F, c->h_tf_a, c->h_tf_b);
         }
         // gfdtd and fem: the next solve's warm start is the written field on
         // the free edges, as after every step (the solution vector is U's
