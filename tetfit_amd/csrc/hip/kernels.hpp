@@ -257,6 +257,27 @@ __device__ __forceinline__ double slot_sum(uint32_t code, const double v[4]) {
     return c;
 }
 
+// Coefficient palette of the grid order: with media that are uniform per
+// region, a kernel's per-item constants (the two coefficients and the 16-bit
+// sign and order code) take few distinct values, so each item stores the
+// 16-bit number of its entry here instead of 2 sizeof(T) + 2 bytes (id 0:
+// not in the main pass). The table (24 bytes an entry in fp64) stays in L1.
+// Both kernels are bound by bytes: an fp64 item moves 26 instead of 42 bytes
+// (E) and, with B stored only where it is read (below), 26 instead of 50 (H).
+template <typename T>
+struct FitPal {
+    T c0, c1;       // E: ca, cb; H: cm, cn
+    uint32_t code;  // slot_sum code, | kStoreB
+};
+constexpr uint32_t kStoreB = 1u << 16;  // H: a probed face, B is stored every step
+
+// id[at[i]] = val[i] (palette ids of faces that become probed or stop to be)
+__global__ void __launch_bounds__(kBlock) set_ids_kernel(int32_t n, const int32_t* __restrict__ at,
+                                                         const uint16_t* __restrict__ val, uint16_t* __restrict__ id) {
+    const int32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) id[at[i]] = val[i];
+}
+
 // E phase (D:1850-1895). The first sp_blocks workgroups take the special
 // items, so that their longer dependent chains (source value, Poynting sum)
 // start with the launch instead of trailing it; the rest cover every edge in
@@ -270,11 +291,13 @@ __device__ __forceinline__ double slot_sum(uint32_t code, const double v[4]) {
 // With code16 (grid order) the main blocks take their edges by slab_item,
 // each edge's faces from its position and its sign and order code from code16
 // (slot_sum); otherwise edges by index order over XCD ranges, faces from the
-// packed face quadruple f4 and the sign byte sg.
+// packed face quadruple f4 and the sign byte sg. With pid (grid order, few
+// distinct coefficients) the code and coefficients come from pal[pid[e]].
 template <typename T>
 __global__ void __launch_bounds__(kBlock) fit_e_kernel(
     int32_t n_edges, int32_t sp_blocks, const uint8_t* __restrict__ sg, const T* __restrict__ ca,
-    const T* __restrict__ cb, const int4* __restrict__ f4, const uint16_t* __restrict__ code16, FitGrid grid,
+    const T* __restrict__ cb, const int4* __restrict__ f4, const uint16_t* __restrict__ code16,
+    const uint16_t* __restrict__ pid, const FitPal<T>* __restrict__ pal, FitGrid grid,
     const T* __restrict__ Fv, T* __restrict__ U,
     int32_t n_sp, const int32_t* __restrict__ sp_edge, const int4* __restrict__ sp_f4,
     const uint8_t* __restrict__ sp_sg, const double* __restrict__ sp_ca, const double* __restrict__ sp_cb,
@@ -283,6 +306,20 @@ __global__ void __launch_bounds__(kBlock) fit_e_kernel(
     const double* __restrict__ carr_step, double* __restrict__ poy_part) {
     const int hb = (int)blockIdx.x;
     if (hb >= sp_blocks) {
+        if (pid) {
+            uint32_t cnt[3];
+            fit_counts(grid, false, cnt);
+            const int32_t e = slab_item(hb - sp_blocks, cnt);
+            if (e < 0) return;
+            const uint32_t id = pid[e];
+            if (id == 0) return;
+            const FitPal<T> q = pal[id];
+            int32_t f[4];
+            fit_edge_slots(grid, (uint32_t)e, f);
+            const double v[4] = {(double)Fv[f[0]], (double)Fv[f[1]], (double)Fv[f[2]], (double)Fv[f[3]]};
+            U[e] = (T)((double)q.c0 * (double)U[e] + (double)q.c1 * slot_sum(q.code, v));
+            return;
+        }
         if (code16) {
             uint32_t cnt[3];
             fit_counts(grid, false, cnt);
@@ -338,13 +375,34 @@ __global__ void __launch_bounds__(kBlock) fit_e_kernel(
 
 // H phase over tbc faces (D:1908-1915): B = cm*F_old - dt*sum s_k U[e_k];
 // F = cn*B with cm = M_mu*fpml, cn = fpml*M_nu, s = curl*(+,-,+,-).
-// code16 / grid as in fit_e_kernel.
+// code16 / pid / grid as in fit_e_kernel. The loop itself never reads B (the
+// update takes F_old): with pid it is stored only where something reads it
+// before the next step overwrites it, on probed faces (kStoreB) every step
+// and on every face with store_b (the run's last step, energy samples).
 template <typename T>
 __global__ void __launch_bounds__(kBlock) fit_h_kernel(int32_t n_faces, const uint8_t* __restrict__ sg,
                                                        const T* __restrict__ cm, const T* __restrict__ cn,
                                                        const int4* __restrict__ e4, const uint16_t* __restrict__ code16,
-                                                       FitGrid grid, const T* __restrict__ U,
-                                                       T* __restrict__ Fv, T* __restrict__ B, double dt) {
+                                                       const uint16_t* __restrict__ pid,
+                                                       const FitPal<T>* __restrict__ pal, int store_b, FitGrid grid,
+                                                       const T* __restrict__ U, T* __restrict__ Fv, T* __restrict__ B,
+                                                       double dt) {
+    if (pid) {
+        uint32_t cnt[3];
+        fit_counts(grid, true, cnt);
+        const int32_t f = slab_item((int)blockIdx.x, cnt);
+        if (f < 0) return;
+        const uint32_t id = pid[f];
+        if (id == 0) return;
+        const FitPal<T> q = pal[id];
+        int32_t e[4];
+        fit_face_slots(grid, (uint32_t)f, e);
+        const double v[4] = {(double)U[e[0]], (double)U[e[1]], (double)U[e[2]], (double)U[e[3]]};
+        const double b = (double)q.c0 * (double)Fv[f] - dt * slot_sum(q.code & 0xFFFFu, v);
+        if (store_b || (q.code & kStoreB)) B[f] = (T)b;
+        Fv[f] = (T)((double)q.c1 * b);
+        return;
+    }
     if (code16) {
         uint32_t cnt[3];
         fit_counts(grid, true, cnt);

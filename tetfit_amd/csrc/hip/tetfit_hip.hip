@@ -20,6 +20,7 @@
 #include <memory>
 #include <string>
 #include <thread>
+#include <unordered_map>
 #include <vector>
 
 #include "common.hpp"
@@ -234,6 +235,12 @@ struct tf_ctx {
     std::vector<int32_t> h_esid, h_fsid;  // reference edge / face -> device position (FIT grid order, tet relabel)
     std::vector<uint16_t> h_fe_code;      // per grid edge: slot map << 8 | signs (0: not in the main pass)
     DevBuf fe_code, fh_code;
+    // coefficient palettes (FitPal), in place of code and coefficient arrays
+    // where few distinct values occur; probed faces carry id + fh_k
+    DevBuf fe_id, fe_pal, fh_id, fh_pal, fh_at, fh_val;
+    std::vector<uint16_t> h_fe_id, h_fh_id;
+    int32_t fh_k = 0;
+    std::vector<int32_t> fh_probed;  // device faces whose id carries kStoreB
     std::vector<double> h_ca_common, h_cb_common;
     DevBuf sp_edge, sp_f4, sp_sg, sp_ca, sp_cb, sp_kind, sp_tb, sp_te;
     int32_t n_sp = 0;
@@ -388,7 +395,7 @@ tf_ctx::~tf_ctx() {
 
 size_t tf_ctx::device_bytes() const {
     size_t s = 0;
-    const DevBuf* all[] = {&U, &Fv, &B, &fit_ep, &fit_nu, &fe_sg, &fe_ca, &fe_cb, &fe_f4, &fh_sg, &fh_cm, &fh_cn, &fh_e4, &fe_code, &fh_code,
+    const DevBuf* all[] = {&U, &Fv, &B, &fit_ep, &fit_nu, &fe_sg, &fe_ca, &fe_cb, &fe_f4, &fh_sg, &fh_cm, &fh_cn, &fh_e4, &fe_code, &fh_code, &fe_id, &fe_pal, &fh_id, &fh_pal, &fh_at, &fh_val,
                            &sp_edge, &sp_f4, &sp_sg, &sp_ca, &sp_cb, &sp_kind, &sp_tb, &sp_te, &c_col, &c_sg,
                            &h_edge, &curl_f, &curl_u, &free_edge, &edge_row, &dir_edge, &dir_new, &fb, &pre, &x, &r, &rs0, &rs1, &z,
                            &p0, &p1, &q, &r0, &hx1, &hx2, &dx, &rr0part, &cg_part, &cg_state, &inj_edge, &inj_kind, &inj_tb, &inj_te,
@@ -920,6 +927,89 @@ bool fit_grid_codes(tf_ctx* c, const tf_fit_ops& f, std::vector<uint16_t>& ecode
     return true;
 }
 
+// Palette of the entities' (code, a, b) triples (device order; bitwise
+// distinct values): id per entity, 0 for code 0. False when there are more
+// than kPalMax: at 161^3 a random medium's E side (every cell its own eps_r)
+// gives one triple per edge and keeps the plain arrays, 42 bytes an edge,
+// while a cavity's holds a few dozen.
+constexpr size_t kPalMax = 32767;
+template <class T>
+bool fit_palette(const std::vector<uint16_t>& code, const std::vector<T>& a, const std::vector<T>& b,
+                 std::vector<uint16_t>& id, std::vector<FitPal<T>>& pal) {
+    struct Key {
+        T a, b;
+        uint32_t code;
+        bool operator==(const Key& o) const {
+            return code == o.code && !std::memcmp(&a, &o.a, sizeof(T)) && !std::memcmp(&b, &o.b, sizeof(T));
+        }
+    };
+    struct Hash {
+        size_t operator()(const Key& k) const {
+            uint64_t x = 0, y = 0;
+            std::memcpy(&x, &k.a, sizeof(T));
+            std::memcpy(&y, &k.b, sizeof(T));
+            uint64_t h = (x ^ (y * 0x9E3779B97F4A7C15ull)) + k.code;
+            h ^= h >> 32;
+            h *= 0x9E3779B97F4A7C15ull;
+            return (size_t)(h ^ (h >> 29));
+        }
+    };
+    std::unordered_map<Key, uint16_t, Hash> seen;
+    id.assign(code.size(), 0);
+    pal.assign(1, FitPal<T>{0, 0, 0});
+    Key last{0, 0, 0};
+    uint16_t last_id = 0;
+    for (size_t i = 0; i < code.size(); ++i) {
+        if (code[i] == 0) continue;
+        const Key k{a[i], b[i], code[i]};
+        if (!(k == last)) {
+            auto it = seen.find(k);
+            if (it == seen.end()) {
+                if (pal.size() > kPalMax) return false;
+                it = seen.emplace(k, (uint16_t)pal.size()).first;
+                pal.push_back(FitPal<T>{k.a, k.b, k.code});
+            }
+            last = k;
+            last_id = it->second;
+        }
+        id[i] = last_id;
+    }
+    return true;
+}
+
+// Marks the faces that the probes read as stored every step (FIT palette).
+void fit_probe_faces(tf_ctx* c, const std::vector<int32_t>& faces) {
+    if (!c->fh_id.p) return;
+    std::vector<int32_t> at;
+    std::vector<uint16_t> val;
+    for (int32_t f : c->fh_probed) {
+        at.push_back(f);
+        val.push_back(c->h_fh_id[f]);
+    }
+    const size_t n_old = at.size();
+    std::vector<int32_t> now = faces;
+    std::sort(now.begin(), now.end());
+    now.erase(std::unique(now.begin(), now.end()), now.end());
+    if (now == c->fh_probed) return;
+    for (int32_t f : now)
+        if (c->h_fh_id[f]) {
+            at.push_back(f);
+            val.push_back((uint16_t)(c->h_fh_id[f] + c->fh_k));
+        }
+    c->fh_probed = now;
+    // two launches in stream order: a face may be in both lists
+    upload(c->fh_at, at);
+    upload(c->fh_val, val);
+    for (int part = 0; part < 2; ++part) {
+        const size_t lo = part ? n_old : 0, n = part ? at.size() - n_old : n_old;
+        if (n)
+            set_ids_kernel<<<blocks_for((int64_t)n), kBlock, 0, c->stream>>>(
+                (int32_t)n, c->fh_at.as<int32_t>() + lo, c->fh_val.as<uint16_t>() + lo, c->fh_id.as<uint16_t>());
+    }
+    TF_HIP(hipGetLastError());
+    TF_HIP(hipStreamSynchronize(c->stream));
+}
+
 template <class T>
 void create_fit(tf_ctx* c, const tf_problem* p) {
     const tf_fit_ops& f = p->fit;
@@ -968,10 +1058,18 @@ void create_fit(tf_ctx* c, const tf_problem* p) {
     c->h_fe_sg = sg;
     c->h_fe_f4 = f4;
     if (c->fit_grid) {
-        c->h_fe_code = ecode;
-        upload(c->fe_code, ecode);
-        upload(c->fe_ca, by_edge(ca));
-        upload(c->fe_cb, by_edge(cb));
+        const std::vector<T> a = by_edge(ca), b = by_edge(cb);
+        std::vector<FitPal<T>> pal;
+        if (fit_palette(ecode, a, b, c->h_fe_id, pal)) {
+            upload(c->fe_id, c->h_fe_id);
+            upload(c->fe_pal, pal);
+        } else {
+            c->h_fe_id.clear();
+            c->h_fe_code = ecode;
+            upload(c->fe_code, ecode);
+            upload(c->fe_ca, a);
+            upload(c->fe_cb, b);
+        }
     } else {
         upload(c->fe_sg, sg);
         upload(c->fe_ca, ca);
@@ -1013,9 +1111,23 @@ void create_fit(tf_ctx* c, const tf_problem* p) {
         cn[fi] = (T)(f.fpml[fi] * f.M_nu[fi]);
     }
     if (c->fit_grid) {
-        upload(c->fh_code, fcode);
-        upload(c->fh_cm, by_face(cm));
-        upload(c->fh_cn, by_face(cn));
+        const std::vector<T> a = by_face(cm), b = by_face(cn);
+        std::vector<FitPal<T>> pal;
+        if (fit_palette(fcode, a, b, c->h_fh_id, pal)) {
+            c->fh_k = (int32_t)pal.size();
+            pal.resize(2 * (size_t)c->fh_k);
+            for (int32_t k = 0; k < c->fh_k; ++k) {
+                pal[c->fh_k + k] = pal[k];
+                pal[c->fh_k + k].code |= kStoreB;
+            }
+            upload(c->fh_id, c->h_fh_id);
+            upload(c->fh_pal, pal);
+        } else {
+            c->h_fh_id.clear();
+            upload(c->fh_code, fcode);
+            upload(c->fh_cm, a);
+            upload(c->fh_cn, b);
+        }
     } else {
         upload(c->fh_sg, hs);
         upload(c->fh_cm, cm);
@@ -1389,7 +1501,8 @@ void build_fit_special(tf_ctx* c, const std::vector<std::vector<std::pair<int32_
     std::vector<double> ca, cb, tw;
     std::vector<int8_t> kind;
     std::vector<uint8_t> main_sg = c->h_fe_sg;
-    std::vector<uint16_t> main_code = c->h_fe_code;
+    // main pass codes, or palette ids (both 0 for an edge left out)
+    std::vector<uint16_t> main_code = c->fe_id.p ? c->h_fe_id : c->h_fe_code;
     auto off_main = [&](int32_t e) {  // the special item updates it
         if (c->fit_grid) main_code[c->h_esid[e]] = 0;
         else main_sg[e] = 0;
@@ -1445,7 +1558,7 @@ void build_fit_special(tf_ctx* c, const std::vector<std::vector<std::pair<int32_
     if (tsrc.empty()) { tsrc.push_back(0); tw.push_back(0); }
     upload(c->term_src, tsrc);
     upload(c->term_w, tw);
-    if (c->fit_grid) upload(c->fe_code, main_code);
+    if (c->fit_grid) upload(c->fe_id.p ? c->fe_id : c->fe_code, main_code);
     else upload(c->fe_sg, main_sg);
 }
 
@@ -1674,26 +1787,30 @@ void run_fit(tf_ctx* c, int64_t first, int64_t n, tf_stats* st) {
         }
     }
     // one step: E phase (with sources and the Poynting partials), H phase
-    auto step = [&](const double* cs, double* poy) {
+    auto step = [&](const double* cs, double* poy, bool store_b) {
         launch_timed(c, "fit_e_kernel", fit_e_kernel<T>, main_blocks + sp_blocks,
             c->E, sp_blocks, c->fe_sg.as<uint8_t>(), c->fe_ca.as<T>(), c->fe_cb.as<T>(), c->fe_f4.as<int4>(),
-            c->fit_grid ? c->fe_code.as<uint16_t>() : nullptr, c->grid, c->Fv.as<T>(), c->U.as<T>(), c->n_sp, c->sp_edge.as<int32_t>(), c->sp_f4.as<int4>(),
+            c->fit_grid ? c->fe_code.as<uint16_t>() : nullptr, c->fe_id.as<uint16_t>(), c->fe_pal.as<FitPal<T>>(),
+            c->grid, c->Fv.as<T>(), c->U.as<T>(), c->n_sp, c->sp_edge.as<int32_t>(), c->sp_f4.as<int4>(),
             c->sp_sg.as<uint8_t>(), c->sp_ca.as<double>(), c->sp_cb.as<double>(), c->sp_kind.as<int8_t>(),
             c->sp_tb.as<int32_t>(), c->sp_te.as<int32_t>(), c->term_src.as<int32_t>(), c->term_w.as<double>(), cs,
             sp_blocks ? poy : nullptr);
         launch_timed(c, "fit_h_kernel", fit_h_kernel<T>, h_blocks, c->F, c->fh_sg.as<uint8_t>(),
                      c->fh_cm.as<T>(), c->fh_cn.as<T>(), c->fh_e4.as<int4>(),
-                     c->fit_grid ? c->fh_code.as<uint16_t>() : nullptr, c->grid, c->U.as<T>(), c->Fv.as<T>(),
-                     c->B.as<T>(), c->dt);
+                     c->fit_grid ? c->fh_code.as<uint16_t>() : nullptr, c->fh_id.as<uint16_t>(),
+                     c->fh_pal.as<FitPal<T>>(), store_b ? 1 : 0, c->grid, c->U.as<T>(), c->Fv.as<T>(), c->B.as<T>(),
+                     c->dt);
     };
-    const int64_t g = graph_steps(c) ? run_graph_chunks(c, 0, n, sp_blocks, [&](int, const double* cs, double* poy) {
-        step(cs, poy);
+    const int64_t g = graph_steps(c) ? run_graph_chunks(c, 0, n, sp_blocks, [&](int k, const double* cs, double* poy) {
+        step(cs, poy, k == kGraphSteps - 1);
     }) : 0;
     for (int64_t k = g; k < n; ++k) {
         const int64_t i = first + k;
         const double t = (double)i * c->dt;
-        step(c->carr.as<double>() + (k + 1) * ns, c->poy.as<double>() + k * sp_blocks);
-        if (allow_print(c, t)) sample<T>(c, t);
+        const bool print = allow_print(c, t);
+        step(c->carr.as<double>() + (k + 1) * ns, c->poy.as<double>() + k * sp_blocks,
+             k == n - 1 || (print && c->energy_out));
+        if (print) sample<T>(c, t);
         if (c->profiling && (k & 63) == 63) ev_flush(c);
     }
     TF_HIP(hipGetLastError());
@@ -3543,6 +3660,11 @@ tf_status tf_set_probes(tf_ctx* c, const tf_probe* probes, int32_t n) {
                 d.h_idx[k] = dev_face(c, p.h_idx[k]);
                 for (int q = 0; q < 3; ++q) d.h_w[k][q] = p.h_w[k][q];
             }
+        }
+        if (c->method == TF_METHOD_FDTD) {
+            std::vector<int32_t> faces;
+            for (const ProbeDev& d : v) faces.insert(faces.end(), d.h_idx, d.h_idx + d.nh);
+            fit_probe_faces(c, faces);
         }
         c->n_probes = n;
         upload(c->probes, v);
