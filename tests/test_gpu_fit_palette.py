@@ -23,7 +23,8 @@ def _build(workdir, media):
 def test_palette_bitwise(workdir, monkeypatch, media, prec):
     """Runs of 64 (a replay and nothing after it), 1 and 70 steps without
     sampling: B is whole after each. Then the probes change between sampled
-    runs: a face that was probed, one that stays probed, new ones."""
+    runs (replays of other sample counts among them): a face that was probed,
+    one that stays probed, new ones. Last an output period that skips steps."""
     b = _build(workdir, media)
     got = {}
     for indexed in ("0", "1"):
@@ -36,12 +37,15 @@ def test_palette_bitwise(workdir, monkeypatch, media, prec):
             out += list(sim.state())
         _ffi.hip_lib().tf_set_output(sim._h, 0.0, 0.0)
         p, _, npr = b.probes_raw()
-        for lo, n in ((0, npr), (1, 2), (0, 0), (2, npr - 2)):
+        for lo, n, steps in ((0, npr, 133), (1, 2, 5), (0, 0, 70), (2, npr - 2, 65), (0, npr, 64)):
             part = (_ffi.tf_probe * max(n, 1))(*[p[lo + k] for k in range(n)])
             assert _ffi.hip_lib().tf_set_probes(sim._h, part, n) == 0
             sim.n_probes = n
-            sim.run(n=5)
-            out += [sim.probes()[1], *sim.state()]
+            sim.run(n=steps)
+            out += [*sim.probes(), *sim.state()]
+        _ffi.hip_lib().tf_set_output(sim._h, sim.next_step * b.dt, 2.5 * b.dt)
+        sim.run(n=70)
+        out += [*sim.probes(), *sim.state()]
         out.append(sim.poynting())
         sim.close()
         got[indexed] = out

@@ -143,54 +143,52 @@ __host__ __device__ inline void fit_counts(const FitGrid g, bool faces, uint32_t
 // items gather (faces of an edge, edges of a face) stay in its own L2; with a
 // single contiguous range per XCD, each gathered plane would be read through
 // the L2s of two XCDs. Workgroup b runs on XCD b % 8 and takes the (b / 8)-th
-// block of that XCD's list (its x, then y, then z blocks). The grid has
-// 8 * (longest list) workgroups (slab_grid); returns the item, or -1 for a
-// workgroup past its XCD's list or a lane past its direction's end.
-__host__ __device__ inline uint32_t slab_len(uint32_t n, uint32_t x) {
-    const uint32_t nb = (n + kBlock - 1) / kBlock;
+// block of `per` items of that XCD's list (its x, then y, then z blocks). The
+// grid has 8 * (longest list) workgroups (slab_grid).
+__host__ __device__ inline uint32_t slab_len(uint32_t n, uint32_t x, uint32_t per) {
+    const uint32_t nb = (n + per - 1) / per;
     return (x + 1) * nb / kXcd - x * nb / kXcd;
 }
-inline int slab_grid(const uint32_t n[3]) {
+inline int slab_grid(const uint32_t n[3], uint32_t per) {
     uint32_t m = 1;
     for (uint32_t x = 0; x < (uint32_t)kXcd; ++x)
-        m = std::max(m, slab_len(n[0], x) + slab_len(n[1], x) + slab_len(n[2], x));
+        m = std::max(m, slab_len(n[0], x, per) + slab_len(n[1], x, per) + slab_len(n[2], x, per));
     return (int)(m * kXcd);
 }
 // The XCD's list interleaves the three directions block by block (x, y, z,
 // x, y, z, ...; the longer directions' last few blocks follow), so that all
 // three advance through the slab's planes together and a plane of gathered
 // neighbours, read by two directions, is fetched once while it is in L2.
-__device__ __forceinline__ int32_t slab_item(int b, const uint32_t n[3]) {
+// dir: the workgroup's direction (-1: none), first: its first item there.
+template <uint32_t per>
+__device__ __forceinline__ void slab_block(int b, const uint32_t n[3], int& dir, uint32_t& first) {
     const uint32_t x = (uint32_t)b % kXcd, i = (uint32_t)b / kXcd;
     uint32_t lo[3], len[3];
 #pragma unroll
     for (int t = 0; t < 3; ++t) {
-        const uint32_t nb = (n[t] + kBlock - 1) / kBlock;
+        const uint32_t nb = (n[t] + per - 1) / per;
         lo[t] = x * nb / kXcd;
         len[t] = (x + 1) * nb / kXcd - lo[t];
     }
     const uint32_t m = min(len[0], min(len[1], len[2]));
-    int t = -1;
     uint32_t j = 0;
+    dir = -1;
     if (i < 3 * m) {
-        t = (int)(i % 3);
+        dir = (int)(i % 3);
         j = i / 3;
     } else {
         uint32_t k = i - 3 * m;
 #pragma unroll
         for (int u = 0; u < 3; ++u) {
-            if (t < 0 && k < len[u] - m) {
-                t = u;
+            if (dir < 0 && k < len[u] - m) {
+                dir = u;
                 j = m + k;
-            } else if (t < 0) {
+            } else if (dir < 0) {
                 k -= len[u] - m;
             }
         }
-        if (t < 0) return -1;
     }
-    const uint32_t base = t == 0 ? 0u : (t == 1 ? n[0] : n[0] + n[1]);
-    const uint32_t r = (lo[t] + j) * kBlock + threadIdx.x;
-    return r < n[t] ? (int32_t)(base + r) : -1;
+    first = dir < 0 ? 0 : ((dir == 0 ? lo[0] : dir == 1 ? lo[1] : lo[2]) + j) * per;
 }
 
 // 32-bit index arithmetic: grid order is used only when edge and face
@@ -244,95 +242,67 @@ __host__ __device__ inline void fit_face_slots(const FitGrid g, uint32_t s, int3
     }
 }
 
-// Sum over the four positions p of sign_p * v[slot_p] in position order,
-// with code = slot map (2 bits per position) << 8 | sign code (2 bits per
-// position: 1 -> +1, 2 -> -1, 0 -> 0): the reference's F0 - F1 + F2 - F3
-// order, whatever slot each of its faces sits in.
-__device__ __forceinline__ double slot_sum(uint32_t code, const double v[4]) {
-    const uint32_t m = code >> 8;
-    double c = sgn2(code & 3) * v[m & 3];
-    c += sgn2((code >> 2) & 3) * v[(m >> 2) & 3];
-    c += sgn2((code >> 4) & 3) * v[(m >> 4) & 3];
-    c += sgn2((code >> 6) & 3) * v[(m >> 6) & 3];
-    return c;
+// The two updates, with the fused multiply-add written out so that every
+// kernel rounds them alike: ca u + cb c and cm f - dt c.
+__device__ __forceinline__ double fit_e_new(double ca, double u, double cb, double c) {
+    return __builtin_fma(ca, u, cb * c);
 }
+__device__ __forceinline__ double fit_b_new(double cm, double f, double dtc) { return __builtin_fma(cm, f, -dtc); }
 
-// Coefficient palette of the grid order: with media that are uniform per
-// region, a kernel's per-item constants (the two coefficients and the 16-bit
-// sign and order code) take few distinct values, so each item stores the
-// 16-bit number of its entry here instead of 2 sizeof(T) + 2 bytes (id 0:
-// not in the main pass). The table (24 bytes an entry in fp64) stays in L1.
-// Both kernels are bound by bytes: an fp64 item moves 26 instead of 42 bytes
-// (E) and, with B stored only where it is read (below), 26 instead of 50 (H).
-template <typename T>
-struct FitPal {
-    T c0, c1;       // E: ca, cb; H: cm, cn
-    uint32_t code;  // slot_sum code, | kStoreB
-};
-constexpr uint32_t kStoreB = 1u << 16;  // H: a probed face, B is stored every step
-
-// id[at[i]] = val[i] (palette ids of faces that become probed or stop to be)
-__global__ void __launch_bounds__(kBlock) set_ids_kernel(int32_t n, const int32_t* __restrict__ at,
-                                                         const uint16_t* __restrict__ val, uint16_t* __restrict__ id) {
-    const int32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i < n) id[at[i]] = val[i];
-}
-
-// E phase (D:1850-1895). The first sp_blocks workgroups take the special
-// items, so that their longer dependent chains (source value, Poynting sum)
-// start with the launch instead of trailing it; the rest cover every edge in
-// index order (XCD-mapped among themselves). Edges whose sign byte is 0
-// (pec / source / non-common) are left to the special items. U = ca*U_old + cb*(sum_k s_k F[f_k])
-//   common:   ca = upml^2 M_h M_q, cb = upml^3 M_h dt, s = dual_curl*(+,-,+,-)
-// Special items (uncommon h-source edges, e/j source edges):
+// One special item of the E phase (D:1850-1895): uncommon h-source edges and
+// e / j source edges, with their own face lists and fp64 coefficients:
 //   kind 0 (h):  U = ca*U_old + cb*(sum s_k F + src)     (ca = M_h M_q, cb = M_h dt)
 //   kind 1 (e):  U = src
 //   kind 2 (j):  U = ca*U_old + cb*(sum s_k F - src)     (common coefficients)
-// With code16 (grid order) the main blocks take their edges by slab_item,
-// each edge's faces from its position and its sign and order code from code16
-// (slot_sum); otherwise edges by index order over XCD ranges, faces from the
-// packed face quadruple f4 and the sign byte sg. With pid (grid order, few
-// distinct coefficients) the code and coefficients come from pal[pid[e]].
+struct FitSpecial {
+    int32_t n;
+    const int32_t* edge;
+    const int4* f4;
+    const uint8_t* sg;
+    const double* ca;
+    const double* cb;
+    const int8_t* kind;
+    const int32_t* tb;
+    const int32_t* te;
+    const int32_t* term_src;
+    const double* term_w;
+};
 template <typename T>
-__global__ void __launch_bounds__(kBlock) fit_e_kernel(
-    int32_t n_edges, int32_t sp_blocks, const uint8_t* __restrict__ sg, const T* __restrict__ ca,
-    const T* __restrict__ cb, const int4* __restrict__ f4, const uint16_t* __restrict__ code16,
-    const uint16_t* __restrict__ pid, const FitPal<T>* __restrict__ pal, FitGrid grid,
-    const T* __restrict__ Fv, T* __restrict__ U,
-    int32_t n_sp, const int32_t* __restrict__ sp_edge, const int4* __restrict__ sp_f4,
-    const uint8_t* __restrict__ sp_sg, const double* __restrict__ sp_ca, const double* __restrict__ sp_cb,
-    const int8_t* __restrict__ sp_kind, const int32_t* __restrict__ sp_tb, const int32_t* __restrict__ sp_te,
-    const int32_t* __restrict__ term_src, const double* __restrict__ term_w,
-    const double* __restrict__ carr_step, double* __restrict__ poy_part) {
+__device__ __forceinline__ double fit_special(const FitSpecial& sp, int32_t i, double uold, double src,
+                                              const T* __restrict__ Fv) {
+    const int k = sp.kind[i];
+    if (k == 1) return src;
+    const int4 f = sp.f4[i];
+    const uint32_t s = sp.sg[i];
+    double c = 0;
+    if (s & 3) c += sgn2(s & 3) * (double)Fv[f.x];
+    if ((s >> 2) & 3) c += sgn2((s >> 2) & 3) * (double)Fv[f.y];
+    if ((s >> 4) & 3) c += sgn2((s >> 4) & 3) * (double)Fv[f.z];
+    if ((s >> 6) & 3) c += sgn2((s >> 6) & 3) * (double)Fv[f.w];
+    c += k == 0 ? src : -src;
+    return fit_e_new(sp.ca[i], uold, sp.cb[i], c);
+}
+// Source value of a special item from one carrier row.
+__device__ __forceinline__ double fit_source(const FitSpecial& sp, int32_t i, const double* __restrict__ carr) {
+    return source_value(sp.tb[i], sp.te[i], sp.term_src, sp.term_w, carr);
+}
+
+// E phase of the index-table layout (D:1850-1895). The first sp_blocks
+// workgroups take the special items, so that their longer dependent chains
+// (source value, Poynting sum) start with the launch instead of trailing it;
+// the rest cover every edge in index order (XCD-mapped among themselves).
+// Edges whose sign byte is 0 (pec / source / non-common) are left to the
+// special items. U = ca*U_old + cb*(sum_k s_k F[f_k])
+//   common:   ca = upml^2 M_h M_q, cb = upml^3 M_h dt, s = dual_curl*(+,-,+,-)
+template <typename T>
+__global__ void __launch_bounds__(kBlock) fit_e_kernel(int32_t n_edges, int32_t sp_blocks,
+                                                       const uint8_t* __restrict__ sg, const T* __restrict__ ca,
+                                                       const T* __restrict__ cb, const int4* __restrict__ f4,
+                                                       const T* __restrict__ Fv, T* __restrict__ U, FitSpecial sp,
+                                                       const double* __restrict__ carr_step,
+                                                       double* __restrict__ poy_part) {
     const int hb = (int)blockIdx.x;
     if (hb >= sp_blocks) {
-        if (pid) {
-            uint32_t cnt[3];
-            fit_counts(grid, false, cnt);
-            const int32_t e = slab_item(hb - sp_blocks, cnt);
-            if (e < 0) return;
-            const uint32_t id = pid[e];
-            if (id == 0) return;
-            const FitPal<T> q = pal[id];
-            int32_t f[4];
-            fit_edge_slots(grid, (uint32_t)e, f);
-            const double v[4] = {(double)Fv[f[0]], (double)Fv[f[1]], (double)Fv[f[2]], (double)Fv[f[3]]};
-            U[e] = (T)((double)q.c0 * (double)U[e] + (double)q.c1 * slot_sum(q.code, v));
-            return;
-        }
-        if (code16) {
-            uint32_t cnt[3];
-            fit_counts(grid, false, cnt);
-            const int32_t e = slab_item(hb - sp_blocks, cnt);
-            if (e < 0) return;
-            const uint32_t code = code16[e];
-            if (code == 0) return;
-            int32_t f[4];
-            fit_edge_slots(grid, (uint32_t)e, f);
-            const double v[4] = {(double)Fv[f[0]], (double)Fv[f[1]], (double)Fv[f[2]], (double)Fv[f[3]]};
-            U[e] = (T)((double)ca[e] * (double)U[e] + (double)cb[e] * slot_sum(code, v));
-            return;
-        }
         const int32_t e = xcd_block_of(hb - sp_blocks, (int)gridDim.x - sp_blocks) * kBlock + threadIdx.x;
         if (e >= n_edges) return;
         const uint32_t s = sg[e];
@@ -340,84 +310,33 @@ __global__ void __launch_bounds__(kBlock) fit_e_kernel(
         const int4 f = f4[e];
         double c = sgn2(s & 3) * (double)Fv[f.x] + sgn2((s >> 2) & 3) * (double)Fv[f.y] +
                    sgn2((s >> 4) & 3) * (double)Fv[f.z] + sgn2((s >> 6) & 3) * (double)Fv[f.w];
-        U[e] = (T)((double)ca[e] * (double)U[e] + (double)cb[e] * c);
+        U[e] = (T)fit_e_new((double)ca[e], (double)U[e], (double)cb[e], c);
         return;
     }
     __shared__ double red[kBlock / kWave];
     const int32_t i = hb * kBlock + threadIdx.x;
     double poy = 0;
-    if (i < n_sp) {
-        const int32_t e = sp_edge[i];
-        const double src = source_value(sp_tb[i], sp_te[i], term_src, term_w, carr_step);
-        const int k = sp_kind[i];
+    if (i < sp.n) {
+        const int32_t e = sp.edge[i];
+        const double src = fit_source(sp, i, carr_step);
         const double uold = (double)U[e];
-        double unew;
-        if (k == 1) {
-            unew = src;
-        } else {
-            const int4 f = sp_f4[i];
-            const uint32_t s = sp_sg[i];
-            double c = 0;
-            if (s & 3) c += sgn2(s & 3) * (double)Fv[f.x];
-            if ((s >> 2) & 3) c += sgn2((s >> 2) & 3) * (double)Fv[f.y];
-            if ((s >> 4) & 3) c += sgn2((s >> 4) & 3) * (double)Fv[f.z];
-            if ((s >> 6) & 3) c += sgn2((s >> 6) & 3) * (double)Fv[f.w];
-            c += k == 0 ? src : -src;
-            unew = sp_ca[i] * uold + sp_cb[i] * c;
-        }
+        const double unew = fit_special<T>(sp, i, uold, src, Fv);
         U[e] = (T)unew;
         // Poynting term 0.5*(U_old+U)*curl_fb, nonzero on h-source edges only (D:1901)
-        if (k == 0) poy = 0.5 * (uold + (double)(T)unew) * src;
+        if (sp.kind[i] == 0) poy = 0.5 * (uold + (double)(T)unew) * src;
     }
     const double s = block_sum(poy, red);
     if (threadIdx.x == 0) poy_part[hb] = s;
 }
 
-// H phase over tbc faces (D:1908-1915): B = cm*F_old - dt*sum s_k U[e_k];
-// F = cn*B with cm = M_mu*fpml, cn = fpml*M_nu, s = curl*(+,-,+,-).
-// code16 / pid / grid as in fit_e_kernel. The loop itself never reads B (the
-// update takes F_old): with pid it is stored only where something reads it
-// before the next step overwrites it, on probed faces (kStoreB) every step
-// and on every face with store_b (the run's last step, energy samples).
+// H phase over tbc faces (D:1908-1915), index-table layout:
+// B = cm*F_old - dt*sum s_k U[e_k]; F = cn*B with cm = M_mu*fpml,
+// cn = fpml*M_nu, s = curl*(+,-,+,-).
 template <typename T>
 __global__ void __launch_bounds__(kBlock) fit_h_kernel(int32_t n_faces, const uint8_t* __restrict__ sg,
                                                        const T* __restrict__ cm, const T* __restrict__ cn,
-                                                       const int4* __restrict__ e4, const uint16_t* __restrict__ code16,
-                                                       const uint16_t* __restrict__ pid,
-                                                       const FitPal<T>* __restrict__ pal, int store_b, FitGrid grid,
-                                                       const T* __restrict__ U, T* __restrict__ Fv, T* __restrict__ B,
-                                                       double dt) {
-    if (pid) {
-        uint32_t cnt[3];
-        fit_counts(grid, true, cnt);
-        const int32_t f = slab_item((int)blockIdx.x, cnt);
-        if (f < 0) return;
-        const uint32_t id = pid[f];
-        if (id == 0) return;
-        const FitPal<T> q = pal[id];
-        int32_t e[4];
-        fit_face_slots(grid, (uint32_t)f, e);
-        const double v[4] = {(double)U[e[0]], (double)U[e[1]], (double)U[e[2]], (double)U[e[3]]};
-        const double b = (double)q.c0 * (double)Fv[f] - dt * slot_sum(q.code & 0xFFFFu, v);
-        if (store_b || (q.code & kStoreB)) B[f] = (T)b;
-        Fv[f] = (T)((double)q.c1 * b);
-        return;
-    }
-    if (code16) {
-        uint32_t cnt[3];
-        fit_counts(grid, true, cnt);
-        const int32_t f = slab_item((int)blockIdx.x, cnt);
-        if (f < 0) return;
-        const uint32_t code = code16[f];
-        if (code == 0) return;
-        int32_t e[4];
-        fit_face_slots(grid, (uint32_t)f, e);
-        const double v[4] = {(double)U[e[0]], (double)U[e[1]], (double)U[e[2]], (double)U[e[3]]};
-        const double b = (double)cm[f] * (double)Fv[f] - dt * slot_sum(code, v);
-        B[f] = (T)b;
-        Fv[f] = (T)((double)cn[f] * b);
-        return;
-    }
+                                                       const int4* __restrict__ e4, const T* __restrict__ U,
+                                                       T* __restrict__ Fv, T* __restrict__ B, double dt) {
     const int32_t f = xcd_block() * kBlock + threadIdx.x;
     if (f >= n_faces) return;
     const uint32_t s = sg[f];
@@ -425,7 +344,7 @@ __global__ void __launch_bounds__(kBlock) fit_h_kernel(int32_t n_faces, const ui
     const int4 e = e4[f];
     double c = sgn2(s & 3) * (double)U[e.x] + sgn2((s >> 2) & 3) * (double)U[e.y] +
                sgn2((s >> 4) & 3) * (double)U[e.z] + sgn2((s >> 6) & 3) * (double)U[e.w];
-    const double b = (double)cm[f] * (double)Fv[f] - dt * c;
+    const double b = fit_b_new((double)cm[f], (double)Fv[f], dt * c);
     B[f] = (T)b;
     Fv[f] = (T)((double)cn[f] * b);
 }
@@ -441,21 +360,319 @@ struct ProbeDev {
     double h_w[6][3];
 };
 
+// Component c of probe q. All loads are issued before the first is used (the
+// terms' sum keeps its order): as a loop of dependent loads the 12 terms of a
+// FIT probe took 8.6 us a launch.
+template <typename T>
+__device__ __forceinline__ double probe_value(const ProbeDev& q, int c, const T* __restrict__ U,
+                                              const T* __restrict__ B) {
+    const bool e = c < 3;
+    const int n = e ? q.ne : q.nh, cc = e ? c : c - 3;
+    double v = 0;
+    if (e) {
+        T x[12];
+        double w[12];
+#pragma unroll
+        for (int k = 0; k < 12; ++k) {
+            x[k] = U[k < n ? q.e_idx[k] : 0];
+            w[k] = q.e_w[k][cc];
+        }
+#pragma unroll
+        for (int k = 0; k < 12; ++k)
+            if (k < n) v += (double)x[k] * w[k];
+    } else {
+        T x[6];
+        double w[6];
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            x[k] = B[k < n ? q.h_idx[k] : 0];
+            w[k] = q.h_w[k][cc];
+        }
+#pragma unroll
+        for (int k = 0; k < 6; ++k)
+            if (k < n) v += (double)x[k] * w[k];
+    }
+    return v;
+}
+
 template <typename T>
 __global__ void probe_kernel(int32_t n_probes, const ProbeDev* __restrict__ pr, const T* __restrict__ U,
                              const T* __restrict__ B, double* __restrict__ out, const CgState* guard) {
     if (!cg_guard_ok(guard)) return;
     const int32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n_probes * 6) return;
-    const int p = t / 6, c = t % 6;
-    const ProbeDev& q = pr[p];
-    double v = 0;
-    if (c < 3) {
-        for (int k = 0; k < q.ne; ++k) v += (double)U[q.e_idx[k]] * q.e_w[k][c];
-    } else {
-        for (int k = 0; k < q.nh; ++k) v += (double)B[q.h_idx[k]] * q.h_w[k][c - 3];
+    out[t] = probe_value<T>(pr[t / 6], t % 6, U, B);
+}
+
+// Sampling inside a step's kernels: workgroups of the launch evaluate the
+// probes for the output sample *slot (negative: none), components [c0, c0 + nc)
+// of each (0..2 from U, 3..5 from B). The probes and the sample buffer are read
+// from device memory, so that captured steps follow a change of either. As a
+// launch of its own a sample cost 5 us of host-launched step at 16^3, and kept
+// the steps out of the graph.
+struct SampleRef {
+    const ProbeDev* probes;
+    double* out;
+    int32_t n_probes;
+};
+template <typename T>
+__device__ __forceinline__ void sample_probes(const SampleRef* __restrict__ ref, const int64_t* __restrict__ slot,
+                                              int32_t t, int c0, int nc, const T* __restrict__ U,
+                                              const T* __restrict__ B) {
+    const int64_t sl = *slot;
+    const SampleRef r = *ref;
+    const int32_t p = t / nc, c = c0 + t % nc;
+    if (sl < 0 || p >= r.n_probes) return;
+    r.out[(sl * r.n_probes + p) * 6 + c] = probe_value<T>(r.probes[p], c, U, B);
+}
+
+template <typename T>
+__global__ void __launch_bounds__(kBlock) probe_tail_kernel(const SampleRef* __restrict__ ref,
+                                                            const int64_t* __restrict__ slot, int c0, int nc,
+                                                            const T* __restrict__ U, const T* __restrict__ B) {
+    sample_probes<T>(ref, slot, (int32_t)(blockIdx.x * kBlock + threadIdx.x), c0, nc, U, B);
+}
+
+// ------------------------------------------------------------------ FIT, grid order
+// Constants of one entity. With media that are uniform per region they take
+// few distinct values: each entity then stores the 16-bit number of its entry
+// (id 0: not updated) and a workgroup keeps the table in LDS. At most kPalMax
+// entries (8 KB in fp64; a cavity holds 2 to 4, a random medium's E side one
+// per edge), else id 1 and plain arrays.
+template <typename T>
+struct FitPal {
+    T c0, c1;  // E: ca, cb; H: cm, cn
+};
+constexpr int kPalMax = 512;
+
+// id[at[i]] = val[i] (faces that become probed or stop to be)
+__global__ void __launch_bounds__(kBlock) set_ids_kernel(int32_t n, const int32_t* __restrict__ at,
+                                                         const uint16_t* __restrict__ val, uint16_t* __restrict__ id) {
+    const int32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) id[at[i]] = val[i];
+}
+
+// spv[i] = source value of special item i from one carrier row.
+__global__ void __launch_bounds__(kBlock) fit_src_kernel(FitSpecial sp, const double* __restrict__ carr,
+                                                         double* __restrict__ spv) {
+    const int32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < sp.n) spv[i] = fit_source(sp, i, carr);
+}
+
+// What the two kernels of a step share. A kernel starts with cold L2 (the
+// other XCDs wrote part of what it reads), so on grids up to about 64^3 each
+// dependent load level costs about 0.8 us of a 5 us launch. Everything an item
+// needs is therefore loaded at once: its neighbours' positions follow from its
+// own (clamped at the boundary, where nothing of them is used), the palette
+// goes to LDS meanwhile, and source values are prepared a step ahead. Larger
+// grids are bound by bytes: an fp64 item moves 26 (E) and 26 (H) with palettes,
+// against 42 and 50 with plain coefficients and B stored every step.
+// One step (both kernels, in a graph): 64^3 fp64 12.1 us, fp32 9.8 us; 161^3
+// random media fp64 163 us (E 94 us, 5.7 TB/s; H 67 us, 4.9 TB/s). With codes
+// read before the neighbours, five-load source chains and one item per thread:
+// 15.4, 12.0 and 185 us.
+template <typename T>
+struct FitStep {
+    FitGrid g;
+    int32_t sp_blocks, probe_blocks, src_blocks;
+    int32_t n_pal;        // entries of pal
+    uint32_t flag;        // H: ids from here on are probed faces
+    const uint16_t* id;
+    const FitPal<T>* pal;
+    const T* c0;          // plain coefficients (no palette)
+    const T* c1;
+    double sg[3];         // sign of the sums per direction (H: times dt)
+    FitSpecial sp;
+    const double* spv;
+    double* spv_next;
+    const double* carr_next;
+    double* poy_part;
+    const SampleRef* ref;
+    const int64_t* slot;  // E: of the step before (its B); H: of this step (its U)
+};
+
+// Palette into LDS (before the loads that follow are waited for).
+template <typename T, bool P>
+__device__ __forceinline__ void fit_pal_load(const FitStep<T>& a, FitPal<T>* __restrict__ lds) {
+    if constexpr (P)
+        for (int t = (int)threadIdx.x; t < a.n_pal; t += kBlock) lds[t] = a.pal[t];
+}
+
+// E phase (D:1850-1895). Workgroups: the special items first (their chains are
+// the longest), then the H components of the sample of the step before, then
+// the edges, N per thread, by slab_block. U = ca U + cb c, c the signed sum of the edge's four
+// faces in the order 0, 2, 3, 1 of fit_edge_slots with signs +, -, +, - and the
+// direction's sign (checked when the context is created). Special items take
+// their source value from spv.
+template <typename T, bool P, int N>
+__global__ void __launch_bounds__(kBlock) fit_e_grid_kernel(FitStep<T> a, const T* __restrict__ Fv, T* __restrict__ U,
+                                                            const T* __restrict__ B) {
+    __shared__ FitPal<T> pal[P ? kPalMax : 1];
+    __shared__ double red[kBlock / kWave];
+    const int hb = (int)blockIdx.x;
+    if (hb < a.sp_blocks) {
+        const int32_t i = hb * kBlock + threadIdx.x;
+        double poy = 0;
+        if (i < a.sp.n) {
+            const int32_t e = a.sp.edge[i];
+            const double src = a.spv[i], uold = (double)U[e];
+            const double unew = fit_special<T>(a.sp, i, uold, src, Fv);
+            U[e] = (T)unew;
+            // Poynting term 0.5*(U_old+U)*curl_fb, nonzero on h-source edges only (D:1901)
+            if (a.sp.kind[i] == 0) poy = 0.5 * (uold + (double)(T)unew) * src;
+        }
+        const double s = block_sum(poy, red);
+        if (threadIdx.x == 0) a.poy_part[hb] = s;
+        return;
     }
-    out[t] = v;
+    if (hb < a.sp_blocks + a.probe_blocks) {
+        sample_probes<T>(a.ref, a.slot, (hb - a.sp_blocks) * kBlock + (int)threadIdx.x, 3, 3, (const T*)nullptr, B);
+        return;
+    }
+    uint32_t cnt[3], first;
+    int dir;
+    fit_counts(a.g, false, cnt);
+    slab_block<N * kBlock>(hb - a.sp_blocks - a.probe_blocks, cnt, dir, first);
+    if (dir < 0) return;
+    const uint32_t nx = a.g.nx, ny = a.g.ny, nz = a.g.nz;
+    const uint32_t nF1 = (nx + 1) * ny * nz, nF2 = nF1 + nx * (ny + 1) * nz;
+    const uint32_t n = dir == 0 ? cnt[0] : dir == 1 ? cnt[1] : cnt[2];
+    const uint32_t base = dir == 0 ? 0 : dir == 1 ? cnt[0] : cnt[0] + cnt[1];
+    const double sg = a.sg[dir];
+    fit_pal_load<T, P>(a, pal);
+    uint32_t id[N];
+    T u[N], v0[N], v1[N], v2[N], v3[N];
+    FitPal<T> q[N];
+#pragma unroll
+    for (int m = 0; m < N; ++m) {
+        // an item past the end repeats the last one's loads
+        const uint32_t r = min(first + m * kBlock + threadIdx.x, n - 1), s = base + r;
+        uint32_t i, j, k, t, f0, f1, f2, f3;
+        bool in;  // all four faces exist
+        if (dir == 0) {
+            fit_divmod(a.g.dx, r, t, i);
+            fit_divmod(a.g.dy1, t, k, j);
+            in = j > 0 && j < ny && k > 0 && k < nz;
+            f1 = nF1 + (k * (ny + 1) + j) * nx + i;
+            f0 = f1 - (ny + 1) * nx;
+            f3 = nF2 + (k * ny + j) * nx + i;
+            f2 = f3 - nx;
+        } else if (dir == 1) {
+            fit_divmod(a.g.dx1, r, t, i);
+            fit_divmod(a.g.dy, t, k, j);
+            in = i > 0 && i < nx && k > 0 && k < nz;
+            f1 = (k * ny + j) * (nx + 1) + i;
+            f0 = f1 - ny * (nx + 1);
+            f3 = nF2 + (k * ny + j) * nx + i;
+            f2 = f3 - 1;
+        } else {
+            fit_divmod(a.g.dx1, r, t, i);
+            fit_divmod(a.g.dy1, t, k, j);
+            in = i > 0 && i < nx && j > 0 && j < ny;
+            f1 = (k * ny + j) * (nx + 1) + i;
+            f0 = f1 - (nx + 1);
+            f3 = nF1 + (k * (ny + 1) + j) * nx + i;
+            f2 = f3 - 1;
+        }
+        id[m] = a.id[s];
+        u[m] = U[s];
+        v0[m] = Fv[in ? f0 : 0];
+        v1[m] = Fv[in ? f1 : 0];
+        v2[m] = Fv[in ? f2 : 0];
+        v3[m] = Fv[in ? f3 : 0];
+        if constexpr (!P) q[m] = FitPal<T>{a.c0[s], a.c1[s]};
+    }
+    if constexpr (P) __syncthreads();
+#pragma unroll
+    for (int m = 0; m < N; ++m) {
+        const uint32_t r = first + m * kBlock + threadIdx.x;
+        if constexpr (P) q[m] = pal[id[m]];
+        const double c = sg * ((((double)v0[m] - (double)v2[m]) + (double)v3[m]) - (double)v1[m]);
+        if (r < n && id[m]) U[base + r] = (T)fit_e_new((double)q[m].c0, (double)u[m], (double)q[m].c1, c);
+    }
+}
+
+// H phase over tbc faces (D:1908-1915): B = cm F_old - dt c, F = cn B, c the
+// signed sum of the face's four edges (order and signs as in the E phase).
+// The loop itself never reads B, so it is stored only where something reads it
+// before the next step overwrites it: on probed faces (id >= flag) every step
+// and on every face with store_b (the run's last step, energy samples). The
+// first workgroups take the U components of this step's sample and the next
+// step's source values.
+template <typename T, bool P, int N>
+__global__ void __launch_bounds__(kBlock) fit_h_grid_kernel(FitStep<T> a, int store_b, const T* __restrict__ U,
+                                                            T* __restrict__ Fv, T* __restrict__ B) {
+    __shared__ FitPal<T> pal[P ? kPalMax : 1];
+    const int hb = (int)blockIdx.x;
+    if (hb < a.src_blocks) {
+        const int32_t i = hb * kBlock + threadIdx.x;
+        if (i < a.sp.n) a.spv_next[i] = fit_source(a.sp, i, a.carr_next);
+        return;
+    }
+    if (hb < a.src_blocks + a.probe_blocks) {
+        sample_probes<T>(a.ref, a.slot, (hb - a.src_blocks) * kBlock + (int)threadIdx.x, 0, 3, U, (const T*)nullptr);
+        return;
+    }
+    uint32_t cnt[3], first;
+    int dir;
+    fit_counts(a.g, true, cnt);
+    slab_block<N * kBlock>(hb - a.src_blocks - a.probe_blocks, cnt, dir, first);
+    if (dir < 0) return;
+    const uint32_t nx = a.g.nx, ny = a.g.ny, nz = a.g.nz;
+    const uint32_t nE1 = nx * (ny + 1) * (nz + 1), nE2 = nE1 + (nx + 1) * ny * (nz + 1);
+    const uint32_t n = dir == 0 ? cnt[0] : dir == 1 ? cnt[1] : cnt[2];
+    const uint32_t base = dir == 0 ? 0 : dir == 1 ? cnt[0] : cnt[0] + cnt[1];
+    const double sg = a.sg[dir];
+    fit_pal_load<T, P>(a, pal);
+    uint32_t id[N];
+    T fo[N], v0[N], v1[N], v2[N], v3[N];
+    FitPal<T> q[N];
+#pragma unroll
+    for (int m = 0; m < N; ++m) {
+        const uint32_t r = min(first + m * kBlock + threadIdx.x, n - 1), s = base + r;
+        uint32_t i, j, k, t, e0, e1, e2, e3;
+        if (dir == 0) {
+            fit_divmod(a.g.dx1, r, t, i);
+            fit_divmod(a.g.dy, t, k, j);
+            e0 = nE1 + (k * ny + j) * (nx + 1) + i;
+            e1 = e0 + ny * (nx + 1);
+            e2 = nE2 + (k * (ny + 1) + j) * (nx + 1) + i;
+            e3 = e2 + (nx + 1);
+        } else if (dir == 1) {
+            fit_divmod(a.g.dx, r, t, i);
+            fit_divmod(a.g.dy1, t, k, j);
+            e0 = (k * (ny + 1) + j) * nx + i;
+            e1 = e0 + (ny + 1) * nx;
+            e2 = nE2 + (k * (ny + 1) + j) * (nx + 1) + i;
+            e3 = e2 + 1;
+        } else {
+            fit_divmod(a.g.dx, r, t, i);
+            fit_divmod(a.g.dy, t, k, j);
+            e0 = (k * (ny + 1) + j) * nx + i;
+            e1 = e0 + nx;
+            e2 = nE1 + (k * ny + j) * (nx + 1) + i;
+            e3 = e2 + 1;
+        }
+        id[m] = a.id[s];
+        fo[m] = Fv[s];
+        v0[m] = U[e0];
+        v1[m] = U[e1];
+        v2[m] = U[e2];
+        v3[m] = U[e3];
+        if constexpr (!P) q[m] = FitPal<T>{a.c0[s], a.c1[s]};
+    }
+    if constexpr (P) __syncthreads();
+#pragma unroll
+    for (int m = 0; m < N; ++m) {
+        const uint32_t r = first + m * kBlock + threadIdx.x;
+        if constexpr (P) q[m] = pal[id[m] >= a.flag ? id[m] - a.flag : id[m]];
+        const double c = (((double)v0[m] - (double)v2[m]) + (double)v3[m]) - (double)v1[m];
+        const double b = fit_b_new((double)q[m].c0, (double)fo[m], sg * c);
+        if (r < n && id[m]) {
+            if (store_b || id[m] >= a.flag) B[base + r] = (T)b;
+            Fv[base + r] = (T)((double)q[m].c1 * b);
+        }
+    }
 }
 
 // ------------------------------------------------------------------ DGA

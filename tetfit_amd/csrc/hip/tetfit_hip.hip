@@ -233,14 +233,15 @@ struct tf_ctx {
     bool wide = false;
     FitGrid grid{};
     std::vector<int32_t> h_esid, h_fsid;  // reference edge / face -> device position (FIT grid order, tet relabel)
-    std::vector<uint16_t> h_fe_code;      // per grid edge: slot map << 8 | signs (0: not in the main pass)
-    DevBuf fe_code, fh_code;
-    // coefficient palettes (FitPal), in place of code and coefficient arrays
-    // where few distinct values occur; probed faces carry id + fh_k
-    DevBuf fe_id, fe_pal, fh_id, fh_pal, fh_at, fh_val;
+    // grid order (fit_e_grid_kernel, fit_h_grid_kernel): id per entity (0: not
+    // in the main pass) and a coefficient palette, or, where too many distinct
+    // values occur, id 1 and the plain arrays; probed faces carry id + fh_flag
+    DevBuf fe_id, fe_pal, fh_id, fh_pal, fh_at, fh_val, spv;
     std::vector<uint16_t> h_fe_id, h_fh_id;
-    int32_t fh_k = 0;
-    std::vector<int32_t> fh_probed;  // device faces whose id carries kStoreB
+    int32_t fe_n = 0, fh_flag = 0;
+    double fit_es[3] = {1, 1, 1}, fit_fs[3] = {1, 1, 1};
+    int sg_probe_blocks = 0;
+    std::vector<int32_t> fh_probed;  // device faces whose id carries fh_flag
     std::vector<double> h_ca_common, h_cb_common;
     DevBuf sp_edge, sp_f4, sp_sg, sp_ca, sp_cb, sp_kind, sp_tb, sp_te;
     int32_t n_sp = 0;
@@ -348,6 +349,9 @@ struct tf_ctx {
     bool energy_out = false;
     int64_t sample_cap = 0, n_samples = 0;
     std::vector<double> sample_times;
+    // sampling inside the steps (plan_samples): sample slot per step of the
+    // run (row 0: the step before it) and what the kernels write to
+    DevBuf slots, samp_ref;
     double next_print = 0, period = 0;
     bool out_enabled = false;
     bool initial_done = false;
@@ -365,7 +369,7 @@ struct tf_ctx {
     struct StepGraph {
         hipGraph_t graph = nullptr;
         hipGraphExec_t exec = nullptr;
-        DevBuf carr, poy;
+        DevBuf carr, poy, slot;
     };
     StepGraph sg;
     int sg_fcur = 0;  // lossy dga: fcur when sg was captured
@@ -395,7 +399,8 @@ tf_ctx::~tf_ctx() {
 
 size_t tf_ctx::device_bytes() const {
     size_t s = 0;
-    const DevBuf* all[] = {&U, &Fv, &B, &fit_ep, &fit_nu, &fe_sg, &fe_ca, &fe_cb, &fe_f4, &fh_sg, &fh_cm, &fh_cn, &fh_e4, &fe_code, &fh_code, &fe_id, &fe_pal, &fh_id, &fh_pal, &fh_at, &fh_val,
+    const DevBuf* all[] = {&U, &Fv, &B, &fit_ep, &fit_nu, &fe_sg, &fe_ca, &fe_cb, &fe_f4, &fh_sg, &fh_cm, &fh_cn, &fh_e4, &fe_id, &fe_pal, &fh_id, &fh_pal, &fh_at, &fh_val,
+                           &spv, &slots, &samp_ref, &sg.carr, &sg.poy, &sg.slot,
                            &sp_edge, &sp_f4, &sp_sg, &sp_ca, &sp_cb, &sp_kind, &sp_tb, &sp_te, &c_col, &c_sg,
                            &h_edge, &curl_f, &curl_u, &free_edge, &edge_row, &dir_edge, &dir_new, &fb, &pre, &x, &r, &rs0, &rs1, &z,
                            &p0, &p1, &q, &r0, &hx1, &hx2, &dx, &rr0part, &cg_part, &cg_state, &inj_edge, &inj_kind, &inj_tb, &inj_te,
@@ -855,13 +860,14 @@ void ev_flush(tf_ctx* c) {
 
 // ---------------------------------------------------------------- create
 
-// Grid order for a FIT problem that carries grid positions: the slot map of
-// every common edge and tbc face (which slot holds the reference's face /
-// edge at each position, fit_edge_slots / fit_face_slots). False (the
-// index-table layout is used) if any of them does not have exactly its
-// slots' entities, or $TETFIT_FIT_INDEXED is set to a non-empty value other
-// than 0.
-bool fit_grid_codes(tf_ctx* c, const tf_fit_ops& f, std::vector<uint16_t>& ecode, std::vector<uint16_t>& fcode) {
+// Grid order for a FIT problem that carries grid positions: used when every
+// common edge and tbc face has exactly its slots' entities (fit_edge_slots /
+// fit_face_slots) in the order 0, 2, 3, 1 and one sign per direction, as the
+// mesher numbers them (D:4643-5080). eon / fon: 1 for the entities at each
+// position that the main pass updates. False (the index-table layout is used)
+// otherwise, or if $TETFIT_FIT_INDEXED is set to a non-empty value other than
+// 0.
+bool fit_grid_positions(tf_ctx* c, const tf_fit_ops& f, std::vector<uint8_t>& eon, std::vector<uint8_t>& fon) {
     const char* forced = std::getenv("TETFIT_FIT_INDEXED");
     if (forced && *forced && std::strcmp(forced, "0") != 0) return false;
     if (!f.edge_sid || !f.face_sid) return false;
@@ -883,43 +889,40 @@ bool fit_grid_codes(tf_ctx* c, const tf_fit_ops& f, std::vector<uint16_t>& ecode
         for (int32_t v : esid) { if (v < 0 || v >= E || seen_e[v]) return false; seen_e[v] = 1; }
         for (int32_t v : fsid) { if (v < 0 || v >= F || seen_f[v]) return false; seen_f[v] = 1; }
     }
-    auto map_of = [](const int32_t slot[4], const int64_t ref[4], uint32_t& m) {
-        m = 0;
-        for (int q = 0; q < 4; ++q) {
-            int hit = -1;
-            for (int k = 0; k < 4; ++k)
-                if (slot[k] == ref[q]) { if (hit >= 0) return false; hit = k; }
-            if (hit < 0) return false;
-            m |= (uint32_t)hit << (2 * q);
-        }
-        return true;
+    const int order[4] = {0, 2, 3, 1};
+    // sign of each direction's sums: that of its first entity
+    double es[3] = {0, 0, 0}, fs[3] = {0, 0, 0};
+    const int64_t eoff[2] = {nx * (ny + 1) * (nz + 1), nx * (ny + 1) * (nz + 1) + (nx + 1) * ny * (nz + 1)};
+    const int64_t foff[2] = {(nx + 1) * ny * nz, (nx + 1) * ny * nz + nx * (ny + 1) * nz};
+    auto same_sign = [](double& have, int d) {
+        if (d != 1 && d != -1) return false;
+        if (have == 0) have = d;
+        return have == d;
     };
-    ecode.assign(E, 0);
+    eon.assign(E, 0);
     for (int64_t q = 0; q < f.n_common; ++q) {
         const int32_t e = f.common_edges[q];
         if (f.ct_ptr[e + 1] - f.ct_ptr[e] != 4) return false;
         int32_t slot[4];
-        int64_t ref[4];
         fit_edge_slots(g, (uint32_t)esid[e], slot);
-        for (int k = 0; k < 4; ++k) ref[k] = fsid[f.ct_face[f.ct_ptr[e] + k]];
-        uint32_t m;
-        if (!map_of(slot, ref, m)) return false;
-        const int d = f.dual_curl[e];
-        const int sg[4] = {d, -d, d, -d};
-        ecode[esid[e]] = (uint16_t)(m << 8 | code4(sg));
+        for (int k = 0; k < 4; ++k)
+            if (fsid[f.ct_face[f.ct_ptr[e] + k]] != slot[order[k]]) return false;
+        if (!same_sign(es[(esid[e] >= eoff[0]) + (esid[e] >= eoff[1])], f.dual_curl[e])) return false;
+        eon[esid[e]] = 1;
     }
-    fcode.assign(F, 0);
+    fon.assign(F, 0);
     for (int64_t q = 0; q < f.n_tbc; ++q) {
         const int32_t fi = f.tbc_faces[q];
         int32_t slot[4];
-        int64_t ref[4];
         fit_face_slots(g, (uint32_t)fsid[fi], slot);
-        for (int k = 0; k < 4; ++k) ref[k] = esid[f.c_edge[4 * (int64_t)fi + k]];
-        uint32_t m;
-        if (!map_of(slot, ref, m)) return false;
-        const int d = f.curl[fi];
-        const int sg[4] = {d, -d, d, -d};
-        fcode[fsid[fi]] = (uint16_t)(m << 8 | code4(sg));
+        for (int k = 0; k < 4; ++k)
+            if (esid[f.c_edge[4 * (int64_t)fi + k]] != slot[order[k]]) return false;
+        if (!same_sign(fs[(fsid[fi] >= foff[0]) + (fsid[fi] >= foff[1])], f.curl[fi])) return false;
+        fon[fsid[fi]] = 1;
+    }
+    for (int k = 0; k < 3; ++k) {
+        c->fit_es[k] = es[k];
+        c->fit_fs[k] = fs[k];
     }
     c->grid = g;
     c->h_esid = std::move(esid);
@@ -927,20 +930,16 @@ bool fit_grid_codes(tf_ctx* c, const tf_fit_ops& f, std::vector<uint16_t>& ecode
     return true;
 }
 
-// Palette of the entities' (code, a, b) triples (device order; bitwise
-// distinct values): id per entity, 0 for code 0. False when there are more
-// than kPalMax: at 161^3 a random medium's E side (every cell its own eps_r)
-// gives one triple per edge and keeps the plain arrays, 42 bytes an edge,
-// while a cavity's holds a few dozen.
-constexpr size_t kPalMax = 32767;
+// Palette of the entities' coefficient pairs (device order; bitwise distinct
+// values): id per entity, 0 where on is 0. When there are more than kPalMax
+// the ids are 1 and pal stays empty (plain arrays).
 template <class T>
-bool fit_palette(const std::vector<uint16_t>& code, const std::vector<T>& a, const std::vector<T>& b,
+void fit_palette(const std::vector<uint8_t>& on, const std::vector<T>& a, const std::vector<T>& b,
                  std::vector<uint16_t>& id, std::vector<FitPal<T>>& pal) {
     struct Key {
         T a, b;
-        uint32_t code;
         bool operator==(const Key& o) const {
-            return code == o.code && !std::memcmp(&a, &o.a, sizeof(T)) && !std::memcmp(&b, &o.b, sizeof(T));
+            return !std::memcmp(&a, &o.a, sizeof(T)) && !std::memcmp(&b, &o.b, sizeof(T));
         }
     };
     struct Hash {
@@ -948,36 +947,39 @@ bool fit_palette(const std::vector<uint16_t>& code, const std::vector<T>& a, con
             uint64_t x = 0, y = 0;
             std::memcpy(&x, &k.a, sizeof(T));
             std::memcpy(&y, &k.b, sizeof(T));
-            uint64_t h = (x ^ (y * 0x9E3779B97F4A7C15ull)) + k.code;
+            uint64_t h = x ^ (y * 0x9E3779B97F4A7C15ull);
             h ^= h >> 32;
             h *= 0x9E3779B97F4A7C15ull;
             return (size_t)(h ^ (h >> 29));
         }
     };
     std::unordered_map<Key, uint16_t, Hash> seen;
-    id.assign(code.size(), 0);
-    pal.assign(1, FitPal<T>{0, 0, 0});
-    Key last{0, 0, 0};
+    id.assign(on.size(), 0);
+    pal.assign(1, FitPal<T>{0, 0});
+    Key last{0, 0};
     uint16_t last_id = 0;
-    for (size_t i = 0; i < code.size(); ++i) {
-        if (code[i] == 0) continue;
-        const Key k{a[i], b[i], code[i]};
-        if (!(k == last)) {
+    for (size_t i = 0; i < on.size(); ++i) {
+        if (!on[i]) continue;
+        const Key k{a[i], b[i]};
+        if (last_id == 0 || !(k == last)) {
             auto it = seen.find(k);
             if (it == seen.end()) {
-                if (pal.size() > kPalMax) return false;
+                if (pal.size() >= (size_t)kPalMax) {
+                    pal.clear();
+                    for (size_t q = 0; q < on.size(); ++q) id[q] = on[q];
+                    return;
+                }
                 it = seen.emplace(k, (uint16_t)pal.size()).first;
-                pal.push_back(FitPal<T>{k.a, k.b, k.code});
+                pal.push_back(FitPal<T>{k.a, k.b});
             }
             last = k;
             last_id = it->second;
         }
         id[i] = last_id;
     }
-    return true;
 }
 
-// Marks the faces that the probes read as stored every step (FIT palette).
+// Marks the faces that the probes read as stored every step (FIT grid order).
 void fit_probe_faces(tf_ctx* c, const std::vector<int32_t>& faces) {
     if (!c->fh_id.p) return;
     std::vector<int32_t> at;
@@ -994,7 +996,7 @@ void fit_probe_faces(tf_ctx* c, const std::vector<int32_t>& faces) {
     for (int32_t f : now)
         if (c->h_fh_id[f]) {
             at.push_back(f);
-            val.push_back((uint16_t)(c->h_fh_id[f] + c->fh_k));
+            val.push_back((uint16_t)(c->h_fh_id[f] + c->fh_flag));
         }
     c->fh_probed = now;
     // two launches in stream order: a face may be in both lists
@@ -1014,8 +1016,8 @@ template <class T>
 void create_fit(tf_ctx* c, const tf_problem* p) {
     const tf_fit_ops& f = p->fit;
     const int32_t E = c->E, F = c->F;
-    std::vector<uint16_t> ecode, fcode;
-    c->fit_grid = fit_grid_codes(c, f, ecode, fcode);
+    std::vector<uint8_t> eon, fon;
+    c->fit_grid = fit_grid_positions(c, f, eon, fon);
     // per-entity arrays in device order
     auto by_edge = [&](auto v) {
         if (!c->fit_grid) return v;
@@ -1060,13 +1062,11 @@ void create_fit(tf_ctx* c, const tf_problem* p) {
     if (c->fit_grid) {
         const std::vector<T> a = by_edge(ca), b = by_edge(cb);
         std::vector<FitPal<T>> pal;
-        if (fit_palette(ecode, a, b, c->h_fe_id, pal)) {
-            upload(c->fe_id, c->h_fe_id);
+        fit_palette(eon, a, b, c->h_fe_id, pal);
+        c->fe_n = (int32_t)pal.size();
+        if (!pal.empty()) {
             upload(c->fe_pal, pal);
         } else {
-            c->h_fe_id.clear();
-            c->h_fe_code = ecode;
-            upload(c->fe_code, ecode);
             upload(c->fe_ca, a);
             upload(c->fe_cb, b);
         }
@@ -1113,21 +1113,15 @@ void create_fit(tf_ctx* c, const tf_problem* p) {
     if (c->fit_grid) {
         const std::vector<T> a = by_face(cm), b = by_face(cn);
         std::vector<FitPal<T>> pal;
-        if (fit_palette(fcode, a, b, c->h_fh_id, pal)) {
-            c->fh_k = (int32_t)pal.size();
-            pal.resize(2 * (size_t)c->fh_k);
-            for (int32_t k = 0; k < c->fh_k; ++k) {
-                pal[c->fh_k + k] = pal[k];
-                pal[c->fh_k + k].code |= kStoreB;
-            }
-            upload(c->fh_id, c->h_fh_id);
+        fit_palette(fon, a, b, c->h_fh_id, pal);
+        c->fh_flag = pal.empty() ? 2 : (int32_t)pal.size();
+        if (!pal.empty()) {
             upload(c->fh_pal, pal);
         } else {
-            c->h_fh_id.clear();
-            upload(c->fh_code, fcode);
             upload(c->fh_cm, a);
             upload(c->fh_cn, b);
         }
+        upload(c->fh_id, c->h_fh_id);
     } else {
         upload(c->fh_sg, hs);
         upload(c->fh_cm, cm);
@@ -1501,10 +1495,9 @@ void build_fit_special(tf_ctx* c, const std::vector<std::vector<std::pair<int32_
     std::vector<double> ca, cb, tw;
     std::vector<int8_t> kind;
     std::vector<uint8_t> main_sg = c->h_fe_sg;
-    // main pass codes, or palette ids (both 0 for an edge left out)
-    std::vector<uint16_t> main_code = c->fe_id.p ? c->h_fe_id : c->h_fe_code;
+    std::vector<uint16_t> main_id = c->h_fe_id;
     auto off_main = [&](int32_t e) {  // the special item updates it
-        if (c->fit_grid) main_code[c->h_esid[e]] = 0;
+        if (c->fit_grid) main_id[c->h_esid[e]] = 0;
         else main_sg[e] = 0;
     };
     auto dev_f4 = [&](int4 q) {
@@ -1558,8 +1551,12 @@ void build_fit_special(tf_ctx* c, const std::vector<std::vector<std::pair<int32_
     if (tsrc.empty()) { tsrc.push_back(0); tw.push_back(0); }
     upload(c->term_src, tsrc);
     upload(c->term_w, tw);
-    if (c->fit_grid) upload(c->fe_id.p ? c->fe_id : c->fe_code, main_code);
-    else upload(c->fe_sg, main_sg);
+    if (c->fit_grid) {
+        upload(c->fe_id, main_id);
+        c->spv.alloc(std::max(c->n_sp, 1) * sizeof(double));
+    } else {
+        upload(c->fe_sg, main_sg);
+    }
 }
 
 void build_tet_inject(tf_ctx* c, const std::vector<std::vector<std::pair<int32_t, double>>>& by_edge_terms,
@@ -1693,11 +1690,12 @@ void sample(tf_ctx* c, double t) {
 }
 
 void ensure_carr(tf_ctx* c, int64_t first, int64_t n) {
-    // carriers for steps first-1 .. first+n-1 (row 0 is the previous step)
+    // carriers for steps first-1 .. first+n (row 0 is the previous step; a
+    // FIT step prepares the next one's source values)
     const size_t ns = std::max<size_t>(c->src.size(), 1);
-    std::vector<double> tab((size_t)(n + 1) * ns, 0.0);
+    std::vector<double> tab((size_t)(n + 2) * ns, 0.0);
     const bool per_src = c->src_dt.size() == c->src.size();
-    for (int64_t k = 0; k <= n; ++k) {
+    for (int64_t k = 0; k <= n + 1; ++k) {
         const int64_t i = first - 1 + k;
         for (size_t s = 0; s < c->src.size(); ++s) {
             const tf_source& so = c->src[s];
@@ -1737,17 +1735,19 @@ bool graph_steps(const tf_ctx* c) {
 // partials per step. Returns the number of steps run (a multiple of
 // kGraphSteps); the caller runs the rest with ordinary launches.
 template <class Step>
-int64_t run_graph_chunks(tf_ctx* c, int64_t first_k, int64_t m, int per_step, Step step) {
+int64_t run_graph_chunks(tf_ctx* c, int64_t first_k, int64_t m, int per_step, bool sampled, Step step) {
     const int64_t chunks = m / kGraphSteps;
     if (chunks == 0) return 0;
     const size_t ns = std::max<size_t>(c->src.size(), 1);
     if (!c->sg.exec) {
-        c->sg.carr.alloc((kGraphSteps + 1) * ns * sizeof(double));
+        c->sg.carr.alloc((kGraphSteps + 2) * ns * sizeof(double));
         c->sg.poy.alloc(std::max(1, kGraphSteps * per_step) * sizeof(double));
+        c->sg.slot.alloc((kGraphSteps + 1) * sizeof(int64_t));
         TF_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
         try {
             for (int k = 0; k < kGraphSteps; ++k)
-                step(k, c->sg.carr.as<double>() + (size_t)(k + 1) * ns, c->sg.poy.as<double>() + (size_t)k * per_step);
+                step(k, c->sg.carr.as<double>() + (size_t)(k + 1) * ns, c->sg.poy.as<double>() + (size_t)k * per_step,
+                     c->sg.slot.as<int64_t>() + k);
         } catch (...) {
             hipGraph_t g = nullptr;
             (void)hipStreamEndCapture(c->stream, &g);
@@ -1759,9 +1759,13 @@ int64_t run_graph_chunks(tf_ctx* c, int64_t first_k, int64_t m, int per_step, St
     }
     for (int64_t q = 0; q < chunks; ++q) {
         const int64_t k0 = first_k + q * kGraphSteps;
-        // carrier rows k0 .. k0 + kGraphSteps of this run (row 0 = the step before)
+        // carrier rows k0 .. k0 + kGraphSteps + 1 of this run (row 0 = the step
+        // before) and, when it samples, the slot rows k0 .. k0 + kGraphSteps
         TF_HIP(hipMemcpyAsync(c->sg.carr.p, c->carr.as<double>() + (size_t)k0 * ns,
-                              (kGraphSteps + 1) * ns * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
+                              (kGraphSteps + 2) * ns * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
+        if (sampled)
+            TF_HIP(hipMemcpyAsync(c->sg.slot.p, c->slots.as<int64_t>() + k0, (kGraphSteps + 1) * sizeof(int64_t),
+                                  hipMemcpyDeviceToDevice, c->stream));
         TF_HIP(hipGraphLaunch(c->sg.exec, c->stream));
         if (per_step)
             TF_HIP(hipMemcpyAsync(c->poy.as<double>() + (size_t)k0 * per_step, c->sg.poy.p,
@@ -1771,47 +1775,156 @@ int64_t run_graph_chunks(tf_ctx* c, int64_t first_k, int64_t m, int per_step, St
     return chunks * kGraphSteps;
 }
 
+// Output samples of steps [first, first + n) that the steps' own kernels
+// take: a slot per step in c->slots (row k + 1: step first + k; row 0, the step
+// before the run, has none: its sample was taken then) and the sample
+// reference. Returns whether the run samples probes.
+bool plan_samples(tf_ctx* c, int64_t first, int64_t n) {
+    std::vector<int64_t> slot((size_t)n + 1, -1);
+    for (int64_t k = 0; k < n; ++k) {
+        const double t = (double)(first + k) * c->dt;
+        if (want_sample(c, first + k, t)) slot[k + 1] = sample_reserve(c, t);
+    }
+    if (c->n_probes == 0 || !(c->batch ? c->batch->every > 0 : c->out_enabled)) return false;
+    const SampleRef ref{c->probes.as<ProbeDev>(), c->samples.as<double>(), c->n_probes};
+    if (c->slots.bytes < slot.size() * sizeof(int64_t)) c->slots.alloc(slot.size() * sizeof(int64_t));
+    if (!c->samp_ref.p) c->samp_ref.alloc(sizeof(SampleRef));
+    TF_HIP(hipMemcpyAsync(c->slots.p, slot.data(), slot.size() * sizeof(int64_t), hipMemcpyHostToDevice, c->stream));
+    TF_HIP(hipMemcpyAsync(c->samp_ref.p, &ref, sizeof(ref), hipMemcpyHostToDevice, c->stream));
+    TF_HIP(hipStreamSynchronize(c->stream));
+    return true;
+}
+
+FitSpecial fit_special_view(const tf_ctx* c) {
+    return FitSpecial{c->n_sp,
+                      c->sp_edge.as<int32_t>(),
+                      c->sp_f4.as<int4>(),
+                      c->sp_sg.as<uint8_t>(),
+                      c->sp_ca.as<double>(),
+                      c->sp_cb.as<double>(),
+                      c->sp_kind.as<int8_t>(),
+                      c->sp_tb.as<int32_t>(),
+                      c->sp_te.as<int32_t>(),
+                      c->term_src.as<int32_t>(),
+                      c->term_w.as<double>()};
+}
+
+// One step of the index-table layout: E phase (with sources and the Poynting
+// partials), H phase.
+template <class T>
+void fit_indexed_step(tf_ctx* c, const FitSpecial& sp, int sp_blocks, const double* cs, double* poy) {
+    launch_timed(c, "fit_e_kernel", fit_e_kernel<T>, blocks_for(c->E) + sp_blocks, c->E, sp_blocks,
+                 c->fe_sg.as<uint8_t>(), c->fe_ca.as<T>(), c->fe_cb.as<T>(), c->fe_f4.as<int4>(), c->Fv.as<T>(),
+                 c->U.as<T>(), sp, cs, sp_blocks ? poy : nullptr);
+    launch_timed(c, "fit_h_kernel", fit_h_kernel<T>, blocks_for(c->F), c->F, c->fh_sg.as<uint8_t>(), c->fh_cm.as<T>(),
+                 c->fh_cn.as<T>(), c->fh_e4.as<int4>(), c->U.as<T>(), c->Fv.as<T>(), c->B.as<T>(), c->dt);
+}
+
+// Items per thread of the grid-order kernels. Two (against one) took 12.1
+// instead of 12.4 us a step at 64^3 fp64, 22.5 instead of 24.7 at 90^3 and 163
+// instead of 185 at 161^3 random fp64; four gain only where an item's loads are
+// 4 bytes and the grid is large: 128^3 fp32 33.1 against 35.3 us, 161^3 fp64
+// 168 against 163, 48^3 fp32 8.7 against 8.3.
+template <class T>
+int fit_items(int64_t edges) {
+    return sizeof(T) == 4 && edges >= (1 << 22) ? 4 : 2;
+}
+
 template <class T>
 void run_fit(tf_ctx* c, int64_t first, int64_t n, tf_stats* st) {
-    uint32_t ecnt[3], fcnt[3];
-    fit_counts(c->grid, false, ecnt);
-    fit_counts(c->grid, true, fcnt);
-    const int main_blocks = c->fit_grid ? slab_grid(ecnt) : blocks_for(c->E);
-    const int h_blocks = c->fit_grid ? slab_grid(fcnt) : blocks_for(c->F);
     const int sp_blocks = c->n_sp ? blocks_for(c->n_sp) : 0;
     const size_t ns = std::max<size_t>(c->src.size(), 1);
-    if (sp_blocks) {
-        if (c->poy_cap < n * sp_blocks) {
-            c->poy.alloc(n * sp_blocks * sizeof(double));
-            c->poy_cap = n * sp_blocks;
-        }
+    if (sp_blocks && c->poy_cap < n * sp_blocks) {
+        c->poy.alloc(n * sp_blocks * sizeof(double));
+        c->poy_cap = n * sp_blocks;
     }
-    // one step: E phase (with sources and the Poynting partials), H phase
-    auto step = [&](const double* cs, double* poy, bool store_b) {
-        launch_timed(c, "fit_e_kernel", fit_e_kernel<T>, main_blocks + sp_blocks,
-            c->E, sp_blocks, c->fe_sg.as<uint8_t>(), c->fe_ca.as<T>(), c->fe_cb.as<T>(), c->fe_f4.as<int4>(),
-            c->fit_grid ? c->fe_code.as<uint16_t>() : nullptr, c->fe_id.as<uint16_t>(), c->fe_pal.as<FitPal<T>>(),
-            c->grid, c->Fv.as<T>(), c->U.as<T>(), c->n_sp, c->sp_edge.as<int32_t>(), c->sp_f4.as<int4>(),
-            c->sp_sg.as<uint8_t>(), c->sp_ca.as<double>(), c->sp_cb.as<double>(), c->sp_kind.as<int8_t>(),
-            c->sp_tb.as<int32_t>(), c->sp_te.as<int32_t>(), c->term_src.as<int32_t>(), c->term_w.as<double>(), cs,
-            sp_blocks ? poy : nullptr);
-        launch_timed(c, "fit_h_kernel", fit_h_kernel<T>, h_blocks, c->F, c->fh_sg.as<uint8_t>(),
-                     c->fh_cm.as<T>(), c->fh_cn.as<T>(), c->fh_e4.as<int4>(),
-                     c->fit_grid ? c->fh_code.as<uint16_t>() : nullptr, c->fh_id.as<uint16_t>(),
-                     c->fh_pal.as<FitPal<T>>(), store_b ? 1 : 0, c->grid, c->U.as<T>(), c->Fv.as<T>(), c->B.as<T>(),
-                     c->dt);
-    };
-    const int64_t g = graph_steps(c) ? run_graph_chunks(c, 0, n, sp_blocks, [&](int k, const double* cs, double* poy) {
-        step(cs, poy, k == kGraphSteps - 1);
-    }) : 0;
-    for (int64_t k = g; k < n; ++k) {
-        const int64_t i = first + k;
-        const double t = (double)i * c->dt;
-        const bool print = allow_print(c, t);
-        step(c->carr.as<double>() + (k + 1) * ns, c->poy.as<double>() + k * sp_blocks,
-             k == n - 1 || (print && c->energy_out));
-        if (print) sample<T>(c, t);
-        if (c->profiling && (k & 63) == 63) ev_flush(c);
+    const FitSpecial sp = fit_special_view(c);
+    if (!c->fit_grid) {
+        const int64_t g = graph_steps(c) ? run_graph_chunks(c, 0, n, sp_blocks, false,
+                                                            [&](int, const double* cs, double* poy, const int64_t*) {
+            fit_indexed_step<T>(c, sp, sp_blocks, cs, poy);
+        }) : 0;
+        for (int64_t k = g; k < n; ++k) {
+            const double t = (double)(first + k) * c->dt;
+            fit_indexed_step<T>(c, sp, sp_blocks, c->carr.as<double>() + (k + 1) * ns,
+                                c->poy.as<double>() + k * sp_blocks);
+            if (allow_print(c, t)) sample<T>(c, t);
+            if (c->profiling && (k & 63) == 63) ev_flush(c);
+        }
+    } else {
+        // energy samples reduce the fields between steps, from the host
+        const bool inside = !c->energy_out && plan_samples(c, first, n);
+        FitStep<T> e{};
+        e.g = c->grid;
+        e.sp_blocks = sp_blocks;
+        e.probe_blocks = inside ? blocks_for((int64_t)c->n_probes * 3) : 0;
+        e.sp = sp;
+        e.spv = c->spv.as<double>();
+        e.ref = c->samp_ref.as<SampleRef>();
+        FitStep<T> h = e;
+        h.src_blocks = sp_blocks;
+        h.spv_next = c->spv.as<double>();
+        e.n_pal = c->fe_n;
+        e.id = c->fe_id.as<uint16_t>();
+        e.pal = c->fe_pal.as<FitPal<T>>();
+        e.c0 = c->fe_ca.as<T>();
+        e.c1 = c->fe_cb.as<T>();
+        h.n_pal = c->fh_flag;
+        h.flag = (uint32_t)c->fh_flag;
+        h.id = c->fh_id.as<uint16_t>();
+        h.pal = c->fh_pal.as<FitPal<T>>();
+        h.c0 = c->fh_cm.as<T>();
+        h.c1 = c->fh_cn.as<T>();
+        for (int d = 0; d < 3; ++d) {
+            e.sg[d] = c->fit_es[d];
+            h.sg[d] = c->fit_fs[d] * c->dt;
+        }
+        uint32_t ecnt[3], fcnt[3];
+        fit_counts(c->grid, false, ecnt);
+        fit_counts(c->grid, true, fcnt);
+        // items per thread
+        const int per = fit_items<T>(c->E);
+        const int e_grid = sp_blocks + e.probe_blocks + slab_grid(ecnt, per * kBlock);
+        const int h_grid = sp_blocks + h.probe_blocks + slab_grid(fcnt, per * kBlock);
+        const auto ek = per == 2 ? (c->fe_pal.p ? fit_e_grid_kernel<T, true, 2> : fit_e_grid_kernel<T, false, 2>)
+                                 : (c->fe_pal.p ? fit_e_grid_kernel<T, true, 4> : fit_e_grid_kernel<T, false, 4>);
+        const auto hk = per == 2 ? (c->fh_pal.p ? fit_h_grid_kernel<T, true, 2> : fit_h_grid_kernel<T, false, 2>)
+                                 : (c->fh_pal.p ? fit_h_grid_kernel<T, true, 4> : fit_h_grid_kernel<T, false, 4>);
+        // slot: row of the step before (its B is sampled by the E phase)
+        auto step = [&](const double* cs, double* poy, const int64_t* slot, bool store_b) {
+            e.poy_part = poy;
+            e.slot = slot;
+            launch_timed(c, "fit_e_kernel", ek, e_grid, e, (const T*)c->Fv.as<T>(), c->U.as<T>(),
+                         (const T*)c->B.as<T>());
+            h.carr_next = cs + ns;
+            h.slot = slot + 1;
+            launch_timed(c, "fit_h_kernel", hk, h_grid, h, store_b ? 1 : 0, (const T*)c->U.as<T>(), c->Fv.as<T>(),
+                         c->B.as<T>());
+        };
+        if (sp_blocks)
+            fit_src_kernel<<<sp_blocks, kBlock, 0, c->stream>>>(sp, c->carr.as<double>() + ns, c->spv.as<double>());
+        int64_t k0 = 0;
+        if (c->use_graphs && !c->profiling && !(c->out_enabled && c->energy_out)) {
+            // a captured step samples with so many workgroups
+            if (c->sg.exec && c->sg_probe_blocks != e.probe_blocks) drop_graph(c);
+            c->sg_probe_blocks = e.probe_blocks;
+            k0 = run_graph_chunks(c, 0, n, sp_blocks, inside,
+                                  [&](int k, const double* cs, double* poy, const int64_t* slot) {
+                                      step(cs, poy, slot, k == kGraphSteps - 1);
+                                  });
+        }
+        for (int64_t k = k0; k < n; ++k) {
+            const double t = (double)(first + k) * c->dt;
+            const bool print = c->energy_out && allow_print(c, t);
+            step(c->carr.as<double>() + (k + 1) * ns, c->poy.as<double>() + k * sp_blocks,
+                 c->slots.as<int64_t>() + k, k == n - 1 || print);
+            if (print) sample<T>(c, t);
+            if (c->profiling && (k & 63) == 63) ev_flush(c);
+        }
+        // the B part of the last step's sample: no E phase follows it in this run
+        if (inside)
+            probe_tail_kernel<T><<<e.probe_blocks, kBlock, 0, c->stream>>>(e.ref, c->slots.as<int64_t>() + n, 3, 3,
+                                                                         c->U.as<T>(), c->B.as<T>());
     }
     TF_HIP(hipGetLastError());
     // Poynting per step
@@ -1927,7 +2040,8 @@ void run_dga_frac(tf_ctx* c, int64_t first, int64_t n, tf_stats* st) {
     if (graph_steps(c)) {
         if (c->sg.exec && c->sg_fcur != c->fcur && n > 0) host_step(h++);
         if (!c->sg.exec) c->sg_fcur = c->fcur;
-        h += run_graph_chunks(c, h, n - h, 2 * inj_blocks, [&](int, const double* cs, double* poy) { step(cs, poy); });
+        h += run_graph_chunks(c, h, n - h, 2 * inj_blocks, false,
+                              [&](int, const double* cs, double* poy, const int64_t*) { step(cs, poy); });
     }
     for (; h < n; ++h) host_step(h);
     TF_HIP(hipGetLastError());
@@ -1998,7 +2112,8 @@ void run_dga(tf_ctx* c, int64_t first, int64_t n, tf_stats* st) {
         TF_LAUNCH_TIMED(c, "sell_n_kernel", c->tune[TK_N].unroll, sell_n_kernel, T, gb_n,
                         tuned_view(c, TK_N, c->N.vals<T>()), c->curl_u.as<T>(), c->Fv.as<T>(), c->dt, 0, fdt, nullptr);
     };
-    const int64_t g = graph_steps(c) ? run_graph_chunks(c, 0, n, per_step, [&](int, const double* cs, double* poy) {
+    const int64_t g = graph_steps(c) ? run_graph_chunks(c, 0, n, per_step, false,
+                                                        [&](int, const double* cs, double* poy, const int64_t*) {
         step(cs, poy);
     }) : 0;
     for (int64_t k = g; k < n; ++k) {
