@@ -426,6 +426,16 @@ __device__ __forceinline__ void sample_probes(const SampleRef* __restrict__ ref,
     r.out[(sl * r.n_probes + p) * 6 + c] = probe_value<T>(r.probes[p], c, U, B);
 }
 
+// A sample taken by workgroups appended to another kernel's grid.
+template <typename T>
+struct SampleArgs {
+    int32_t blocks = 0;
+    const SampleRef* ref = nullptr;
+    const int64_t* slot = nullptr;
+    const T* U = nullptr;
+    const T* B = nullptr;
+};
+
 template <typename T>
 __global__ void __launch_bounds__(kBlock) probe_tail_kernel(const SampleRef* __restrict__ ref,
                                                             const int64_t* __restrict__ slot, int c0, int nc,
@@ -676,39 +686,68 @@ __global__ void __launch_bounds__(kBlock) fit_h_grid_kernel(FitStep<T> a, int st
 }
 
 // ------------------------------------------------------------------ DGA
-// Source injection for the tetrahedral methods: h sources add Fb to curl_f
-// (Ctb*Fb, one +1 per boundary edge), e sources set U (class-4 edges).
-// The Poynting partial uses U before the E update: 0.5*U_old*fb.
+// Sources of the lossless dga step. h sources add Fb to curl_f (Ctb Fb, one +1
+// per boundary edge), e sources set U (class-4 edges). As a kernel between
+// sell_ct and sell_h they cost a launch of 4.2 us a step; now the h values of a
+// step are left by the step before, in fp64, at 64 slots per Ct slice that has
+// any (fbv, fb_pos), and sell_ct adds them to its rows, while workgroups
+// appended to it set the e values and form the first Poynting half.
+struct InjItems {
+    int32_t n = 0;
+    const int32_t* edge = nullptr;
+    const int8_t* kind = nullptr;
+    const int32_t* tb = nullptr;
+    const int32_t* te = nullptr;
+    const int32_t* term_src = nullptr;
+    const double* term_w = nullptr;
+};
+__device__ __forceinline__ double inj_value(const InjItems& q, int32_t i, const double* __restrict__ carr) {
+    return source_value(q.tb[i], q.te[i], q.term_src, q.term_w, carr);
+}
 template <typename T>
-__global__ void __launch_bounds__(kBlock) dga_inject_kernel(
-    int32_t n_inj, const int32_t* __restrict__ inj_edge, const int8_t* __restrict__ inj_kind,
-    const int32_t* __restrict__ inj_tb, const int32_t* __restrict__ inj_te, const int32_t* __restrict__ term_src,
-    const double* __restrict__ term_w, const double* __restrict__ carr_step, T* __restrict__ curl_f,
-    T* __restrict__ U, double* __restrict__ poy_part, int init) {
-    __shared__ double red[kBlock / kWave];
-    const int32_t i = blockIdx.x * kBlock + threadIdx.x;
+struct CtSources {
+    int32_t blocks = 0;                    // appended workgroups
+    InjItems q;
+    const int32_t* slice_slot = nullptr;   // per Ct slice: its slot of fbv, or -1 (null: no h sources)
+    const int32_t* fb_pos = nullptr;       // per item
+    const double* fbv = nullptr;
+    const double* carr_step = nullptr;
+    T* U = nullptr;
+    double* poy_part = nullptr;
+};
+template <typename T>
+__device__ __forceinline__ void ct_source_block(const CtSources<T>& a, int32_t blk, double* red) {
+    const int32_t i = blk * kBlock + (int32_t)threadIdx.x;
     double poy = 0;
-    if (i < n_inj) {
-        const int32_t e = inj_edge[i];
-        const double v = source_value(inj_tb[i], inj_te[i], term_src, term_w, carr_step);
-        if (init && inj_kind[i] == 0) {
-            // before the loop every source edge takes its e-source sum at
-            // t = 0 (D:746-765), which is 0 on an h edge
-            U[e] = (T)0;
-        } else if (inj_kind[i] == 0) {
-            curl_f[e] = (T)((double)curl_f[e] + v);
-            poy = 0.5 * (double)U[e] * v;
-        } else {
-            U[e] = (T)v;
-        }
+    if (i < a.q.n) {
+        const int32_t e = a.q.edge[i];
+        // the Poynting partial uses U before the E update: 0.5*U_old*fb
+        if (a.q.kind[i] == 0) poy = 0.5 * (double)a.U[e] * a.fbv[a.fb_pos[i]];
+        else a.U[e] = (T)inj_value(a.q, i, a.carr_step);
     }
     const double s = block_sum(poy, red);
-    if (threadIdx.x == 0) poy_part[blockIdx.x] = s;
+    if (threadIdx.x == 0) a.poy_part[blk] = s;
+}
+
+// The h values of the first step of a run.
+__global__ void __launch_bounds__(kBlock) dga_src_kernel(InjItems q, const int32_t* __restrict__ fb_pos,
+                                                         const double* __restrict__ carr, double* __restrict__ fbv) {
+    const int32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < q.n && q.kind[i] == 0) fbv[fb_pos[i]] = inj_value(q, i, carr);
+}
+
+// Before the loop every source edge takes its e-source sum at t = 0
+// (D:746-765), which is 0 on an h edge.
+template <typename T>
+__global__ void __launch_bounds__(kBlock) dga_init_kernel(InjItems q, const double* __restrict__ carr,
+                                                          T* __restrict__ U) {
+    const int32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < q.n) U[q.edge[i]] = q.kind[i] == 0 ? (T)0 : (T)inj_value(q, i, carr);
 }
 
 // ---- lossy dga: fractional unknowns (D:883-920, tf_dga_frac)
-// Sources of a lossy dga step. h edges as in dga_inject_kernel (curl_f and
-// the first Poynting partial); the other kinds write their value into the
+// Sources of a lossy dga step. h edges add their value to curl_f and give the
+// first Poynting partial, 0.5*U_old*fb; the other kinds write their value into the
 // edge's U_frac entry slot[e] (U_d of a class-4 edge, U_a of a class-1
 // edge; none for classes 2/3, whose entries the update rebuilds from their
 // old values, D:888-890). With init (the pass before the loop, D:726-790)
@@ -760,7 +799,7 @@ __global__ void __launch_bounds__(kBlock) frac_gather_kernel(int32_t n, const in
 // Source work taken by workgroups appended to dga_curl_kernel's grid (after
 // the face workgroups in logical order), one injection item per thread:
 //   mode 1 (dga): the second Poynting half of the step, 0.5 U_new v on the
-//     h-source edges;
+//     h-source edges, and (fbv) their values of the next step;
 //   mode 2 (gfdtd, fem): the step's sources as gf_inject_kernel forms them
 //     (fb, dir_new and the Poynting term from U_old).
 // One fp64 partial per appended workgroup into poy_part; mode 0: none.
@@ -780,6 +819,9 @@ struct CurlSources {
     T* dir_new = nullptr;
     int32_t delta = 0;                  // mode 2, fem: an h edge's forcing is Fb - Fb_old
     double* poy_part = nullptr;
+    double* fbv = nullptr;              // mode 1: h values of the next step (CtSources)
+    const int32_t* fb_pos = nullptr;
+    const double* carr_next = nullptr;
 };
 
 // gfdtd sources of one item (D:1478-1502): returns its Poynting term.
@@ -824,9 +866,17 @@ __global__ void __launch_bounds__(kBlock) dga_curl_kernel(int32_t n_faces, const
         double poy = 0;
         if (i < py.n_inj) {
             if (py.mode == 1) {
-                if (py.kind[i] == 0)
-                    poy = 0.5 * (double)U[py.edge[i]] *
-                          source_value(py.tb[i], py.te[i], py.term_src, py.term_w, py.carr_step);
+                if (py.kind[i] == 0) {
+                    const int32_t tb = py.tb[i], te = py.te[i];
+                    if (py.fbv) {
+                        const int32_t at = py.fb_pos[i];
+                        poy = 0.5 * (double)U[py.edge[i]] * py.fbv[at];
+                        py.fbv[at] = source_value(tb, te, py.term_src, py.term_w, py.carr_next);
+                    } else {
+                        poy = 0.5 * (double)U[py.edge[i]] *
+                              source_value(tb, te, py.term_src, py.term_w, py.carr_step);
+                    }
+                }
             } else {
                 poy = gf_source_item<T>(i, py.edge, py.kind, py.tb, py.te, py.term_src, py.term_w, py.carr_step,
                                         py.carr_prev, py.fb, py.dir_new, U, py.delta);

@@ -299,33 +299,41 @@ struct SellStream {
     }
 };
 
-// curl_f = Ct F over edges (dga, D:878-879).
+// curl_f = Ct F + Ctb Fb over edges (dga, D:878-879); src.blocks workgroups
+// behind the rows' take the rest of the source work (CtSources).
 template <typename T, int NB, bool W = false>
 __global__ void __launch_bounds__(kBlock) sell_ct_kernel(SellView<int8_t> m, const T* __restrict__ x,
-                                                         T* __restrict__ y) {
-    const int lane = lane_id();
+                                                         T* __restrict__ y, CtSources<T> src) {
+    const int lane = lane_id(), grid = (int)gridDim.x - src.blocks;
+    if ((int)blockIdx.x >= grid) {
+        __shared__ double red[kBlock / kWave];
+        ct_source_block<T>(src, (int)blockIdx.x - grid, red);
+        return;
+    }
+    auto store = [&](int sl, T v) {
+        const int32_t r = sl * kSlice + lane;
+        if (src.slice_slot) {
+            const int32_t q = scalar_load(src.slice_slot + __builtin_amdgcn_readfirstlane(sl));
+            if (q >= 0) v = (T)((double)v + src.fbv[(int64_t)q * kSlice + lane]);
+        }
+        if (r < m.nrows) y[r] = v;
+    };
+    const SliceRange srng = block_slices_of(m.nslices, m.band, (int)blockIdx.x, grid);
     if constexpr (W) {
         if (m.col16 && m.cwin) {
             struct Ent { uint16_t c; int8_t v; };
-            SellStream<NB, Ent, T, int8_t> ss(m, block_slices(m.nslices, m.band), lane);
+            SellStream<NB, Ent, T, int8_t> ss(m, srng, lane);
             auto load = [&](int64_t pos) { return Ent{stream_load<W>(m.col16 + pos), stream_load<W>(m.val + pos)}; };
             ss.start(load);
             ss.run(
                 load, [&](const Ent& e, const ColWin& cw) { return x[win_col(cw, e.c)]; },
                 [&](T& a, const Ent& e, T gv) { a += (T)e.v * gv; }, [&](int) { return 0; },
-                [&](int sl, T v, int) {
-                    const int32_t r = sl * kSlice + lane;
-                    if (r < m.nrows) y[r] = v;
-                });
+                [&](int sl, T v, int) { store(sl, v); });
             return;
         }
     }
-    TF_FOR_SLICES(m) {
-        const int s = sr_.s;
-        const double v = sell_dot<T, NB, W>(m, s, lane, [&](int32_t j) { return x[j]; });
-        const int32_t r = s * kSlice + lane;
-        if (r < m.nrows) y[r] = (T)v;
-    }
+    for (SliceRange sr_ = srng; sr_.s < sr_.end; sr_.s += sr_.step)
+        store(sr_.s, (T)sell_dot<T, NB, W>(m, sr_.s, lane, [&](int32_t j) { return x[j]; }));
 }
 
 // U[edge(r)] += dt * (H curl_f)[r] (dga, D:889); row_dt (batches) gives
@@ -445,17 +453,22 @@ __global__ void __launch_bounds__(kBlock) sell_frac_kernel(SellView<T> K, SellVi
 }
 
 // mode 0: F -= dt * N x (dga, D:917); mode 1: F = N x (gfdtd, D:1468);
-// row_dt as in sell_h_kernel; guard as in cg_guard_ok.
+// row_dt as in sell_h_kernel; guard as in cg_guard_ok. U and B are not written
+// here, so smp.blocks workgroups behind the rows' sample the probes.
 template <typename T, int NB, bool W = false>
 __global__ void __launch_bounds__(kBlock) sell_n_kernel(SellView<T> m, const T* __restrict__ x, T* __restrict__ Fv,
                                                         double dt, int mode, const double* __restrict__ row_dt,
-                                                        const CgState* guard) {
+                                                        const CgState* guard, SampleArgs<T> smp) {
     if (!cg_guard_ok(guard)) return;
-    const int lane = lane_id();
+    const int lane = lane_id(), grid = (int)gridDim.x - smp.blocks;
+    if ((int)blockIdx.x >= grid) {
+        sample_probes<T>(smp.ref, smp.slot, ((int)blockIdx.x - grid) * kBlock + (int)threadIdx.x, 0, 6, smp.U, smp.B);
+        return;
+    }
     // (the slice stream measured slower here: N's rows hold about 7 entries,
     // one batch, and its extra registers cost more occupancy than the
     // overlap gains)
-    TF_FOR_SLICES(m) {
+    for (SliceRange sr_ = block_slices_of(m.nslices, m.band, (int)blockIdx.x, grid); sr_.s < sr_.end; sr_.s += sr_.step) {
         const int s = sr_.s;
         const double v = sell_dot<T, NB, W>(m, s, lane, [&](int32_t j) { return x[j]; });
         const int32_t r = s * kSlice + lane;

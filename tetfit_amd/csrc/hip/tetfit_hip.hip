@@ -300,6 +300,7 @@ struct tf_ctx {
     std::vector<int32_t> h_dir_edge;
     std::vector<double> h_fixed_value;
     DevBuf inj_edge, inj_kind, inj_tb, inj_te;
+    DevBuf fb_slot, fb_pos, fbv;  // dga: h source values by Ct slice (CtSources)
     int32_t n_inj = 0;
     CgState* h_state = nullptr;  // pinned, two slots (as cg_state)
     CgState init_src[2] = {};     // host sources of the initial-state copies, per slot
@@ -403,7 +404,7 @@ size_t tf_ctx::device_bytes() const {
                            &spv, &slots, &samp_ref, &sg.carr, &sg.poy, &sg.slot,
                            &sp_edge, &sp_f4, &sp_sg, &sp_ca, &sp_cb, &sp_kind, &sp_tb, &sp_te, &c_col, &c_sg,
                            &h_edge, &curl_f, &curl_u, &free_edge, &edge_row, &dir_edge, &dir_new, &fb, &pre, &x, &r, &rs0, &rs1, &z,
-                           &p0, &p1, &q, &r0, &hx1, &hx2, &dx, &rr0part, &cg_part, &cg_state, &inj_edge, &inj_kind, &inj_tb, &inj_te,
+                           &p0, &p1, &q, &r0, &hx1, &hx2, &dx, &rr0part, &cg_part, &cg_state, &inj_edge, &inj_kind, &inj_tb, &inj_te, &fb_slot, &fb_pos, &fbv,
                            &term_src, &term_w, &carr, &probes, &samples, &eser, &epart, &poy, &row_dt_h, &row_dt_f,
                            &mu_a, &mu_b, &tf_a, &tf_b, &fslot, &row_dt_cg, &bt_inst, &bt_s0, &bt_s1, &bt_w0, &bt_w1, &uf[0], &uf[1], &ff[0], &ff[1], &u_out, &f_out, &u_two, &f_two,
                            &lu.row, &lu.ptr, &lu.col, &lu.val, &lu.mask, &lf.row, &lf.ptr, &lf.col, &lf.val, &lf.mask, &U_older, &fw, &fw2};
@@ -1587,6 +1588,21 @@ void build_tet_inject(tf_ctx* c, const std::vector<std::vector<std::pair<int32_t
     upload(c->inj_kind, kind);
     upload(c->inj_tb, tb);
     upload(c->inj_te, te);
+    if (c->method == TF_METHOD_DGA && !c->frac) {
+        // 64 value slots per Ct slice that holds an h edge (rows are edges)
+        std::vector<int32_t> slot(std::max(c->sCt.nslices, 1), -1), pos(std::max<size_t>(edge.size(), 1), 0);
+        int32_t used = 0;
+        for (size_t i = 0; i < edge.size(); ++i) {
+            if (kind[i] != 0) continue;
+            int32_t& q = slot[edge[i] / kSlice];
+            if (q < 0) q = used++;
+            pos[i] = q * kSlice + edge[i] % kSlice;
+        }
+        if (used) upload(c->fb_slot, slot);
+        else c->fb_slot.release();
+        upload(c->fb_pos, pos);
+        upload(c->fbv, std::vector<double>(std::max<size_t>((size_t)used * kSlice, 1), 0.0));
+    }
     if (tsrc.empty()) { tsrc.push_back(0); tw.push_back(0); }
     upload(c->term_src, tsrc);
     upload(c->term_w, tw);
@@ -1722,13 +1738,6 @@ void drop_graph(tf_ctx* c) {
     c->sg.graph = nullptr;
 }
 
-// Graph replay is used when no launch of the chunk depends on the host: no
-// probe sampling and no per-kernel event timing.
-bool graph_steps(const tf_ctx* c) {
-    if (!c->use_graphs || c->profiling) return false;
-    return c->batch ? c->batch->every <= 0 : !c->out_enabled;
-}
-
 // Captures kGraphSteps calls of step(local step, carrier row, Poynting slot)
 // into the context's graph (once), then runs steps [first_k, first_k + m) of
 // the current tf_run in chunks of kGraphSteps by replay; per_step = Poynting
@@ -1775,15 +1784,17 @@ int64_t run_graph_chunks(tf_ctx* c, int64_t first_k, int64_t m, int per_step, bo
     return chunks * kGraphSteps;
 }
 
-// Output samples of steps [first, first + n) that the steps' own kernels
-// take: a slot per step in c->slots (row k + 1: step first + k; row 0, the step
-// before the run, has none: its sample was taken then) and the sample
-// reference. Returns whether the run samples probes.
-bool plan_samples(tf_ctx* c, int64_t first, int64_t n) {
+// Output samples that the steps' own kernels take, for n steps of a run: step
+// k samples the state at index(k) = (step number, time). Their slots go to
+// c->slots (row k + 1; row 0, the step before the run, has none: its sample was
+// taken then) and what the kernels write to into c->samp_ref. Returns whether
+// the run samples probes.
+template <class Index>
+bool plan_samples(tf_ctx* c, int64_t n, Index index) {
     std::vector<int64_t> slot((size_t)n + 1, -1);
     for (int64_t k = 0; k < n; ++k) {
-        const double t = (double)(first + k) * c->dt;
-        if (want_sample(c, first + k, t)) slot[k + 1] = sample_reserve(c, t);
+        const std::pair<int64_t, double> it = index(k);
+        if (want_sample(c, it.first, it.second)) slot[k + 1] = sample_reserve(c, it.second);
     }
     if (c->n_probes == 0 || !(c->batch ? c->batch->every > 0 : c->out_enabled)) return false;
     const SampleRef ref{c->probes.as<ProbeDev>(), c->samples.as<double>(), c->n_probes};
@@ -1793,6 +1804,25 @@ bool plan_samples(tf_ctx* c, int64_t first, int64_t n) {
     TF_HIP(hipMemcpyAsync(c->samp_ref.p, &ref, sizeof(ref), hipMemcpyHostToDevice, c->stream));
     TF_HIP(hipStreamSynchronize(c->stream));
     return true;
+}
+// The sample of row `slot` of the table, by workgroups of another kernel.
+template <class T>
+SampleArgs<T> sample_args(tf_ctx* c, bool inside, const int64_t* slot) {
+    if (!inside) return SampleArgs<T>{};
+    return SampleArgs<T>{blocks_for((int64_t)c->n_probes * 6), c->samp_ref.as<SampleRef>(), slot, c->U.as<T>(),
+                         c->B.as<T>()};
+}
+// Whether the steps of an explicit method replay in graphs: per-kernel event
+// timing and energy samples (reductions between steps) need host launches, and
+// so do samples that the steps' kernels do not take themselves.
+bool graph_steps(const tf_ctx* c, bool inside) {
+    if (!c->use_graphs || c->profiling) return false;
+    return inside || !(c->batch ? c->batch->every > 0 : c->out_enabled);
+}
+// A captured step samples with so many workgroups: another count drops the graph.
+void graph_for_samples(tf_ctx* c, int probe_blocks) {
+    if (c->sg.exec && c->sg_probe_blocks != probe_blocks) drop_graph(c);
+    c->sg_probe_blocks = probe_blocks;
 }
 
 FitSpecial fit_special_view(const tf_ctx* c) {
@@ -1840,7 +1870,7 @@ void run_fit(tf_ctx* c, int64_t first, int64_t n, tf_stats* st) {
     }
     const FitSpecial sp = fit_special_view(c);
     if (!c->fit_grid) {
-        const int64_t g = graph_steps(c) ? run_graph_chunks(c, 0, n, sp_blocks, false,
+        const int64_t g = graph_steps(c, false) ? run_graph_chunks(c, 0, n, sp_blocks, false,
                                                             [&](int, const double* cs, double* poy, const int64_t*) {
             fit_indexed_step<T>(c, sp, sp_blocks, cs, poy);
         }) : 0;
@@ -1853,7 +1883,9 @@ void run_fit(tf_ctx* c, int64_t first, int64_t n, tf_stats* st) {
         }
     } else {
         // energy samples reduce the fields between steps, from the host
-        const bool inside = !c->energy_out && plan_samples(c, first, n);
+        const bool inside = !c->energy_out && plan_samples(c, n, [&](int64_t k) {
+            return std::make_pair(first + k, (double)(first + k) * c->dt);
+        });
         FitStep<T> e{};
         e.g = c->grid;
         e.sp_blocks = sp_blocks;
@@ -1904,10 +1936,9 @@ void run_fit(tf_ctx* c, int64_t first, int64_t n, tf_stats* st) {
         if (sp_blocks)
             fit_src_kernel<<<sp_blocks, kBlock, 0, c->stream>>>(sp, c->carr.as<double>() + ns, c->spv.as<double>());
         int64_t k0 = 0;
-        if (c->use_graphs && !c->profiling && !(c->out_enabled && c->energy_out)) {
-            // a captured step samples with so many workgroups
-            if (c->sg.exec && c->sg_probe_blocks != e.probe_blocks) drop_graph(c);
-            c->sg_probe_blocks = e.probe_blocks;
+        // (without probes a sample records nothing on the device)
+        if (graph_steps(c, !c->energy_out)) {
+            graph_for_samples(c, e.probe_blocks);
             k0 = run_graph_chunks(c, 0, n, sp_blocks, inside,
                                   [&](int k, const double* cs, double* poy, const int64_t* slot) {
                                       step(cs, poy, slot, k == kGraphSteps - 1);
@@ -2002,9 +2033,15 @@ void run_dga_frac(tf_ctx* c, int64_t first, int64_t n, tf_stats* st) {
     c->initial_done = true;
     const int gb_ct = tuned_blocks(c, TK_CT, c->sCt, kSpmvCap);
     const int gb_u = sell_blocks(c->fKu, kSpmvCap) + c->lu.n, gb_f = sell_blocks(c->fKf, kSpmvCap) + c->lf.n;
-    auto step = [&](const double* cs, double* poy) {
+    // samples ride in sell_n where F steps in place
+    const bool mine = c->f_plain && !c->energy_out;
+    const bool inside = mine && plan_samples(c, n, [&](int64_t k) {
+        return std::make_pair(first + k, (double)(first + k) * c->dt);
+    });
+    const SampleArgs<T> smp = sample_args<T>(c, inside, nullptr);
+    auto step = [&](const double* cs, double* poy, const int64_t* slot) {
         TF_LAUNCH_TIMED(c, "sell_ct_kernel", c->tune[TK_CT].unroll, sell_ct_kernel, T, gb_ct,
-                        tuned_view(c, TK_CT, c->sCt.signs()), c->Fv.as<T>(), c->curl_f.as<T>());
+                        tuned_view(c, TK_CT, c->sCt.signs()), c->Fv.as<T>(), c->curl_f.as<T>(), CtSources<T>{});
         inject(cs, poy, 0);
         const int nx = c->fcur ^ 1;
         if (c->nU > 0)
@@ -2017,8 +2054,10 @@ void run_dga_frac(tf_ctx* c, int64_t first, int64_t n, tf_stats* st) {
                      c->c_col.as<int32_t>(), c->c_fixed_signs ? nullptr : c->c_sg.as<int8_t>(), (const T*)c->U.as<T>(),
                      c->curl_u.as<T>(), c->B.as<T>(), c->dt, (const double*)nullptr, (const CgState*)nullptr, py);
         if (c->f_plain) {
-            TF_LAUNCH_TIMED(c, "sell_n_kernel", 8, sell_n_kernel, T, gb_f, c->fKf.vals<T>(), c->curl_u.as<T>(),
-                            c->Fv.as<T>(), c->dt, 0, nullptr, nullptr);
+            SampleArgs<T> sm = smp;
+            sm.slot = slot;
+            TF_LAUNCH_TIMED(c, "sell_n_kernel", 8, sell_n_kernel, T, gb_f + sm.blocks, c->fKf.vals<T>(),
+                            c->curl_u.as<T>(), c->Fv.as<T>(), c->dt, 0, nullptr, nullptr, sm);
         } else if (c->nF > 0) {
             TF_LAUNCH_TIMED(c, "sell_frac_kernel", 8, sell_frac_kernel, T, gb_f, c->fKf.vals<T>(), c->fRf.vals<T>(),
                             (const T*)c->curl_u.as<T>(), (const T*)c->ff[c->fcur].as<T>(), c->ff[nx].as<T>(), -c->dt,
@@ -2033,15 +2072,16 @@ void run_dga_frac(tf_ctx* c, int64_t first, int64_t n, tf_stats* st) {
     auto host_step = [&](int64_t k) {
         const int64_t i = first + k;
         const double t = (double)i * c->dt;
-        step(c->carr.as<double>() + (k + 1) * ns, c->poy.as<double>() + 2 * k * inj_blocks);
-        if (want_sample(c, i, t)) sample<T>(c, t);
+        step(c->carr.as<double>() + (k + 1) * ns, c->poy.as<double>() + 2 * k * inj_blocks, c->slots.as<int64_t>() + k + 1);
+        if (!mine && want_sample(c, i, t)) sample<T>(c, t);
         if (c->profiling && (k & 63) == 63) ev_flush(c);
     };
-    if (graph_steps(c)) {
+    if (graph_steps(c, mine)) {
+        graph_for_samples(c, smp.blocks);
         if (c->sg.exec && c->sg_fcur != c->fcur && n > 0) host_step(h++);
         if (!c->sg.exec) c->sg_fcur = c->fcur;
-        h += run_graph_chunks(c, h, n - h, 2 * inj_blocks, false,
-                              [&](int, const double* cs, double* poy, const int64_t*) { step(cs, poy); });
+        h += run_graph_chunks(c, h, n - h, 2 * inj_blocks, inside,
+                              [&](int, const double* cs, double* poy, const int64_t* slot) { step(cs, poy, slot + 1); });
     }
     for (; h < n; ++h) host_step(h);
     TF_HIP(hipGetLastError());
@@ -2070,9 +2110,12 @@ void run_dga(tf_ctx* c, int64_t first, int64_t n, tf_stats* st) {
     const double* fdt = c->batch ? c->row_dt_f.as<double>() : nullptr;
     const int gb_ct = tuned_blocks(c, TK_CT, c->sCt, kSpmvCap), gb_h = tuned_blocks(c, TK_H, c->H, kSpmvCap);
     const int gb_n = tuned_blocks(c, TK_N, c->N, kSpmvCap);
-    // Poynting partials of a step: the injection kernel's workgroups (first
-    // half, 0.5 U_old v), then the workgroups appended to dga_curl (second
-    // half, 0.5 U_new v)
+    const InjItems items{c->n_inj,           c->inj_edge.as<int32_t>(), c->inj_kind.as<int8_t>(),
+                         c->inj_tb.as<int32_t>(), c->inj_te.as<int32_t>(),   c->term_src.as<int32_t>(),
+                         c->term_w.as<double>()};
+    // Poynting partials of a step: the workgroups appended to sell_ct (first
+    // half, 0.5 U_old v), then those appended to dga_curl (second half, 0.5
+    // U_new v)
     const int per_step = c->n_inj ? 2 * inj_blocks : 0;
     if (per_step && c->poy_cap < (int64_t)per_step * n) {
         c->poy.alloc((size_t)per_step * n * sizeof(double));
@@ -2080,47 +2123,61 @@ void run_dga(tf_ctx* c, int64_t first, int64_t n, tf_stats* st) {
     }
     if (!c->initial_done && first == 1) {
         // initial export at t = 0 (D:805-806), after the t = 0 e-source values
-        if (c->n_inj) {
-            const double* cs0 = c->carr.as<double>();  // row 0 = step first-1 = 0
-            dga_inject_kernel<T><<<inj_blocks, kBlock, 0, c->stream>>>(
-                c->n_inj, c->inj_edge.as<int32_t>(), c->inj_kind.as<int8_t>(), c->inj_tb.as<int32_t>(),
-                c->inj_te.as<int32_t>(), c->term_src.as<int32_t>(), c->term_w.as<double>(), cs0, c->curl_f.as<T>(),
-                c->U.as<T>(), c->poy.as<double>(), 1);
-        }
+        if (c->n_inj)  // row 0 = step first-1 = 0
+            dga_init_kernel<T><<<inj_blocks, kBlock, 0, c->stream>>>(items, c->carr.as<double>(), c->U.as<T>());
         if (want_sample(c, 0, 0.0)) sample<T>(c, 0.0);
     }
     c->initial_done = true;
-    // one step (D:810-939): curl_f = Ct F, the sources (h into curl_f, e into
-    // U, the first Poynting half), U += dt H curl_f, curl_u = C U with the B
-    // update and, in dga_curl's appended workgroups, the second Poynting half,
-    // F -= dt N curl_u
-    auto step = [&](const double* cs, double* poy) {
-        TF_LAUNCH_TIMED(c, "sell_ct_kernel", c->tune[TK_CT].unroll, sell_ct_kernel, T, gb_ct,
-                        tuned_view(c, TK_CT, c->sCt.signs()), c->Fv.as<T>(), c->curl_f.as<T>());
+    const bool inside = !c->energy_out && plan_samples(c, n, [&](int64_t k) {
+        return std::make_pair(first + k, (double)(first + k) * c->dt);
+    });
+    const SampleArgs<T> smp = sample_args<T>(c, inside, nullptr);
+    if (c->n_inj)
+        dga_src_kernel<<<inj_blocks, kBlock, 0, c->stream>>>(items, c->fb_pos.as<int32_t>(),
+                                                             c->carr.as<double>() + ns, c->fbv.as<double>());
+    // one step (D:810-939): curl_f = Ct F with the sources (h into curl_f, e
+    // into U, the first Poynting half), U += dt H curl_f, curl_u = C U with the
+    // B update and, in dga_curl's appended workgroups, the second Poynting half
+    // and the next step's h values, F -= dt N curl_u with the step's sample
+    auto step = [&](const double* cs, double* poy, const int64_t* slot) {
+        CtSources<T> src;
         if (c->n_inj)
-            launch_timed(c, "dga_inject_kernel", dga_inject_kernel<T>, inj_blocks, c->n_inj, c->inj_edge.as<int32_t>(),
-                         c->inj_kind.as<int8_t>(), c->inj_tb.as<int32_t>(), c->inj_te.as<int32_t>(),
-                         c->term_src.as<int32_t>(), c->term_w.as<double>(), cs, c->curl_f.as<T>(), c->U.as<T>(), poy,
-                         0);
+            src = CtSources<T>{inj_blocks,           items,
+                               c->fb_slot.as<int32_t>(), c->fb_pos.as<int32_t>(), c->fbv.as<double>(), cs,
+                               c->U.as<T>(),         poy};
+        TF_LAUNCH_TIMED(c, "sell_ct_kernel", c->tune[TK_CT].unroll, sell_ct_kernel, T, gb_ct + src.blocks,
+                        tuned_view(c, TK_CT, c->sCt.signs()), c->Fv.as<T>(), c->curl_f.as<T>(), src);
         TF_LAUNCH_TIMED(c, "sell_h_kernel", c->tune[TK_H].unroll, sell_h_kernel, T, gb_h,
                         tuned_view(c, TK_H, c->H.vals<T>()), c->h_edge.as<int32_t>(), c->curl_f.as<T>(), c->U.as<T>(),
                         c->dt, hdt);
-        const CurlSources<T> py = c->n_inj ? curl_sources<T>(c, 1, cs, nullptr, poy + inj_blocks) : CurlSources<T>{};
+        CurlSources<T> py;
+        if (c->n_inj) {
+            py = curl_sources<T>(c, 1, cs, nullptr, poy + inj_blocks);
+            py.fbv = c->fbv.as<double>();
+            py.fb_pos = c->fb_pos.as<int32_t>();
+            py.carr_next = cs + ns;
+        }
         launch_timed(c, "dga_curl_kernel", dga_curl_kernel<T>, blocks_for(c->F) + (c->n_inj ? inj_blocks : 0), c->F,
                      c->c_col.as<int32_t>(), c->c_fixed_signs ? nullptr : c->c_sg.as<int8_t>(), c->U.as<T>(),
                      c->curl_u.as<T>(), c->B.as<T>(), c->dt, fdt, (const CgState*)nullptr, py);
-        TF_LAUNCH_TIMED(c, "sell_n_kernel", c->tune[TK_N].unroll, sell_n_kernel, T, gb_n,
-                        tuned_view(c, TK_N, c->N.vals<T>()), c->curl_u.as<T>(), c->Fv.as<T>(), c->dt, 0, fdt, nullptr);
+        SampleArgs<T> sm = smp;
+        sm.slot = slot;
+        TF_LAUNCH_TIMED(c, "sell_n_kernel", c->tune[TK_N].unroll, sell_n_kernel, T, gb_n + sm.blocks,
+                        tuned_view(c, TK_N, c->N.vals<T>()), c->curl_u.as<T>(), c->Fv.as<T>(), c->dt, 0, fdt, nullptr,
+                        sm);
     };
-    const int64_t g = graph_steps(c) ? run_graph_chunks(c, 0, n, per_step, false,
-                                                        [&](int, const double* cs, double* poy, const int64_t*) {
-        step(cs, poy);
-    }) : 0;
+    int64_t g = 0;
+    if (graph_steps(c, !c->energy_out)) {
+        graph_for_samples(c, smp.blocks);
+        g = run_graph_chunks(c, 0, n, per_step, inside,
+                             [&](int, const double* cs, double* poy, const int64_t* slot) { step(cs, poy, slot + 1); });
+    }
     for (int64_t k = g; k < n; ++k) {
         const int64_t i = first + k;
         const double t = (double)i * c->dt;
-        step(c->carr.as<double>() + (k + 1) * ns, c->poy.as<double>() + (size_t)per_step * k);
-        if (want_sample(c, i, t)) sample<T>(c, t);
+        step(c->carr.as<double>() + (k + 1) * ns, c->poy.as<double>() + (size_t)per_step * k,
+             c->slots.as<int64_t>() + k + 1);
+        if (c->energy_out && want_sample(c, i, t)) sample<T>(c, t);
         if (c->profiling && (k & 63) == 63) ev_flush(c);
     }
     TF_HIP(hipGetLastError());
@@ -2833,6 +2890,11 @@ void run_gfdtd(tf_ctx* c, int64_t first, int64_t n, const tf_cg_opts* cg, tf_sta
     // zero there now.
     auto dir_terms = [&](int64_t k) { return !(c->dir_zero_static && (k > 0 || c->ud_zero)); };
     // Kernels of step k up to the start of its solve (guard: the previous solve's state).
+    // step k samples U_old and B at t - dt (row k + 1 of the slot table)
+    const bool mine = !c->energy_out;
+    const bool inside = mine && plan_samples(c, n, [&](int64_t k) {
+        return std::make_pair(first + k - 1, (double)(first + k) * c->dt - c->dt);
+    });
     auto pre = [&](int64_t k, GfPre& g, bool fresh, const CgState* guard) {
         const int64_t i = first + k;
         const double t = (double)i * c->dt;
@@ -2848,10 +2910,14 @@ void run_gfdtd(tf_ctx* c, int64_t first, int64_t n, const tf_cg_opts* cg, tf_sta
                      c->c_col.as<int32_t>(), c->c_fixed_signs ? nullptr : c->c_sg.as<int8_t>(), c->U.as<T>(),
                      c->curl_u.as<T>(), c->B.as<T>(), c->dt, (const double*)nullptr, guard, inj);
         // gfdtd: F = N B (D:1468); fem: N C U_old for the curl-curl term (D:1729)
-        TF_LAUNCH_TIMED(c, "sell_n_kernel", c->tune[TK_N].unroll, sell_n_kernel, T, gb_n,
-                        tuned_view(c, TK_N, c->N.vals<T>()), c->fem ? c->curl_u.as<T>() : c->B.as<T>(), c->Fv.as<T>(), c->dt, 1, nullptr, guard);
-        if (fresh) g.sample_slot = allow_print(c, t - c->dt) ? sample_reserve(c, t - c->dt) : -1;
-        sample_launch<T>(c, g.sample_slot, guard);
+        const SampleArgs<T> smp = sample_args<T>(c, inside, c->slots.as<int64_t>() + k + 1);
+        TF_LAUNCH_TIMED(c, "sell_n_kernel", c->tune[TK_N].unroll, sell_n_kernel, T, gb_n + smp.blocks,
+                        tuned_view(c, TK_N, c->N.vals<T>()), c->fem ? c->curl_u.as<T>() : c->B.as<T>(), c->Fv.as<T>(),
+                        c->dt, 1, nullptr, guard, smp);
+        if (!mine) {
+            if (fresh) g.sample_slot = allow_print(c, t - c->dt) ? sample_reserve(c, t - c->dt) : -1;
+            sample_launch<T>(c, g.sample_slot, guard);
+        }
         if (lossy) {
             // U_old.SigMat U_old of the losses (D:1519)
             TF_LAUNCH_TIMED(c, "quad_form_kernel", 8, quad_form_kernel, T, loss_blocks,
@@ -3310,7 +3376,7 @@ void autotune(tf_ctx* c) {
     if (c->method == TF_METHOD_DGA) {
         c->tune[TK_CT] = tune_one(c, TK_CT, c->sCt, kSpmvCap, [&](const KTune& t) {
             TF_LAUNCH_NB(c->wide, t.unroll, sell_ct_kernel, T, t.blocks, s, with_band(c->sCt.signs(), t),
-                         c->Fv.as<T>(), c->curl_f.as<T>());
+                         c->Fv.as<T>(), c->curl_f.as<T>(), CtSources<T>{});
         });
         if (c->frac) return;  // lossy media: only sell_ct of the tuned kernels runs
         c->tune[TK_H] = tune_one(c, TK_H, c->H, kSpmvCap, [&](const KTune& t) {
@@ -3319,12 +3385,12 @@ void autotune(tf_ctx* c) {
         });
         c->tune[TK_N] = tune_one(c, TK_N, c->N, kSpmvCap, [&](const KTune& t) {
             TF_LAUNCH_NB(c->wide, t.unroll, sell_n_kernel, T, t.blocks, s, with_band(c->N.vals<T>(), t),
-                         c->curl_u.as<T>(), c->Fv.as<T>(), 0.0, 0, nullptr, nullptr);
+                         c->curl_u.as<T>(), c->Fv.as<T>(), 0.0, 0, nullptr, nullptr, SampleArgs<T>{});
         });
     } else if (c->method == TF_METHOD_GFDTD || c->method == TF_METHOD_FEM) {
         c->tune[TK_N] = tune_one(c, TK_N, c->N, kSpmvCap, [&](const KTune& t) {
             TF_LAUNCH_NB(c->wide, t.unroll, sell_n_kernel, T, t.blocks, s, with_band(c->N.vals<T>(), t), c->B.as<T>(),
-                         c->Fv.as<T>(), c->dt, 1, nullptr, nullptr);
+                         c->Fv.as<T>(), c->dt, 1, nullptr, nullptr, SampleArgs<T>{});
         });
         // Tuning launches run pass 1 (the full work of a pass) on a scratch
         // CG state that never stops (tol 0, no iteration cap, rr0 = 1: the
@@ -3582,7 +3648,7 @@ void run_gfdtd_batch(tf_ctx* c, int64_t first, int64_t n, const tf_cg_opts* cg, 
                      c->curl_u.as<T>(), c->B.as<T>(), c->dt, fdt, (const CgState*)nullptr, inj);
         TF_LAUNCH_TIMED(c, "sell_n_kernel", c->tune[TK_N].unroll, sell_n_kernel, T, gb_n,
                         tuned_view(c, TK_N, c->N.vals<T>()), c->B.as<T>(), c->Fv.as<T>(), c->dt, 1, nullptr,
-                        nullptr);
+                        nullptr, SampleArgs<T>{});
         // the state before the solve, at t - dt (as run_gfdtd samples it)
         if (want_sample(c, i - 1, t - c->dt)) sample<T>(c, t - c->dt);
         TF_HIP(hipMemcpyAsync(states, inits.data(), inits.size() * sizeof(CgState), hipMemcpyHostToDevice,
