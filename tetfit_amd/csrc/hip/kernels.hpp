@@ -477,10 +477,13 @@ __global__ void __launch_bounds__(kBlock) fit_src_kernel(FitSpecial sp, const do
 // goes to LDS meanwhile, and source values are prepared a step ahead. Larger
 // grids are bound by bytes: an fp64 item moves 26 (E) and 26 (H) with palettes,
 // against 42 and 50 with plain coefficients and B stored every step.
+// Plain coefficients are loaded non-temporally: read once a step, they would
+// push the fields out of the 256 MB Infinity Cache.
 // One step (both kernels, in a graph): 64^3 fp64 12.1 us, fp32 9.8 us; 161^3
-// random media fp64 163 us (E 94 us, 5.7 TB/s; H 67 us, 4.9 TB/s). With codes
-// read before the neighbours, five-load source chains and one item per thread:
-// 15.4, 12.0 and 185 us.
+// random media fp64 141 us (E 87 us, H 55 us; 163 us with ordinary coefficient
+// loads, which cost H its cached fields). With codes read before the
+// neighbours, five-load source chains and one item per thread: 15.4, 12.0 and
+// 185 us.
 template <typename T>
 struct FitStep {
     FitGrid g;
@@ -590,7 +593,7 @@ __global__ void __launch_bounds__(kBlock) fit_e_grid_kernel(FitStep<T> a, const 
         v1[m] = Fv[in ? f1 : 0];
         v2[m] = Fv[in ? f2 : 0];
         v3[m] = Fv[in ? f3 : 0];
-        if constexpr (!P) q[m] = FitPal<T>{a.c0[s], a.c1[s]};
+        if constexpr (!P) q[m] = FitPal<T>{__builtin_nontemporal_load(a.c0 + s), __builtin_nontemporal_load(a.c1 + s)};
     }
     if constexpr (P) __syncthreads();
 #pragma unroll
@@ -669,7 +672,7 @@ __global__ void __launch_bounds__(kBlock) fit_h_grid_kernel(FitStep<T> a, int st
         v1[m] = U[e1];
         v2[m] = U[e2];
         v3[m] = U[e3];
-        if constexpr (!P) q[m] = FitPal<T>{a.c0[s], a.c1[s]};
+        if constexpr (!P) q[m] = FitPal<T>{__builtin_nontemporal_load(a.c0 + s), __builtin_nontemporal_load(a.c1 + s)};
     }
     if constexpr (P) __syncthreads();
 #pragma unroll
