@@ -1003,6 +1003,24 @@ __global__ void __launch_bounds__(kBlock) gf_inject_kernel(
     if (threadIdx.x == 0) poy_part[blockIdx.x] = s;
 }
 
+// ------------------------------------------------------------------ state
+// A field in the caller's numbering and in fp64: out[i] = x[pos[i]] (pos null:
+// the same order), and the other way round. The permutation and the conversion
+// run here, bound by the gather (161^3 fp64, 300 MB: 1 ms), so that the host
+// only receives the bytes.
+template <typename T>
+__global__ void __launch_bounds__(kBlock) state_gather_kernel(int64_t n, const int32_t* __restrict__ pos,
+                                                              const T* __restrict__ x, double* __restrict__ out) {
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) out[i] = (double)x[pos ? pos[i] : i];
+}
+template <typename T>
+__global__ void __launch_bounds__(kBlock) state_scatter_kernel(int64_t n, const int32_t* __restrict__ pos,
+                                                               const double* __restrict__ in, T* __restrict__ x) {
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) x[pos ? pos[i] : i] = (T)in[i];
+}
+
 // ------------------------------------------------------------------ energy
 // part[block] = sum over this block's entries of w_i x_i^2 (fp64).
 template <typename T>

@@ -232,6 +232,7 @@ struct tf_ctx {
     // each step exceed the 256 MB Infinity Cache
     bool wide = false;
     FitGrid grid{};
+    DevBuf d_esid, d_fsid, stage;         // the same on the device; staging of state reads and writes
     std::vector<int32_t> h_esid, h_fsid;  // reference edge / face -> device position (FIT grid order, tet relabel)
     // grid order (fit_e_grid_kernel, fit_h_grid_kernel): id per entity (0: not
     // in the main pass) and a coefficient palette, or, where too many distinct
@@ -401,7 +402,7 @@ tf_ctx::~tf_ctx() {
 size_t tf_ctx::device_bytes() const {
     size_t s = 0;
     const DevBuf* all[] = {&U, &Fv, &B, &fit_ep, &fit_nu, &fe_sg, &fe_ca, &fe_cb, &fe_f4, &fh_sg, &fh_cm, &fh_cn, &fh_e4, &fe_id, &fe_pal, &fh_id, &fh_pal, &fh_at, &fh_val,
-                           &spv, &slots, &samp_ref, &sg.carr, &sg.poy, &sg.slot,
+                           &spv, &d_esid, &d_fsid, &stage, &slots, &samp_ref, &sg.carr, &sg.poy, &sg.slot,
                            &sp_edge, &sp_f4, &sp_sg, &sp_ca, &sp_cb, &sp_kind, &sp_tb, &sp_te, &c_col, &c_sg,
                            &h_edge, &curl_f, &curl_u, &free_edge, &edge_row, &dir_edge, &dir_new, &fb, &pre, &x, &r, &rs0, &rs1, &z,
                            &p0, &p1, &q, &r0, &hx1, &hx2, &dx, &rr0part, &cg_part, &cg_state, &inj_edge, &inj_kind, &inj_tb, &inj_te, &fb_slot, &fb_pos, &fbv,
@@ -467,7 +468,7 @@ void upload_sell(Sell& d, const tf_csr& c, bool values, bool windows = true) {
     std::vector<int32_t> col(d.entries, 0);
     std::vector<T> val(values ? d.entries : 0, (T)0);
     std::vector<int8_t> sg(values ? 0 : d.entries, 0);
-    par_chunks(d.nslices, 1024, [&](int64_t lo, int64_t hi) {
+    par_chunks(d.nslices, 4096, [&](int64_t lo, int64_t hi) {
       for (int32_t s = (int32_t)lo; s < (int32_t)hi; ++s) {
         const int64_t w = (sptr[s + 1] - sptr[s]) / kSlice;
         // rows without entries (and lanes past the last row) pad with a column
@@ -511,7 +512,7 @@ void upload_sell(Sell& d, const tf_csr& c, bool values, bool windows = true) {
     std::vector<int32_t> cb(std::max(d.nslices, 1), 0);
     bool fits = !force32 && !env_on("TETFIT_SELL_WIN");
     std::atomic<bool> ok{fits};
-    par_chunks(d.nslices, 1024, [&](int64_t s0, int64_t s1) {
+    par_chunks(d.nslices, 4096, [&](int64_t s0, int64_t s1) {
         for (int64_t s = s0; s < s1 && ok; ++s) {
             int32_t lo = INT32_MAX, hi = 0;
             for (int64_t o = sptr[s]; o < sptr[s + 1]; ++o) { lo = std::min(lo, col[o]); hi = std::max(hi, col[o]); }
@@ -532,7 +533,7 @@ void upload_sell(Sell& d, const tf_csr& c, bool values, bool windows = true) {
         cb.assign(4 * std::max(d.nslices, 1), 0);
         std::vector<uint8_t> nwin(std::max(d.nslices, 1), 0);
         ok = true;
-        par_chunks(d.nslices, 1024, [&](int64_t lo, int64_t hi) {
+        par_chunks(d.nslices, 4096, [&](int64_t lo, int64_t hi) {
             std::vector<int32_t> cs;
             for (int64_t s = lo; s < hi && ok; ++s) {
                 cs.assign(col.begin() + sptr[s], col.begin() + sptr[s + 1]);
@@ -551,7 +552,7 @@ void upload_sell(Sell& d, const tf_csr& c, bool values, bool windows = true) {
         if (fits) {
             c16.assign(std::max<int64_t>(d.entries, 1), 0);
             ok = true;
-            par_chunks(d.nslices, 1024, [&](int64_t lo, int64_t hi) {
+            par_chunks(d.nslices, 4096, [&](int64_t lo, int64_t hi) {
                 for (int64_t s = lo; s < hi; ++s)
                     for (int64_t o = sptr[s]; o < sptr[s + 1]; ++o) {
                         // the last opened window whose base is <= the column; the
@@ -1600,8 +1601,10 @@ void build_tet_inject(tf_ctx* c, const std::vector<std::vector<std::pair<int32_t
         }
         if (used) upload(c->fb_slot, slot);
         else c->fb_slot.release();
-        upload(c->fb_pos, pos);
-        upload(c->fbv, std::vector<double>(std::max<size_t>((size_t)used * kSlice, 1), 0.0));
+        if (!edge.empty()) {
+            upload(c->fb_pos, pos);
+            upload(c->fbv, std::vector<double>(std::max<size_t>((size_t)used * kSlice, 1), 0.0));
+        }
     }
     if (tsrc.empty()) { tsrc.push_back(0); tw.push_back(0); }
     upload(c->term_src, tsrc);
@@ -3114,6 +3117,56 @@ tf_status guarded(F f) {
     }
 }
 
+// Entries [off, off + n) of a field, in the caller's numbering (pos: device
+// position of each, or null) and fp64, to host memory at dst (null: skipped).
+// Chunks of at most kStage values are permuted and converted on the device (8
+// MB a chunk: 161^3 fp64, 101 MB a field, 10 ms into fresh memory, 33 ms when
+// the host permuted; half or an eighth of it 0-10% slower).
+constexpr int64_t kStage = 1 << 20;
+double* stage_buffer(tf_ctx* c, int64_t n) {
+    const size_t need = (size_t)std::min(n, kStage) * sizeof(double);
+    if (c->stage.bytes < need) c->stage.alloc(need);
+    return c->stage.as<double>();
+}
+void read_field(tf_ctx* c, const DevBuf& b, const int32_t* pos, int64_t off, int64_t n, double* dst) {
+    if (!dst || n <= 0) return;
+    const bool f64 = c->prec == TF_PREC_FP64;
+    if (f64 && !pos) {
+        TF_HIP(hipStreamSynchronize(c->stream));
+        TF_HIP(hipMemcpy(dst, b.as<double>() + off, n * sizeof(double), hipMemcpyDeviceToHost));
+        return;
+    }
+    double* st = stage_buffer(c, n);
+    for (int64_t k = 0; k < n; k += kStage) {
+        const int64_t m = std::min(kStage, n - k);
+        const int32_t* p = pos ? pos + off + k : nullptr;
+        const int64_t o = pos ? 0 : off + k;
+        if (f64) state_gather_kernel<double><<<blocks_for(m), kBlock, 0, c->stream>>>(m, p, b.as<double>() + o, st);
+        else state_gather_kernel<float><<<blocks_for(m), kBlock, 0, c->stream>>>(m, p, b.as<float>() + o, st);
+        TF_HIP(hipGetLastError());
+        // (a synchronous copy: on the context's own stream the runtime set up
+        // its staging once more per context, 10 ms on the first read)
+        TF_HIP(hipStreamSynchronize(c->stream));
+        TF_HIP(hipMemcpy(dst + k, st, m * sizeof(double), hipMemcpyDeviceToHost));
+    }
+}
+// The same to the device, all n entries.
+void write_field(tf_ctx* c, DevBuf& b, const int32_t* pos, int64_t n, const double* src) {
+    if (!src || n <= 0) return;
+    const bool f64 = c->prec == TF_PREC_FP64;
+    double* st = stage_buffer(c, n);
+    for (int64_t k = 0; k < n; k += kStage) {
+        const int64_t m = std::min(kStage, n - k);
+        const int32_t* p = pos ? pos + k : nullptr;
+        const int64_t o = pos ? 0 : k;
+        TF_HIP(hipMemcpy(st, src + k, m * sizeof(double), hipMemcpyHostToDevice));
+        if (f64) state_scatter_kernel<double><<<blocks_for(m), kBlock, 0, c->stream>>>(m, p, st, b.as<double>() + o);
+        else state_scatter_kernel<float><<<blocks_for(m), kBlock, 0, c->stream>>>(m, p, st, b.as<float>() + o);
+        TF_HIP(hipGetLastError());
+        TF_HIP(hipStreamSynchronize(c->stream));
+    }
+}
+
 std::unique_ptr<tf_ctx> make_ctx(const tf_problem* p, int32_t prec,
                                  const std::vector<int32_t>* batch_rows = nullptr) {
     if (p->method < 0 || p->method > 3) throw std::runtime_error("unknown method");
@@ -3158,6 +3211,10 @@ std::unique_ptr<tf_ctx> make_ctx(const tf_problem* p, int32_t prec,
         std::vector<std::vector<std::pair<int32_t, double>>> none(c->E);
         std::vector<int> fld(c->E, TF_FIELD_H);
         build_tet_inject(c.get(), none, fld);
+    }
+    if (c->fit_grid || c->tet_relabel) {
+        upload(c->d_esid, c->h_esid);
+        upload(c->d_fsid, c->h_fsid);
     }
     ensure_carr(c.get(), 1, 0);
     TF_HIP(hipStreamSynchronize(c->stream));
@@ -3905,33 +3962,12 @@ tf_status tf_run(tf_ctx* c, int64_t first, int64_t n, const tf_cg_opts* cg, tf_s
 tf_status tf_read_state(tf_ctx* c, double* U, double* F, double* B) {
     if (!c) { g_err = "null argument"; return TF_ERR_ARG; }
     return guarded([&] {
-        TF_HIP(hipStreamSynchronize(c->stream));
-        auto rd = [&](const DevBuf& b, double* dst, int64_t n) {
-            if (!dst) return;
-            if (c->prec == TF_PREC_FP64) {
-                TF_HIP(hipMemcpy(dst, b.p, n * 8, hipMemcpyDeviceToHost));
-            } else {
-                std::vector<float> tmp(n);
-                TF_HIP(hipMemcpy(tmp.data(), b.p, n * 4, hipMemcpyDeviceToHost));
-                for (int64_t i = 0; i < n; ++i) dst[i] = tmp[i];
-            }
-        };
-        // FIT grid order or tet locality order: entity i sits at device position pos[i]
-        auto rd_perm = [&](const DevBuf& b, double* dst, int64_t n, const std::vector<int32_t>& pos) {
-            if (!dst) return;
-            std::vector<double> tmp(n);
-            rd(b, tmp.data(), n);
-            for (int64_t i = 0; i < n; ++i) dst[i] = tmp[pos[i]];
-        };
-        if (c->fit_grid || c->tet_relabel) {
-            rd_perm(c->U, U, c->E, c->h_esid);
-            if (!c->fem) rd_perm(c->Fv, F, c->F, c->h_fsid);
-            rd_perm(c->B, B, c->F, c->h_fsid);
-        } else {
-            rd(c->U, U, c->E);
-            if (!c->fem) rd(c->Fv, F, c->F);
-            rd(c->B, B, c->F);
-        }
+        const bool perm = c->fit_grid || c->tet_relabel;
+        const int32_t* ep = perm ? c->d_esid.as<int32_t>() : nullptr;
+        const int32_t* fp = perm ? c->d_fsid.as<int32_t>() : nullptr;
+        read_field(c, c->U, ep, 0, c->E, U);
+        if (!c->fem) read_field(c, c->Fv, fp, 0, c->F, F);
+        read_field(c, c->B, fp, 0, c->F, B);
         // fem has no F field (its buffer holds N C U_old of the last step)
         if (c->fem && F) std::fill(F, F + c->F, 0.0);
     });
@@ -3952,21 +3988,12 @@ tf_status tf_write_state(tf_ctx* c, const double* U, const double* F, const doub
                 TF_HIP(hipMemcpy(b.p, tmp.data(), n * 4, hipMemcpyHostToDevice));
             }
         };
-        if (c->fit_grid || c->tet_relabel) {
-            auto wr_perm = [&](DevBuf& b, const double* src, int64_t n, const std::vector<int32_t>& pos) {
-                if (!src) return;
-                std::vector<double> tmp(n);
-                for (int64_t i = 0; i < n; ++i) tmp[pos[i]] = src[i];
-                wr(b, tmp.data(), n);
-            };
-            wr_perm(c->U, U, c->E, c->h_esid);
-            wr_perm(c->Fv, F, c->F, c->h_fsid);
-            wr_perm(c->B, B, c->F, c->h_fsid);
-        } else {
-            wr(c->U, U, c->E);
-            wr(c->Fv, F, c->F);
-            wr(c->B, B, c->F);
-        }
+        const bool perm = c->fit_grid || c->tet_relabel;
+        const int32_t* ep = perm ? c->d_esid.as<int32_t>() : nullptr;
+        const int32_t* fp = perm ? c->d_fsid.as<int32_t>() : nullptr;
+        write_field(c, c->U, ep, c->E, U);
+        write_field(c, c->Fv, fp, c->F, F);
+        write_field(c, c->B, fp, c->F, B);
         if (U) {
             c->ud_zero = true;
             for (int32_t e : c->h_dir_edge)
@@ -4323,14 +4350,12 @@ tf_status tf_batch_read_probes(tf_ctx* c, int32_t inst, double* times, double* v
 tf_status tf_batch_read_state(tf_ctx* c, int32_t inst, double* U, double* F, double* B) {
     if (!c || !c->batch || inst < 0 || inst >= c->batch->n) { g_err = "bad argument"; return TF_ERR_ARG; }
     return guarded([&] {
+        // the instance's range only (batches keep the instances' numbering)
         auto& b = *c->batch;
-        std::vector<double> u(c->E), f(c->F), bb(c->F);
-        const tf_status rc = tf_read_state(c, u.data(), f.data(), bb.data());
-        if (rc != TF_OK) throw std::runtime_error(g_err);
-        const int32_t eo = b.eoff[inst], fo = b.foff[inst];
-        if (U) std::copy(u.begin() + eo, u.begin() + eo + b.ecnt[inst], U);
-        if (F) std::copy(f.begin() + fo, f.begin() + b.foff[inst + 1], F);
-        if (B) std::copy(bb.begin() + fo, bb.begin() + b.foff[inst + 1], B);
+        const int32_t eo = b.eoff[inst], fo = b.foff[inst], nf = b.foff[inst + 1] - fo;
+        read_field(c, c->U, nullptr, eo, b.ecnt[inst], U);
+        read_field(c, c->Fv, nullptr, fo, nf, F);
+        read_field(c, c->B, nullptr, fo, nf, B);
     });
 }
 
