@@ -40,6 +40,7 @@ struct SellView {
     const V* val;
     int32_t cwin;
     int32_t band;  // waves take each XCD's slices round-robin (block_slices)
+    int32_t keep;  // wide-mesh kernels: slices s with s % 8 < keep are loaded to stay in cache (sell_dot)
 };
 
 // Column of a 16-bit code in the windowed form, with the slice's four bases
@@ -102,8 +103,8 @@ __device__ __forceinline__ double sell_value<double, uint16_t>(uint16_t v) {
 // depend on U or on the launch shape. W selects the wide-mesh instantiation:
 // the windowed 16-bit column decode compiled in and non-temporal operator
 // loads (stream_load); the kernels below take W from their launch.
-template <typename A, int U, bool W, typename V, class G>
-__device__ __forceinline__ double sell_dot(const SellView<V>& m, int s, int lane, G gather) {
+template <typename A, int U, bool W, bool NT, typename V, class G>
+__device__ __forceinline__ double sell_dot_nt(const SellView<V>& m, int s, int lane, G gather) {
     s = __builtin_amdgcn_readfirstlane(s);
     const int64_t base = m.sptr[s];
     const int w = __builtin_amdgcn_readfirstlane((int)((m.sptr[s + 1] - base) / kSlice));
@@ -116,7 +117,7 @@ __device__ __forceinline__ double sell_dot(const SellView<V>& m, int s, int lane
         for (int u = 0; u < U; ++u) {
             const int kk = full ? k0 + u : min(k0 + u, w - 1);  // clamped: loads stay inside the slice
             ci[u] = col_at(kk * kSlice + lane);
-            vi[u] = sell_value<A, V>(stream_load<W>(v + kk * kSlice + lane));
+            vi[u] = sell_value<A, V>(stream_load<NT>(v + kk * kSlice + lane));
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) gi[u] = (A)gather(ci[u]);
@@ -132,16 +133,28 @@ __device__ __forceinline__ double sell_dot(const SellView<V>& m, int s, int lane
     if (W && m.col16 && m.cwin) {
         const uint16_t* c = m.col16 + base;
         const ColWin cw = col_windows(m, s);
-        rows([&](int o) { return win_col(cw, stream_load<W>(c + o)); });
+        rows([&](int o) { return win_col(cw, stream_load<NT>(c + o)); });
     } else if (m.col16) {
         const uint16_t* c = m.col16 + base;
         const int32_t cb = __builtin_amdgcn_readfirstlane(m.cbase[s]);
-        rows([&](int o) { return cb + (int32_t)stream_load<W>(c + o); });
+        rows([&](int o) { return cb + (int32_t)stream_load<NT>(c + o); });
     } else {
         const int32_t* c = m.col + base;
-        rows([&](int o) { return stream_load<W>(c + o); });
+        rows([&](int o) { return stream_load<NT>(c + o); });
     }
     return (double)acc;
+}
+
+// The wide-mesh instantiation loads the operator non-temporally, except for the
+// share m.keep / 8 of its slices (spread over all XCDs).
+template <typename A, int U, bool W, typename V, class G>
+__device__ __forceinline__ double sell_dot(const SellView<V>& m, int s, int lane, G gather) {
+    if constexpr (W) {
+        if ((__builtin_amdgcn_readfirstlane(s) & 7) < m.keep) return sell_dot_nt<A, U, W, false>(m, s, lane, gather);
+        return sell_dot_nt<A, U, W, true>(m, s, lane, gather);
+    } else {
+        return sell_dot_nt<A, U, W, false>(m, s, lane, gather);
+    }
 }
 
 __device__ __forceinline__ int wave_id() { return (blockIdx.x * blockDim.x + threadIdx.x) / kWave; }

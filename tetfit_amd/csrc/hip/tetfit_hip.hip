@@ -97,12 +97,13 @@ struct Sell {
     bool c16 = false;   // 16-bit column codes (col16 + cbase) in the kernels' view
     bool cwin = false;  // ... in the four-window form (SellView::cwin)
     bool band = false;  // banded slice order (SellView::band), batched dga
+    int32_t keep = 0;       // SellView::keep
     int64_t min_width = 0;  // narrowest slice (the CG kernels' slice streams need >= 1)
     template <class V>
     SellView<V> view(const DevBuf& v) const {
         return SellView<V>{nrows, nslices, sptr.as<int64_t>(), c16 ? nullptr : col.as<int32_t>(),
                            c16 ? col16.as<uint16_t>() : nullptr, cbase.as<int32_t>(), v.as<V>(), cwin ? 1 : 0,
-                           band ? 1 : 0};
+                           band ? 1 : 0, keep};
     }
     template <class T>
     SellView<T> vals() const { return view<T>(val); }
@@ -231,6 +232,7 @@ struct tf_ctx {
     // operator uses windowed 16-bit columns, or when the operators stepped
     // each step exceed the 256 MB Infinity Cache
     bool wide = false;
+    bool wide_cg = false;  // the same for the kernels of the CG passes, by A (and G) alone
     FitGrid grid{};
     DevBuf d_esid, d_fsid, stage;         // the same on the device; staging of state reads and writes
     std::vector<int32_t> h_esid, h_fsid;  // reference edge / face -> device position (FIT grid order, tet relabel)
@@ -770,9 +772,19 @@ SellView<V> tuned_view(const tf_ctx* c, int k, SellView<V> v) {
     return with_band(v, c->tune[k]);
 }
 
+// Default grid of the CG pass kernels: as many workgroups as give every wave
+// the same number of slices, at most cap. (Up to the cap itself, 48^3's 11,881
+// slices left waves with one or two: learned FP32 0.499 ms a step against 0.444,
+// plain FP64 1.149 against 1.089; 64^3 FP64 3.00 against 2.93.)
+int even_blocks(const Sell& m, int cap) {
+    constexpr int wpb = kBlock / kWave;
+    const int per = std::max(1, (m.nslices + cap * wpb - 1) / (cap * wpb));
+    return std::max(1, (m.nslices + per * wpb - 1) / (per * wpb));
+}
 int tuned_blocks(const tf_ctx* c, int k, const Sell& m, int cap) {
     const int b = c->tune[k].blocks;
-    return b > 0 ? std::max(1, std::min(b, std::min(cap, sell_blocks(m, INT32_MAX)))) : sell_blocks(m, cap);
+    if (b <= 0) return k >= TK_W ? even_blocks(m, cap) : sell_blocks(m, cap);
+    return std::max(1, std::min(b, std::min(cap, sell_blocks(m, INT32_MAX))));
 }
 
 template <class T>
@@ -831,8 +843,10 @@ void launch_timed(tf_ctx* c, const char* name, K kernel, int grid, Args... args)
     hipExtLaunchKernelGGL(kernel, dim3(grid), dim3(kBlock), 0, c->stream, r.a, r.b, 0, args...);
 }
 #define TF_LAUNCH_TIMED(c, name, nb, kern, T, grid, ...)                                       \
+    TF_LAUNCH_TIMED_W(c, (c)->wide, name, nb, kern, T, grid, __VA_ARGS__)
+#define TF_LAUNCH_TIMED_W(c, w, name, nb, kern, T, grid, ...)                                  \
     do {                                                                                    \
-        if ((c)->wide) {                                                                    \
+        if (w) {                                                                            \
             switch (nb) {                                                                   \
                 case 4: launch_timed(c, name, kern<T, 4, true>, grid, __VA_ARGS__); break;     \
                 case 16: launch_timed(c, name, kern<T, 16, true>, grid, __VA_ARGS__); break;   \
@@ -1474,11 +1488,32 @@ void create_tet(tf_ctx* c, const tf_problem* p, const std::vector<int32_t>* batc
                                 ? bytes(c->sCt) + bytes(c->H) + bytes(c->N) + bytes(c->fKu) + bytes(c->fRu) +
                                       bytes(c->fKf) + bytes(c->fRf)
                                 : bytes(c->A) + 4 * (size_t)c->A.entries;
+    c->wide_cg = c->A.cwin || streamed > ((size_t)256 << 20);
     c->wide = c->wide || streamed > ((size_t)256 << 20);
     // $TETFIT_SELL_WIDE (non-empty, not 0) selects the wide-mesh kernels on
     // any mesh, to exercise them with one-base columns on small meshes
     if (const char* v = std::getenv("TETFIT_SELL_WIDE"))
-        if (*v && std::strcmp(v, "0") != 0) c->wide = true;
+        if (*v && std::strcmp(v, "0") != 0) c->wide = c->wide_cg = true;
+    // Resident share of an operator that is read over and over: next to the
+    // vectors the passes use (kept by their ordinary loads) about 215 MB of the
+    // Infinity Cache hold. A cyclic read of more than fits would keep none of
+    // it (64^3 fp64 gfdtd, A 206 MB beside 102 MB of vectors: cg_w 71 us all
+    // non-temporal, 73 us all cached, 60 us with half cached and the step 2.95 ->
+    // 2.72 ms; dga 56^3 fp64 152 -> 144 us, 72^3 fp32 204 -> 198 us a step).
+    auto share = [&](Sell& m, size_t& used) {
+        const size_t budget = (size_t)215 << 20, nb = bytes(m);
+        if (!nb || used >= budget) return;
+        m.keep = (int32_t)std::min<size_t>(8, 8 * (budget - used) / nb);
+        used += nb / 8 * m.keep;
+    };
+    if (p->method == TF_METHOD_DGA) {
+        size_t used = c->tsize * (2 * (size_t)E + 3 * (size_t)F) + c->c_col.bytes;
+        if (c->wide) share(c->N, used);
+        if (c->wide && !c->H.cwin) share(c->H, used);
+    } else if (c->wide_cg && !c->A.cwin) {
+        size_t used = 7 * c->tsize * (size_t)c->n_free;
+        share(c->A, used);
+    }
     // initial U: fixed (class-4) values
     std::vector<T> u0(E, 0);
     for (int32_t e = 0; e < E; ++e)
@@ -2322,17 +2357,17 @@ void cg_passes(tf_ctx* c, CgSolve& cs, int n) {
     const int stop = std::min(cs.it + n, cs.init.maxiter + 1);
     for (int& it = cs.it; it < stop; ++it) {
         if (cs.learned) {
-            TF_LAUNCH_TIMED(c, "cg_pg_kernel", c->tune[TK_G].unroll, cg_pg_kernel, T, v.nb_g, it, v.G, v.gpk,
+            TF_LAUNCH_TIMED_W(c, c->wide_cg, "cg_pg_kernel", c->tune[TK_G].unroll, cg_pg_kernel, T, v.nb_g, it, v.G, v.gpk,
                             (const RS<T>*)v.rs[it == 0 ? 0 : (it - 1) & 1], v.rs[it & 1], (const T*)v.p, v.x,
                             v.u, (const double*)v.part_del, v.nb_w, v.part_gl, v.part_rl, dst);
             tag(it, 1);
-            TF_LAUNCH_TIMED(c, "cg_wu_kernel", c->tune[TK_WU].unroll, cg_wu_kernel, T, v.nb_w, it, v.A,
+            TF_LAUNCH_TIMED_W(c, c->wide_cg, "cg_wu_kernel", c->tune[TK_WU].unroll, cg_wu_kernel, T, v.nb_w, it, v.A,
                             (const T*)v.u, v.p, v.rs[it & 1], (const double*)v.part_rl, (const double*)v.part_gl,
                             v.nb_g, v.part_del, dst);
             tag(it, 0);
             continue;  // at it == maxiter the stop test of cg_wu ends the solve
         }
-        TF_LAUNCH_TIMED(c, "cg_w_kernel", c->tune[TK_W].unroll, cg_w_kernel, T, v.nb_w, it, v.A, (const T*)v.u,
+        TF_LAUNCH_TIMED_W(c, c->wide_cg, "cg_w_kernel", c->tune[TK_W].unroll, cg_w_kernel, T, v.nb_w, it, v.A, (const T*)v.u,
                         v.w, 1, (const double*)v.part_rr, v.nb_b, v.part_del, dst, CgBatch{});
         tag(it, 0);
         if (it == cs.init.maxiter) { ++it; break; }  // the pass at maxiter only runs the stop test
@@ -3473,7 +3508,7 @@ void autotune(tf_ctx* c) {
         const int nbb = std::max(1, std::min(blocks_for(nf), kCgPartB));  // cg_upd's grid (CgView)
         // Jacobi pass: cg_w (stop test on cg_upd's partials) + the cg_upd that sums its b partials
         c->tune[TK_W] = tune_one(c, TK_W, c->A, kCgPartA, [&](const KTune& t) {
-            TF_LAUNCH_NB(c->wide, t.unroll, cg_w_kernel, T, t.blocks, s, 1, with_band(c->A.vals<T>(), t), c->z.as<T>(),
+            TF_LAUNCH_NB(c->wide_cg, t.unroll, cg_w_kernel, T, t.blocks, s, 1, with_band(c->A.vals<T>(), t), c->z.as<T>(),
                          c->q.as<T>(), 1, one, nbb, part, st, CgBatch{});
             cg_upd_kernel<T><<<nbb, kBlock, 0, s>>>(1, nf, c->pre.as<T>(), c->q.as<T>(), c->r.as<T>(), c->z.as<T>(),
                                                     c->q.as<T>(), c->p0.as<T>(), c->p1.as<T>(), one, nbb, one,
@@ -3483,12 +3518,12 @@ void autotune(tf_ctx* c) {
             const SellView<uint16_t> gv = c->A.view<uint16_t>(c->lp.gval);
             const uint32_t* gpk = c->lp.gpk.p ? c->lp.gpk.as<uint32_t>() : nullptr;
             auto pg = [&](const KTune& t, int nparts) {
-                TF_LAUNCH_NB(c->wide, t.unroll, cg_pg_kernel, T, t.blocks, s, 1, with_band(gv, t), gpk,
+                TF_LAUNCH_NB(c->wide_cg, t.unroll, cg_pg_kernel, T, t.blocks, s, 1, with_band(gv, t), gpk,
                              c->rs0.as<RS<T>>(), c->rs1.as<RS<T>>(), c->p0.as<T>(), c->q.as<T>(), c->z.as<T>(), one,
                              nparts, part, part, st);
             };
             auto wu = [&](const KTune& t, int nparts) {
-                TF_LAUNCH_NB(c->wide, t.unroll, cg_wu_kernel, T, t.blocks, s, 1, with_band(c->A.vals<T>(), t),
+                TF_LAUNCH_NB(c->wide_cg, t.unroll, cg_wu_kernel, T, t.blocks, s, 1, with_band(c->A.vals<T>(), t),
                              c->z.as<T>(), c->p0.as<T>(), c->rs1.as<RS<T>>(), one, one, nparts, part, st);
             };
             // cg_pg (summing cg_wu's partials) + the cg_wu that sums its b partials, then
@@ -3721,7 +3756,7 @@ void run_gfdtd_batch(tf_ctx* c, int64_t first, int64_t n, const tf_cg_opts* cg, 
         auto passes = [&](int m) {
             const int stop = std::min(it + m, init.maxiter + 1);
             for (; it < stop; ++it) {
-                TF_LAUNCH_TIMED(c, "cg_w_kernel", c->tune[TK_W].unroll, cg_w_kernel, T, nb, it, A,
+                TF_LAUNCH_TIMED_W(c, c->wide_cg, "cg_w_kernel", c->tune[TK_W].unroll, cg_w_kernel, T, nb, it, A,
                                 (const T*)c->z.as<T>(), c->q.as<T>(), 1, (const double*)part_rr, nb, part_del, states,
                                 bt);
                 if (it == init.maxiter) { ++it; break; }
