@@ -601,6 +601,25 @@ __device__ __forceinline__ void block_sum2_all(double& a, double& b, double* red
 }
 constexpr int kRed2 = 2 * (kBlock / kWave) + 2;
 
+// The same for three values; red holds 3 * (waves per block) doubles.
+__device__ __forceinline__ void block_sum3_all(double (&v)[3], double* red) {
+    constexpr int nw = kBlock / kWave;
+    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        v[a] = group_sum<kWave>(v[a]);
+        if (lane == 0) red[a * nw + w] = v[a];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        double s = 0;
+        for (int i = 0; i < nw; ++i) s += red[a * nw + i];
+        v[a] = s;
+    }
+    __syncthreads();
+}
+
 // Stop decision of pass `it` from the residual norm RR = ||r_it||^2 (the
 // reference's test, ConjugateGradientSolver.hpp:68-74): stop unless
 // ||r|| / ||r0|| > tol and it < maxiter. Every block decides the same;
@@ -761,6 +780,167 @@ __global__ void __launch_bounds__(kBlock) cg_w_kernel(int32_t it, SellView<T> m,
     }
     block_sum2_all(wu, none, red);
     if (threadIdx.x == 0) part_del[blockIdx.x] = wu;
+}
+
+// One Jacobi iteration per launch, for systems whose passes are bound by
+// launches and latency rather than bytes. Per row the solver keeps (r, w, s,
+// 1/diag) side by side; with alpha and beta of pass `it` known, every lane that
+// needs u_{it+1} of a row forms it from that quadruple,
+//   s' = w + beta s,  r' = r - alpha s',  u' = pre r',
+// with the roundings of the row's owner, so that w' = A u' needs no kernel
+// boundary after the updates. One launch then does: the stop test on r_it, the
+// scalars, p, s, x, r of the owned rows, w_{it+1} = A u_{it+1}, and the partials
+// of gamma, delta and ||r||^2 of pass it + 1. it = -1 starts a solve: w_0 = A u_0
+// from r_0. The first batch of entries and quadruples is loaded before the
+// scalars are reduced. Iterates are those of cg_w / cg_upd.
+// 16^3 fp64: 8.3 us a pass against 6.5 + 4.7, the step 331 -> 273 us; 32^3 fp32
+// 11.6 against 7.6 + 6.5, 432 -> 364 us. A gathered row is four values instead
+// of one, so it loses once the rows leave an XCD's 4 MB L2: 32^3 fp64 (7.1 MB)
+// 538 -> 625 us. Twelve entries a batch spill the gain (16^3 fp64 302 us).
+template <typename T>
+struct alignas(4 * sizeof(T)) CgRow {
+    T r, w, s, pre;
+};
+template <typename T>
+__device__ __forceinline__ CgRow<T> cg_row_next(const CgRow<T>& q, double alpha, double beta, int32_t it, T& u) {
+    CgRow<T> o = q;
+    if (it >= 0) {
+        o.s = it == 0 ? q.w : (T)__builtin_fma(beta, (double)q.s, (double)q.w);
+        o.r = cg_r_next(q.r, o.s, alpha);
+    }
+    u = (T)((double)q.pre * (double)o.r);
+    return o;
+}
+constexpr int kOneMax = 1024;  // partials per array (workgroups of a solve) at most
+
+template <typename T, int NB>
+__global__ void __launch_bounds__(kBlock) cg_one_kernel(int32_t it, SellView<T> m, const CgRow<T>* __restrict__ q,
+                                                        CgRow<T>* __restrict__ qo, T* __restrict__ p,
+                                                        T* __restrict__ x, const double* __restrict__ part_in,
+                                                        double* __restrict__ part_out, int32_t nb, CgState* st) {
+    __shared__ double red[3 * (kBlock / kWave)];
+    constexpr int per = kOneMax / kBlock;
+    const bool leader = blockIdx.x == 0;
+    double sums[3] = {0, 0, 0};  // gamma, delta, ||r||^2 of pass it
+    double pv[3][per];
+    const int np = it >= 0 ? nb : 0;
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+        for (int k = 0; k < per; ++k) {
+            const int i = (int)threadIdx.x + k * kBlock;
+            pv[a][k] = part_in[a * kOneMax + (i < np ? i : 0)];
+        }
+    const int done = st->done;
+    const double rr0 = st->rr0, tol = st->tol, gam_prev = st->gam[(it - 1) & 1], alpha_prev = st->alpha[(it - 1) & 1];
+    const int32_t maxiter = st->maxiter, given = st->rr0_given;
+    const int lane = lane_id();
+    SliceRange sr = block_slices(m.nslices, m.band);
+    T v[NB];
+    CgRow<T> g[NB], own;
+    T pown = 0, xown = 0;
+    int w = 0;
+    auto load = [&](int s, int k0) {
+        s = __builtin_amdgcn_readfirstlane(s);
+        const int64_t base = scalar_load(m.sptr + s);
+        w = (int)((scalar_load(m.sptr + s + 1) - base) / kSlice);
+        int32_t ci[NB];
+        auto entries = [&](auto col_at) {
+#pragma unroll
+            for (int u = 0; u < NB; ++u) {
+                const int64_t o = base + (int64_t)min(k0 + u, w - 1) * kSlice + lane;  // clamped: inside the slice
+                ci[u] = col_at(o);
+                v[u] = m.val[o];
+            }
+        };
+        if (m.col16 && m.cwin) {
+            const ColWin cw = col_windows(m, s);
+            entries([&](int64_t o) { return win_col(cw, m.col16[o]); });
+        } else if (m.col16) {
+            const int32_t cb = scalar_load(m.cbase + s);
+            entries([&](int64_t o) { return cb + (int32_t)m.col16[o]; });
+        } else {
+            entries([&](int64_t o) { return m.col[o]; });
+        }
+#pragma unroll
+        for (int u = 0; u < NB; ++u) g[u] = q[ci[u]];
+        if (k0 == 0) {
+            const int32_t i = min(s * kSlice + lane, m.nrows - 1);
+            own = q[i];
+            pown = p[i];
+            xown = x[i];
+        }
+    };
+    if (sr.s < sr.end) load(sr.s, 0);
+    if (done) return;
+    double alpha = 0, beta = 0;
+    if (it >= 0) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+#pragma unroll
+            for (int k = 0; k < per; ++k) sums[a] += (int)threadIdx.x + k * kBlock < np ? pv[a][k] : 0.0;
+        block_sum3_all(sums, red);
+        if (cg_decide_stop(it, sums[2], rr0, given, tol, maxiter, st, leader)) return;
+        if (it == 0) {
+            alpha = sums[0] / sums[1];
+        } else {
+            beta = sums[0] / gam_prev;
+            alpha = sums[0] / (sums[1] - beta * sums[0] / alpha_prev);
+        }
+        if (threadIdx.x == 0 && leader) {
+            st->gam[it & 1] = sums[0];
+            st->alpha[it & 1] = alpha;
+        }
+    }
+    double ru = 0, wu = 0, rr = 0;
+    for (; sr.s < sr.end; sr.s += sr.step) {
+        T acc = 0;
+        for (int k0 = 0;;) {
+#pragma unroll
+            for (int u = 0; u < NB; ++u) {
+                T uj;
+                cg_row_next(g[u], alpha, beta, it, uj);
+                if (k0 + u < w) acc += v[u] * uj;
+            }
+            k0 += NB;
+            if (k0 >= w) break;
+            load(sr.s, k0);
+        }
+        const int32_t i = sr.s * kSlice + lane;
+        const CgRow<T> o = own;
+        const T po = pown, xo = xown;
+        const int sn = sr.s + sr.step;
+        if (sn < sr.end) load(sn, 0);
+        if (i < m.nrows) {
+            T ui;
+            CgRow<T> n = cg_row_next(o, alpha, beta, it, ui);
+            if (it >= 0) {
+                // p and x of pass it (u_it = pre r_it)
+                const T uo = (T)((double)o.pre * (double)o.r);
+                const T pi = it == 0 ? uo : (T)__builtin_fma(beta, (double)po, (double)uo);
+                p[i] = pi;
+                x[i] = (T)__builtin_fma(alpha, (double)pi, (double)xo);
+            } else {
+                n.s = 0;
+            }
+            n.w = acc;
+            qo[i] = n;
+            ru += (double)n.r * (double)ui;
+            wu += (double)acc * (double)ui;
+            rr += (double)n.r * (double)n.r;
+        }
+    }
+    double out[3] = {ru, wu, rr};
+    block_sum3_all(out, red);
+    if (threadIdx.x < 3) part_out[threadIdx.x * kOneMax + blockIdx.x] = out[threadIdx.x];
+}
+
+// q[i].pre = pre[i]: the part of the rows that no pass changes.
+template <typename T>
+__global__ void __launch_bounds__(kBlock) cg_rows_init_kernel(int32_t n, const T* __restrict__ pre,
+                                                              CgRow<T>* __restrict__ q) {
+    const int32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) q[i] = CgRow<T>{(T)0, (T)0, (T)0, pre[i]};
 }
 
 // Jacobi vector updates of pass `it`; gamma and delta from their partials,

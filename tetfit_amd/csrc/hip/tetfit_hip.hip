@@ -287,6 +287,7 @@ struct tf_ctx {
     DevBuf free_edge, dir_edge, dir_new, fb, pre, x, r, z, p0, p1, q, r0, cg_part, cg_state;
     DevBuf edge_row;  // per edge: its free row in the CG order, or -1 (Dirichlet)
     DevBuf rs0, rs1;  // (r, s) pairs of the learned passes, even / odd pass
+    DevBuf q4[2], one_part;  // cg_one_kernel: rows before / after a pass, partials of two passes
     // extrapolated starts (tf_cg_opts.guess): U_{n-1}, U_{n-2} on the free
     // rows, the start's shift d, gf_rhs_init's partials of ||b - A U_old||^2;
     // hist = steps of history held, valid for the solve of step hist_next
@@ -406,7 +407,7 @@ size_t tf_ctx::device_bytes() const {
     const DevBuf* all[] = {&U, &Fv, &B, &fit_ep, &fit_nu, &fe_sg, &fe_ca, &fe_cb, &fe_f4, &fh_sg, &fh_cm, &fh_cn, &fh_e4, &fe_id, &fe_pal, &fh_id, &fh_pal, &fh_at, &fh_val,
                            &spv, &d_esid, &d_fsid, &stage, &slots, &samp_ref, &sg.carr, &sg.poy, &sg.slot,
                            &sp_edge, &sp_f4, &sp_sg, &sp_ca, &sp_cb, &sp_kind, &sp_tb, &sp_te, &c_col, &c_sg,
-                           &h_edge, &curl_f, &curl_u, &free_edge, &edge_row, &dir_edge, &dir_new, &fb, &pre, &x, &r, &rs0, &rs1, &z,
+                           &h_edge, &curl_f, &curl_u, &free_edge, &edge_row, &dir_edge, &dir_new, &fb, &pre, &x, &r, &rs0, &rs1, &q4[0], &q4[1], &one_part, &z,
                            &p0, &p1, &q, &r0, &hx1, &hx2, &dx, &rr0part, &cg_part, &cg_state, &inj_edge, &inj_kind, &inj_tb, &inj_te, &fb_slot, &fb_pos, &fbv,
                            &term_src, &term_w, &carr, &probes, &samples, &eser, &epart, &poy, &row_dt_h, &row_dt_f,
                            &mu_a, &mu_b, &tf_a, &tf_b, &fslot, &row_dt_cg, &bt_inst, &bt_s0, &bt_s1, &bt_w0, &bt_w1, &uf[0], &uf[1], &ff[0], &ff[1], &u_out, &f_out, &u_two, &f_two,
@@ -1892,10 +1893,11 @@ void fit_indexed_step(tf_ctx* c, const FitSpecial& sp, int sp_blocks, const doub
 // instead of 12.4 us a step at 64^3 fp64, 22.5 instead of 24.7 at 90^3 and 163
 // instead of 185 at 161^3 random fp64; four gain only where an item's loads are
 // 4 bytes and the grid is large: 128^3 fp32 33.1 against 35.3 us, 161^3 fp64
-// 168 against 163, 48^3 fp32 8.7 against 8.3.
+// 168 against 163, 48^3 fp32 8.7 against 8.3. Below about 17^3 the step is one
+// workgroup's latency: 16^3 fp64 6.6 us with one item, 6.7 with two.
 template <class T>
 int fit_items(int64_t edges) {
-    return sizeof(T) == 4 && edges >= (1 << 22) ? 4 : 2;
+    return edges < (1 << 16) ? 1 : sizeof(T) == 4 && edges >= (1 << 22) ? 4 : 2;
 }
 
 template <class T>
@@ -1956,9 +1958,11 @@ void run_fit(tf_ctx* c, int64_t first, int64_t n, tf_stats* st) {
         const int per = fit_items<T>(c->E);
         const int e_grid = sp_blocks + e.probe_blocks + slab_grid(ecnt, per * kBlock);
         const int h_grid = sp_blocks + h.probe_blocks + slab_grid(fcnt, per * kBlock);
-        const auto ek = per == 2 ? (c->fe_pal.p ? fit_e_grid_kernel<T, true, 2> : fit_e_grid_kernel<T, false, 2>)
+        const auto ek = per == 1 ? (c->fe_pal.p ? fit_e_grid_kernel<T, true, 1> : fit_e_grid_kernel<T, false, 1>)
+                      : per == 2 ? (c->fe_pal.p ? fit_e_grid_kernel<T, true, 2> : fit_e_grid_kernel<T, false, 2>)
                                  : (c->fe_pal.p ? fit_e_grid_kernel<T, true, 4> : fit_e_grid_kernel<T, false, 4>);
-        const auto hk = per == 2 ? (c->fh_pal.p ? fit_h_grid_kernel<T, true, 2> : fit_h_grid_kernel<T, false, 2>)
+        const auto hk = per == 1 ? (c->fh_pal.p ? fit_h_grid_kernel<T, true, 1> : fit_h_grid_kernel<T, false, 1>)
+                      : per == 2 ? (c->fh_pal.p ? fit_h_grid_kernel<T, true, 2> : fit_h_grid_kernel<T, false, 2>)
                                  : (c->fh_pal.p ? fit_h_grid_kernel<T, true, 4> : fit_h_grid_kernel<T, false, 4>);
         // slot: row of the step before (its B is sampled by the E phase)
         auto step = [&](const double* cs, double* poy, const int64_t* slot, bool store_b) {
@@ -2247,6 +2251,7 @@ void run_dga(tf_ctx* c, int64_t first, int64_t n, tf_stats* st) {
 struct CgSolve {
     CgState init{};
     bool learned = false;
+    bool one = false;  // one launch per pass (cg_one_kernel)
     const std::vector<std::pair<int, int>>* snaps = nullptr;
     int slot = 0;  // CG state slot (device cg_state[slot], pinned h_state[slot])
     bool dir_terms = true;  // gf_rhs_init: apply K U_old - RHS1 SrcFld (false: known to be zero)
@@ -2306,8 +2311,8 @@ void cg_start(tf_ctx* c, CgSolve& cs, bool with_rhs, const CgState* guard, int e
     // for the solve after next, after the host has waited on this one
     c->init_src[cs.slot] = cs.init;
     TF_HIP(hipMemcpyAsync(dst, &c->init_src[cs.slot], sizeof(CgState), hipMemcpyHostToDevice, c->stream));
-    T* r0 = cs.learned ? &v.rs[0]->r : v.rj;
-    const int r0_stride = cs.learned ? 2 : 1;
+    T* r0 = cs.learned ? &v.rs[0]->r : cs.one ? &c->q4[0].as<CgRow<T>>()->r : v.rj;
+    const int r0_stride = cs.learned ? 2 : cs.one ? 4 : 1;
     if (with_rhs) {
         // gfdtd: r0 = (K U - RHS1 SrcFld) + dt Ct F + dt fb; fem: r0 = (E W /
         // dt^2 - 0.5/dt SigMat W2) - Ct (N C U_old) + fb / dt
@@ -2322,7 +2327,7 @@ void cg_start(tf_ctx* c, CgSolve& cs, bool with_rhs, const CgState* guard, int e
                         c->free_edge.as<int32_t>(), c->fem ? c->fw.as<T>() : c->U.as<T>(),
                         c->fem ? c->fw2.as<T>() : c->dir_new.as<T>(), c->Fv.as<T>(), c->fb.as<T>(),
                         c->r0.as<T>(), co, c->pre.as<T>(), r0, r0_stride, v.u, v.part_rr, v.part_gj[0], dst,
-                        cs.learned ? 0 : 1, guard, v.A, shifted ? (const T*)c->dx.as<T>() : nullptr,
+                        cs.learned || cs.one ? 0 : 1, guard, v.A, shifted ? (const T*)c->dx.as<T>() : nullptr,
                         c->rr0part.as<double>(), CgBatch{}, (const double*)nullptr);
         if (shifted)
             launch_timed(c, "cg_set_rr0_kernel", cg_set_rr0_kernel, 1, c->rr0part.as<double>(), v.nb_b, dst, guard);
@@ -2344,6 +2349,31 @@ void cg_capture(tf_ctx* c, const CgSolve& cs, const CgView<T>& v, int k) {
                                                                                      c->lp.Cb.as<float>());
 }
 
+// Whether the Jacobi solves of a context run one launch per pass
+// (cg_one_kernel): its rows fit an XCD's 4 MB L2 (fp64 up to about 25^3 Kuhn
+// meshes, fp32 up to about 32^3; the kernel's comment has both sides).
+template <class T>
+bool one_launch_passes(const tf_ctx* c) {
+    return c->n_free > 0 && (size_t)c->n_free * sizeof(CgRow<T>) <= ((size_t)4 << 20);
+}
+// Buffers of cg_one_kernel (partials: three arrays per pass parity).
+template <class T>
+void one_prepare(tf_ctx* c) {
+    if (c->q4[0].p) return;
+    for (DevBuf& b : c->q4) b.alloc((size_t)c->n_free * sizeof(CgRow<T>));
+    c->one_part.alloc(6 * (size_t)kOneMax * sizeof(double));
+    cg_rows_init_kernel<T><<<blocks_for(c->n_free), kBlock, 0, c->stream>>>(c->n_free, c->pre.as<T>(),
+                                                                          c->q4[0].as<CgRow<T>>());
+}
+template <class T>
+void cg_one_launch(tf_ctx* c, int it, int nb, CgState* st) {
+    const int in = (it + 1) & 1, out = in ^ 1;
+    double* part = c->one_part.as<double>();
+    launch_timed(c, "cg_one_kernel", cg_one_kernel<T, 8>, nb, it, c->A.vals<T>(),
+                 (const CgRow<T>*)c->q4[in].as<CgRow<T>>(), c->q4[out].as<CgRow<T>>(), c->p0.as<T>(), c->x.as<T>(),
+                 (const double*)(part + in * 3 * (size_t)kOneMax), part + out * 3 * (size_t)kOneMax, nb, st);
+}
+
 // Launches passes [cs.it, min(cs.it + n, maxiter + 1)) and then an async copy
 // of the state into the pinned slot.
 template <class T>
@@ -2355,6 +2385,14 @@ void cg_passes(tf_ctx* c, CgSolve& cs, int n) {
     };
     if (cs.it == 0) cg_capture<T>(c, cs, v, 0);
     const int stop = std::min(cs.it + n, cs.init.maxiter + 1);
+    if (cs.one) {
+        const int nb = even_blocks(c->A, kOneMax);
+        for (int it = cs.it == 0 ? -1 : cs.it; it < stop; ++it) {
+            cg_one_launch<T>(c, it, nb, dst);
+            tag(it, 0);
+        }
+        cs.it = stop;
+    }
     for (int& it = cs.it; it < stop; ++it) {
         if (cs.learned) {
             TF_LAUNCH_TIMED_W(c, c->wide_cg, "cg_pg_kernel", c->tune[TK_G].unroll, cg_pg_kernel, T, v.nb_g, it, v.G, v.gpk,
@@ -2921,6 +2959,8 @@ void run_gfdtd(tf_ctx* c, int64_t first, int64_t n, const tf_cg_opts* cg, tf_sta
     LearnedPc& L = c->lp;
     const int gb_n = tuned_blocks(c, TK_N, c->N, kSpmvCap);
     CgState* states = c->cg_state.as<CgState>();
+    const bool one = !want_learned && one_launch_passes<T>(c);
+    if (one) one_prepare<T>(c);
 
     // The Dirichlet terms of step k's residual vanish when every Dirichlet
     // value is zero: always for steps after the first of the run (the
@@ -2968,6 +3008,7 @@ void run_gfdtd(tf_ctx* c, int64_t first, int64_t n, const tf_cg_opts* cg, tf_sta
         CgSolve s0;
         s0.init = init;
         s0.learned = g.learned;
+        s0.one = one;
         s0.slot = (int)(k & 1);
         s0.dir_terms = dir_terms(k);
         if (fresh) g.extrap = start_of(i, g.learned);
@@ -3018,6 +3059,7 @@ void run_gfdtd(tf_ctx* c, int64_t first, int64_t n, const tf_cg_opts* cg, tf_sta
         CgSolve sol;
         sol.init = init;
         sol.learned = learned;
+        sol.one = one;
         sol.slot = (int)(k & 1);
         std::vector<std::pair<int, int>> snaps;
         if (want_learned && L.state == LearnedPc::kCollecting) snaps = collection_snaps();
