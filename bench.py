@@ -230,16 +230,16 @@ def batch_workload(d, count=256, steps=2000, seed=4, workers=16, method="dga"):
 
 
 def fit_bytes(b, kernel, vb, grid_order=True):
-    """Algorithmic bytes per launch of the FIT kernels: E phase reads U, ca,
-    cb and the per-edge code, writes U, gathers F once; H phase reads B, cm,
-    cn and the per-face code, writes B and F, gathers U once. The code is
-    2 bytes (slot order and signs) in grid order, 17 bytes (packed faces or
-    edges and a sign byte) in the index-table layout."""
+    """Algorithmic bytes per launch of the FIT kernels on a medium of few
+    distinct coefficients. Grid order: E phase reads U and the 2-byte id,
+    writes U, gathers F once; H phase reads F and the id, writes F, gathers U
+    once (B is stored on probed faces and at the end of a run only). Index
+    tables: 17 bytes of faces or edges and signs and the two coefficients
+    besides, and H reads and writes B each step."""
     E, F = b.n_edges, b.n_faces
-    cb = 2 if grid_order else 17
     if kernel == "fit_e_kernel":
-        return E * (4 * vb + cb) + F * vb
-    return F * (5 * vb + cb) + E * vb
+        return E * (2 * vb + 2 if grid_order else 4 * vb + 17) + F * vb
+    return F * (2 * vb + 2 if grid_order else 5 * vb + 17) + E * vb
 
 
 def run_chunks(sim, steps, chunk, label, precond="jacobi", learn_steps=200, stop_before_last=False, guess=0):

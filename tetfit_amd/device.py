@@ -177,7 +177,7 @@ class Simulation:
         return self.tuning()
 
     def set_graphs(self, on):
-        """tf_set_graphs: step fdtd / dga in HIP graphs when nothing is sampled (default on)."""
+        """tf_set_graphs: step fdtd / dga in HIP graphs unless energy output or profiling is on (default on)."""
         _check(hip_lib().tf_set_graphs(self._h, int(bool(on))))
 
     def set_tuning(self, choice):
@@ -244,7 +244,7 @@ class BatchSimulation:
         self.close()
 
     def set_graphs(self, on):
-        """tf_set_graphs: step the batch in HIP graphs when nothing is sampled (default on)."""
+        """tf_set_graphs: step a dga batch in HIP graphs unless profiling is on (default on)."""
         _check(hip_lib().tf_set_graphs(self._h, int(bool(on))))
 
     def run(self, n, first=None, cg_tol=None, cg_maxiter=100):
