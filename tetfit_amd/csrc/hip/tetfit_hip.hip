@@ -4102,9 +4102,12 @@ tf_status tf_write_state(tf_ctx* c, const double* U, const double* F, const doub
         write_field(c, c->Fv, fp, c->F, F);
         write_field(c, c->B, fp, c->F, B);
         if (U) {
+            // U in the caller's numbering, h_dir_edge device edges
             c->ud_zero = true;
-            for (int32_t e : c->h_dir_edge)
-                if (U[e] != 0) c->ud_zero = false;
+            std::vector<uint8_t> dir(c->h_dir_edge.empty() ? 0 : c->E, 0);
+            for (int32_t e : c->h_dir_edge) dir[e] = 1;
+            for (size_t i = 0; i < dir.size() && c->ud_zero; ++i)
+                if (dir[dev_edge(c, (int32_t)i)] && U[i] != 0) c->ud_zero = false;
         }
         // lossy dga: each edge's (face's) value split evenly over its
         // fractional entries, the entries no edge (face) reads set to zero
