@@ -6,10 +6,12 @@ another row order, so its solves, each stopped at relative residual
 tol = 1e-10, agree within steps x tol x cond(A) / 2 per field; cond(A) of these
 meshes (epsilon contrast 10, jitter 0.2) is below 1e3: 12 steps -> 6e-7."""
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
-from tetfit_amd import configs
+from tetfit_amd import _ffi, configs
 from tetfit_amd.host import Model
 
 pytestmark = pytest.mark.gpu
@@ -45,6 +47,47 @@ def test_batch_locality_order(tmp_path, monkeypatch, method, prec):
         runs[order] = [sim.probes(k)[1:] + tuple(sim.state(k)) for k in range(len(bs))]
         sim.close()
     for k, (a, b) in enumerate(zip(runs["numbering"], runs["rank"])):
+        assert np.abs(a[1]).max() > 0, k
+        for x, y in zip(a, b):
+            if method == "dga":
+                np.testing.assert_array_equal(x, y)
+            else:
+                assert np.linalg.norm(np.asarray(x) - y) <= 6e-7 * np.linalg.norm(x), k
+
+
+class Altered:
+    """A build whose problem carries other locality ranks."""
+
+    def __init__(self, build, edge_rank, face_rank):
+        self._build = build
+        self._keep = [np.ascontiguousarray(r, np.int32) for r in (edge_rank, face_rank)]
+        p = _ffi.tf_problem.from_buffer_copy(build.problem_ptr.contents)
+        p.dga.edge_rank, p.dga.face_rank = (r.ctypes.data_as(_ffi.i32p) for r in self._keep)
+        self.problem_ptr = C.pointer(p)
+
+    def __getattr__(self, name):
+        return getattr(self._build, name)
+
+
+@pytest.mark.parametrize("method", ["dga", "gfdtd"])
+def test_batch_with_unusable_ranks(tmp_path, monkeypatch, method):
+    """Ranks that are no permutation of an instance's own entities (repeated
+    ones, and ones past its block of the stacked problem) are not used for that
+    instance, as in a batch in the instances' numbering; the others keep their
+    order."""
+    from tetfit_amd.device import BatchSimulation
+    good = instances(tmp_path, method)
+    bad = list(good)
+    bad[0] = Altered(good[0], np.zeros(good[0].n_edges), good[0].face_rank())
+    bad[2] = Altered(good[2], good[2].edge_rank() + 1, good[2].face_rank())
+    runs = []
+    for order, bs in (("numbering", good), ("rank", bad)):
+        monkeypatch.setenv("TETFIT_TET_ORDER", order)
+        sim = BatchSimulation(bs, "fp64", sample_every=1)
+        sim.run(STEPS)
+        runs.append([sim.probes(k)[1:] + tuple(sim.state(k)) for k in range(len(bs))])
+        sim.close()
+    for k, (a, b) in enumerate(zip(*runs)):
         assert np.abs(a[1]).max() > 0, k
         for x, y in zip(a, b):
             if method == "dga":

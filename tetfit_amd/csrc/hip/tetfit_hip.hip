@@ -1378,7 +1378,10 @@ void create_tet(tf_ctx* c, const tf_problem* p, const std::vector<int32_t>* batc
         upload_sell<T>(c->H, hs.v, true);
         std::vector<int32_t> row_edge(d.H.nrows, -1);
         for (int32_t e = 0; e < E; ++e)
-            if (d.h_row[e] >= 0) row_edge[d.h_row[e]] = e;
+            if (d.h_row[e] >= 0) {
+                if (d.h_row[e] >= d.H.nrows) throw std::runtime_error("h_row out of range");
+                row_edge[d.h_row[e]] = e;
+            }
         std::vector<int32_t> he(d.H.nrows);
         for (int32_t r = 0; r < d.H.nrows; ++r) {
             he[r] = row_edge[c->h_perm[r]];
@@ -3315,8 +3318,31 @@ struct MergedDga {
     tf_problem p{};
 };
 
+// Whether rank[0..n) is a permutation.
+bool is_permutation(const int32_t* rank, int32_t n) {
+    std::vector<uint8_t> seen(n, 0);
+    for (int32_t i = 0; i < n; ++i) {
+        if (rank[i] < 0 || rank[i] >= n || seen[rank[i]]) return false;
+        seen[rank[i]] = 1;
+    }
+    return true;
+}
+// Whether an instance of a batch is relabeled by its locality ranks: they are
+// permutations of its own edges and faces, and (dga) each row of H belongs to
+// one edge. Any other keeps its own numbering, which asks nothing of either.
+bool usable_ranks(const tf_problem* p) {
+    const tf_dga_ops& d = p->dga;
+    if (!d.edge_rank || !d.face_rank) return false;
+    if (!is_permutation(d.edge_rank, p->n_edges) || !is_permutation(d.face_rank, p->n_faces)) return false;
+    if (p->method != TF_METHOD_DGA) return true;
+    std::vector<int32_t> rows;
+    for (int32_t e = 0; e < p->n_edges; ++e)
+        if (d.h_row[e] >= 0) rows.push_back(d.h_row[e]);
+    return (int64_t)rows.size() == d.H.nrows && is_permutation(rows.data(), d.H.nrows);
+}
+
 // Appends an instance's locality ranks at its offsets (its own numbering when
-// it carries none), extra entries after its edges in place. The merged problem
+// it carries none to use), extra entries after its edges in place. The merged problem
 // is then relabeled inside each instance's block (relabel_tet), as a single
 // simulation is: in the instances' own numbering a slice's gathers touch about
 // twelve cache lines instead of four or five. Measured, 16 Kuhn cavities
@@ -3325,7 +3351,7 @@ struct MergedDga {
 void append_ranks(const tf_problem* p, int32_t eo, int32_t extra, int32_t fo, std::vector<int32_t>& er,
                   std::vector<int32_t>& fr, bool& ranked) {
     const tf_dga_ops& d = p->dga;
-    const bool have = d.edge_rank && d.face_rank;
+    const bool have = usable_ranks(p);
     ranked = ranked || have;
     for (int32_t e = 0; e < p->n_edges + extra; ++e)
         er.push_back(eo + (have && e < p->n_edges ? d.edge_rank[e] : e));
