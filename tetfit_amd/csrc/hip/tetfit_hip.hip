@@ -24,6 +24,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "par.hpp"
 #include "kernels.hpp"
 #include "learned.hpp"
 #include "mlp.hpp"
@@ -143,27 +144,6 @@ struct KTune {
             }                                                                               \
         }                                                                                   \
     } while (0)
-
-// Runs f(lo, hi) over [0, n) in chunks of `chunk` entries on up to 16 host
-// threads (chunk boundaries do not depend on the thread count). f must not
-// throw.
-template <class Fn>
-void par_chunks(int64_t n, int64_t chunk, const Fn& f) {
-    const int64_t nc = (n + chunk - 1) / chunk;
-    const int64_t hw = std::max(1u, std::thread::hardware_concurrency());
-    const int nt = (int)std::min<int64_t>(nc, std::min<int64_t>(hw, 16));
-    if (nt <= 1) {
-        for (int64_t k = 0; k < nc; ++k) f(k * chunk, std::min(n, (k + 1) * chunk));
-        return;
-    }
-    std::atomic<int64_t> next{0};
-    std::vector<std::thread> th;
-    for (int t = 0; t < nt; ++t)
-        th.emplace_back([&] {
-            for (int64_t k; (k = next++) < nc;) f(k * chunk, std::min(n, (k + 1) * chunk));
-        });
-    for (auto& t : th) t.join();
-}
 
 // Rows of the free-row order the learned preconditioner is trained on: all
 // of them up to this many, else a window of this many in the middle of the
