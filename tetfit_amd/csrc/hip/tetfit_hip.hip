@@ -79,11 +79,33 @@ double carrier_value(const tf_source& s, double t) {
     return ret;
 }
 
-template <class T>
-void upload(DevBuf& b, const std::vector<T>& v) {
+template <class T, class A>
+void upload(DevBuf& b, const std::vector<T, A>& v) {
     b.alloc(v.size() * sizeof(T));
     if (!v.empty()) TF_HIP(hipMemcpy(b.p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
 }
+
+// A vector whose resize() leaves new elements unset: large host tables are
+// written once, by the threads that fill them.
+template <class T>
+struct RawAlloc {
+    using value_type = T;
+    RawAlloc() = default;
+    template <class U>
+    RawAlloc(const RawAlloc<U>&) {}
+    T* allocate(size_t n) { return std::allocator<T>().allocate(n); }
+    void deallocate(T* p, size_t n) { std::allocator<T>().deallocate(p, n); }
+    template <class U>
+    void construct(U* p) { ::new ((void*)p) U; }
+    template <class U, class A>
+    void construct(U* p, A&& a) { ::new ((void*)p) U(std::forward<A>(a)); }
+    template <class U>
+    bool operator==(const RawAlloc<U>&) const { return true; }
+    template <class U>
+    bool operator!=(const RawAlloc<U>&) const { return false; }
+};
+template <class T>
+using RawVec = std::vector<T, RawAlloc<T>>;
 
 struct Csr32 {
     DevBuf ptr, col, val, sg;
@@ -294,8 +316,8 @@ struct tf_ctx {
     // host copy of A (free rows, CSR) and its SELL slice pointers, kept for
     // the learned preconditioner's pair list and features
     std::vector<int64_t> hA_ptr, hA_sptr;
-    std::vector<int32_t> hA_col;
-    std::vector<double> hA_val;
+    RawVec<int32_t> hA_col;
+    RawVec<double> hA_val;
     LearnedPc lp;
     KTune tune[TK_COUNT];
 
@@ -609,40 +631,129 @@ std::vector<int32_t> batch_row_order(const tf_dga_ops& d, const std::vector<int3
     return perm;
 }
 
-// Rows rows[0..n) of m in that order (entries keep their order), columns
-// relabeled through cmap when given.
 struct CsrBuf {
     std::vector<int64_t> rp;
-    std::vector<int32_t> col;
-    std::vector<double> val;
-    std::vector<int8_t> sg;
+    RawVec<int32_t> col;
+    RawVec<double> val;
+    RawVec<int8_t> sg;
     tf_csr v{};
 };
-void select_rows(const tf_csr& m, const int32_t* rows, int32_t n, const int32_t* cmap, CsrBuf& o) {
-    o.rp.resize((size_t)n + 1);
-    o.rp[0] = 0;
-    for (int32_t k = 0; k < n; ++k) o.rp[k + 1] = o.rp[k] + (m.rowptr[rows[k] + 1] - m.rowptr[rows[k]]);
-    o.col.resize(o.rp[n]);
-    o.val.resize(m.val ? o.rp[n] : 0);
-    o.sg.resize(m.sgn ? o.rp[n] : 0);
-    par_chunks(n, 65536, [&](int64_t lo, int64_t hi) {
-        for (int64_t k = lo; k < hi; ++k) {
-            int64_t w = o.rp[k];
-            for (int64_t q = m.rowptr[rows[k]]; q < m.rowptr[rows[k] + 1]; ++q, ++w) {
-                o.col[w] = cmap ? cmap[m.col[q]] : m.col[q];
-                if (m.val) o.val[w] = m.val[q];
-                if (m.sgn) o.sg[w] = m.sgn[q];
+// n rows appended to `out`: rows rows[0..n) of m (null: 0..n-1) in that order,
+// their entries in theirs, column j as coff + cmap[j] (null: j). Without m:
+// empty rows, or (unit) rows of one entry 1 at columns coff, coff + 1, ...
+struct RowCopy {
+    const tf_csr* m = nullptr;
+    const int32_t* rows = nullptr;
+    int32_t n = 0;
+    const int32_t* cmap = nullptr;
+    int32_t ncmap = 0;  // columns that cmap covers
+    int32_t coff = 0;
+    CsrBuf* out = nullptr;
+    bool unit = false;
+    int64_t row0 = 0;  // copy_rows: first row in out
+};
+// All copies in one threaded pass each for the row lengths and the entries
+// (a thread costs about as much to start as 10,000 rows to copy). The parts of
+// one `out` follow one another in the order given and agree on which of values
+// and signs they carry. Fills out->v.
+void copy_rows(std::vector<RowCopy> jobs) {
+    constexpr int64_t kPiece = 16384;
+    struct Piece {
+        RowCopy* j;
+        int64_t lo, hi;
+    };
+    std::vector<Piece> pieces;
+    for (RowCopy& j : jobs) {
+        auto& rp = j.out->rp;
+        if (rp.empty()) rp.push_back(0);
+        j.row0 = (int64_t)rp.size() - 1;
+        rp.resize(j.row0 + j.n + 1);
+        for (int64_t lo = 0; lo < j.n; lo += kPiece) pieces.push_back({&j, lo, std::min<int64_t>(j.n, lo + kPiece)});
+    }
+    // pieces a thread takes at a time (a few: no threads)
+    const int64_t np = (int64_t)pieces.size(), per = np <= 4 ? std::max<int64_t>(np, 1) : std::min<int64_t>(4, np / 4);
+    par_chunks(np, per, [&](int64_t p0, int64_t p1) {
+        for (int64_t q = p0; q < p1; ++q) {
+            const RowCopy& j = *pieces[q].j;
+            int64_t* len = j.out->rp.data() + j.row0 + 1;
+            for (int64_t k = pieces[q].lo; k < pieces[q].hi; ++k) {
+                const int64_t r = j.rows ? j.rows[k] : k;
+                len[k] = j.m ? j.m->rowptr[r + 1] - j.m->rowptr[r] : j.unit;
             }
         }
     });
-    o.v = tf_csr{};
-    o.v.nrows = n;
-    o.v.ncols = m.ncols;
-    o.v.nnz = o.rp.back();
-    o.v.rowptr = o.rp.data();
-    o.v.col = o.col.data();
-    o.v.val = m.val ? o.val.data() : nullptr;
-    o.v.sgn = m.sgn ? o.sg.data() : nullptr;
+    for (RowCopy& j : jobs) {
+        auto& rp = j.out->rp;
+        for (int64_t k = 0; k < j.n; ++k) rp[j.row0 + k + 1] += rp[j.row0 + k];
+    }
+    for (RowCopy& j : jobs) {
+        CsrBuf& o = *j.out;
+        o.col.resize(o.rp.back());
+        if (j.m ? j.m->val != nullptr : j.unit) o.val.resize(o.rp.back());
+        if (j.m && j.m->sgn) o.sg.resize(o.rp.back());
+    }
+    std::atomic<bool> bad{false};
+    par_chunks(np, per, [&](int64_t p0, int64_t p1) {
+        for (int64_t q = p0; q < p1; ++q) {
+            const RowCopy& j = *pieces[q].j;
+            const int64_t* rp = j.out->rp.data() + j.row0;
+            int32_t* col = j.out->col.data();
+            double* val = j.out->val.data();
+            int8_t* sg = j.out->sg.data();
+            for (int64_t k = pieces[q].lo; k < pieces[q].hi; ++k) {
+                int64_t w = rp[k];
+                if (!j.m) {
+                    if (j.unit) {
+                        col[w] = j.coff + (int32_t)k;
+                        val[w] = 1.0;
+                    }
+                    continue;
+                }
+                const int64_t r = j.rows ? j.rows[k] : k, b = j.m->rowptr[r], n = rp[k + 1] - w;
+                const int32_t* mc = j.m->col + b;
+                for (int64_t i = 0; i < n; ++i) {
+                    int64_t c = mc[i];
+                    if (j.cmap) {
+                        if (c < 0 || c >= j.ncmap) { bad = true; c = 0; }
+                        c = j.cmap[c];
+                    }
+                    c += j.coff;
+                    if (c > INT32_MAX) bad = true;
+                    col[w + i] = (int32_t)c;
+                }
+                if (j.m->val) std::copy(j.m->val + b, j.m->val + b + n, val + w);
+                if (j.m->sgn) std::copy(j.m->sgn + b, j.m->sgn + b + n, sg + w);
+            }
+        }
+    });
+    if (bad) throw std::runtime_error("operator column out of range");
+    for (RowCopy& j : jobs) {
+        CsrBuf& o = *j.out;
+        o.v = tf_csr{};
+        o.v.nrows = (int32_t)(o.rp.size() - 1);
+        o.v.ncols = j.m ? j.m->ncols : 0;
+        o.v.nnz = o.rp.back();
+        o.v.rowptr = o.rp.data();
+        o.v.col = o.col.data();
+        o.v.val = o.val.empty() ? nullptr : o.val.data();
+        o.v.sgn = o.sg.empty() ? nullptr : o.sg.data();
+    }
+}
+// Rows rows[0..n) of m in that order (entries keep their order), columns
+// relabeled through cmap (of m.ncols entries) when given.
+void select_rows(const tf_csr& m, const int32_t* rows, int32_t n, const int32_t* cmap, int32_t ncmap, CsrBuf& o) {
+    o.rp.clear();
+    o.col.clear();
+    o.val.clear();
+    o.sg.clear();
+    RowCopy j;
+    j.m = &m;
+    j.rows = rows;
+    j.n = n;
+    j.cmap = cmap;
+    j.ncmap = ncmap;
+    j.out = &o;
+    copy_rows({j});
 }
 
 // A tet problem renumbered by its locality ranks (tf_dga_ops.edge_rank,
@@ -682,23 +793,54 @@ bool relabel_tet(const tf_problem* src, TetRelabel& r) {
     const int32_t* ep = r.ep.data();
     const int32_t* fp = r.fp.data();
     if (d.C.nrows != F || d.Ct.nrows != E || d.N.nrows != F) throw std::runtime_error("operator sizes");
-    select_rows(d.C, finv.data(), F, ep, r.C);
-    select_rows(d.Ct, einv.data(), E, fp, r.Ct);
-    select_rows(d.N, finv.data(), F, fp, r.N);
-    auto full = [&](const tf_csr& m, CsrBuf& o) -> tf_csr {
-        if (m.nrows != E) return m;  // absent (0 rows)
-        select_rows(m, einv.data(), E, ep, o);
-        return o.v;
+    std::vector<RowCopy> jobs;
+    auto add = [&](const tf_csr& m, const int32_t* rows, int32_t n, const int32_t* cmap, int32_t ncmap, CsrBuf& o) {
+        RowCopy j;
+        j.m = &m;
+        j.rows = rows;
+        j.n = n;
+        j.cmap = cmap;
+        j.ncmap = ncmap;
+        j.out = &o;
+        jobs.push_back(j);
     };
+    add(d.C, finv.data(), F, ep, E, r.C);
+    add(d.Ct, einv.data(), E, fp, F, r.Ct);
+    add(d.N, finv.data(), F, fp, F, r.N);
+    auto full = [&](const tf_csr& m, CsrBuf& o) {
+        if (m.nrows == E) add(m, einv.data(), E, ep, E, o);  // (absent: 0 rows)
+    };
+    full(d.E, r.E);
+    full(d.RHS1, r.RHS1);
+    full(d.Sig, r.Sig);
+    std::vector<int32_t> hrows;
+    if (d.h_row && d.H.nrows > 0) {
+        hrows.reserve(d.H.nrows);
+        r.h_row.assign(E, -1);
+        for (int32_t e2 = 0; e2 < E; ++e2) {
+            const int32_t h = d.h_row[einv[e2]];
+            if (h < 0) continue;
+            if (h >= d.H.nrows) throw std::runtime_error("h_row out of range");
+            r.h_row[e2] = (int32_t)hrows.size();
+            hrows.push_back(h);
+        }
+        if ((int32_t)hrows.size() != d.H.nrows) throw std::runtime_error("H rows and class-1 edges differ");
+        add(d.H, hrows.data(), d.H.nrows, ep, E, r.H);
+    }
+    copy_rows(std::move(jobs));
     tf_problem& p = r.p;
     p = *src;
     tf_dga_ops& o = p.dga;
     o.C = r.C.v;
     o.Ct = r.Ct.v;
     o.N = r.N.v;
-    o.E = full(d.E, r.E);
-    o.RHS1 = full(d.RHS1, r.RHS1);
-    o.Sig = full(d.Sig, r.Sig);
+    if (d.E.nrows == E) o.E = r.E.v;
+    if (d.RHS1.nrows == E) o.RHS1 = r.RHS1.v;
+    if (d.Sig.nrows == E) o.Sig = r.Sig.v;
+    if (!hrows.empty()) {
+        o.H = r.H.v;
+        o.h_row = r.h_row.data();
+    }
     r.bnd_edge.assign(E, -1);
     r.edge_class.assign(E, 0);
     r.fixed_value.assign(E, 0.0);
@@ -710,22 +852,6 @@ bool relabel_tet(const tf_problem* src, TetRelabel& r) {
     o.bnd_edge = d.bnd_edge ? r.bnd_edge.data() : nullptr;
     o.edge_class = r.edge_class.data();
     o.fixed_value = r.fixed_value.data();
-    if (d.h_row && d.H.nrows > 0) {
-        std::vector<int32_t> hrows;
-        hrows.reserve(d.H.nrows);
-        r.h_row.assign(E, -1);
-        for (int32_t e2 = 0; e2 < E; ++e2) {
-            const int32_t h = d.h_row[einv[e2]];
-            if (h < 0) continue;
-            if (h >= d.H.nrows) throw std::runtime_error("h_row out of range");
-            r.h_row[e2] = (int32_t)hrows.size();
-            hrows.push_back(h);
-        }
-        if ((int32_t)hrows.size() != d.H.nrows) throw std::runtime_error("H rows and class-1 edges differ");
-        select_rows(d.H, hrows.data(), d.H.nrows, ep, r.H);
-        o.H = r.H.v;
-        o.h_row = r.h_row.data();
-    }
     if (d.n_free > 0) {
         r.free_edges.resize(d.n_free);
         for (int32_t k = 0; k < d.n_free; ++k) r.free_edges[k] = ep[d.free_edges[k]];
@@ -1322,7 +1448,7 @@ void create_tet(tf_ctx* c, const tf_problem* p, const std::vector<int32_t>* batc
             c->f_plain = fr.Kf.rowptr[r + 1] - fr.Kf.rowptr[r] <= kLongRow;
         if (c->f_plain) {
             CsrBuf nb;
-            select_rows(fr.Kf, c->h_tf_a.data(), F, nullptr, nb);
+            select_rows(fr.Kf, c->h_tf_a.data(), F, nullptr, 0, nb);
             upload_sell<T>(c->fKf, nb.v, true);
         } else {
             upload_frac_k<T>(c->fKf, c->lf, fr.Kf);
@@ -1353,9 +1479,13 @@ void create_tet(tf_ctx* c, const tf_problem* p, const std::vector<int32_t>* batc
         } else {
             c->h_perm = sigma_order(d.H);
         }
-        CsrBuf hs;
-        select_rows(d.H, c->h_perm.data(), d.H.nrows, nullptr, hs);
-        upload_sell<T>(c->H, hs.v, true);
+        if (c->tet_relabel) {
+            upload_sell<T>(c->H, d.H, true);
+        } else {
+            CsrBuf hs;
+            select_rows(d.H, c->h_perm.data(), d.H.nrows, nullptr, 0, hs);
+            upload_sell<T>(c->H, hs.v, true);
+        }
         std::vector<int32_t> row_edge(d.H.nrows, -1);
         for (int32_t e = 0; e < E; ++e)
             if (d.h_row[e] >= 0) {
@@ -1378,7 +1508,7 @@ void create_tet(tf_ctx* c, const tf_problem* p, const std::vector<int32_t>* batc
         std::vector<int32_t> inv(d.n_free);
         for (int32_t k = 0; k < d.n_free; ++k) inv[perm[k]] = k;
         CsrBuf a;
-        select_rows(d.A, perm.data(), d.n_free, inv.data(), a);
+        select_rows(d.A, perm.data(), d.n_free, inv.data(), d.n_free, a);
         upload_sell<T>(c->A, a.v, true);
         // the CG kernels stream A's (and G's) slices assuming width >= 1:
         // every free row holds its diagonal
@@ -1393,11 +1523,11 @@ void create_tet(tf_ctx* c, const tf_problem* p, const std::vector<int32_t>* batc
             // fem residual: E and SigMat on the free rows (fem_w_kernel)
             c->fem = true;
             CsrBuf m;
-            select_rows(d.E, fe.data(), d.n_free, nullptr, m);
+            select_rows(d.E, fe.data(), d.n_free, nullptr, 0, m);
             upload_sell<T>(c->Kf, m.v, true);
             c->k_dir_only = false;
             if (d.Sig.nnz > 0) {
-                select_rows(d.Sig, fe.data(), d.n_free, nullptr, m);
+                select_rows(d.Sig, fe.data(), d.n_free, nullptr, 0, m);
             } else {
                 m = CsrBuf{};
                 m.rp.assign(d.n_free + 1, 0);
@@ -1409,7 +1539,7 @@ void create_tet(tf_ctx* c, const tf_problem* p, const std::vector<int32_t>* batc
                 m.v.val = m.val.data();
             }
             upload_sell<T>(c->R1f, m.v, true);
-            select_rows(d.Ct, fe.data(), d.n_free, nullptr, m);
+            select_rows(d.Ct, fe.data(), d.n_free, nullptr, 0, m);
             upload_sell<T>(c->Ctf, m.v, false);
             for (DevBuf* b : {&c->U_older, &c->fw, &c->fw2}) zero_field<T>(*b, E, c->stream);
         } else {
@@ -1421,9 +1551,9 @@ void create_tet(tf_ctx* c, const tf_problem* p, const std::vector<int32_t>* batc
             c->k_dir_only = true;
             for (int32_t col : m.col)
                 if (free_col[col]) c->k_dir_only = false;
-            select_rows(d.RHS1, fe.data(), d.n_free, nullptr, m);
+            select_rows(d.RHS1, fe.data(), d.n_free, nullptr, 0, m);
             upload_sell<T>(c->R1f, m.v, true);
-            select_rows(d.Ct, fe.data(), d.n_free, nullptr, m);
+            select_rows(d.Ct, fe.data(), d.n_free, nullptr, 0, m);
             upload_sell<T>(c->Ctf, m.v, false);
         }
         c->n_free = d.n_free;
@@ -3232,8 +3362,236 @@ void write_field(tf_ctx* c, DevBuf& b, const int32_t* pos, int64_t n, const doub
     }
 }
 
-std::unique_ptr<tf_ctx> make_ctx(const tf_problem* p, int32_t prec,
-                                 const std::vector<int32_t>* batch_rows = nullptr) {
+// The stacked problem of a batch: block-diagonal operators, edge, face and row
+// indices of instance k offset by the sizes of instances 0..k-1. Inside its
+// block an instance is in its locality order, as a single simulation is
+// (relabel_tet; rows keep their entries' order, so fields are bitwise those of
+// its own numbering): in that numbering a slice's gathers touch about twelve
+// cache lines instead of four or five. Measured, 16 Kuhn cavities n in
+// [16, 24], FP32 (FP64): dga 46.8 -> 43.3 us a step (68.4 -> 66.6; sell_h 19.2
+// -> 16.4), gfdtd 656 -> 633 (920 -> 890; cg_w 12.3 -> 11.4 a pass). The
+// operators are copied once, straight to their place.
+struct Stack {
+    CsrBuf C, Ct, H, N, E, A, RHS1;
+    std::vector<int32_t> eoff, foff, ecnt, row0;  // row0: first CG row per instance (gfdtd)
+    std::vector<int32_t> ep, fp;      // place of every edge / face of the instances (ranked)
+    std::vector<int32_t> erow, frow;  // instance k's edge (face) at each place of its block
+    std::vector<uint8_t> use;         // instance k is in its locality order
+    bool ranked = false;              // some instance is
+    std::vector<int32_t> h_row, h_sel, bnd_edge, free_edges;
+    std::vector<int8_t> edge_class;
+    std::vector<double> fixed_value, h_dt, f_dt, cg_dt;
+    tf_problem p{};
+};
+
+// Whether rank[0..n) is a permutation.
+bool is_permutation(const int32_t* rank, int32_t n) {
+    std::vector<uint8_t> seen(n, 0);
+    for (int32_t i = 0; i < n; ++i) {
+        if (rank[i] < 0 || rank[i] >= n || seen[rank[i]]) return false;
+        seen[rank[i]] = 1;
+    }
+    return true;
+}
+// Whether an instance of a batch is relabeled by its locality ranks: they are
+// permutations of its own edges and faces, and (dga) each row of H belongs to
+// one edge. Any other keeps its own numbering, which asks nothing of either.
+bool usable_ranks(const tf_problem* p) {
+    const tf_dga_ops& d = p->dga;
+    if (!d.edge_rank || !d.face_rank) return false;
+    if (!is_permutation(d.edge_rank, p->n_edges) || !is_permutation(d.face_rank, p->n_faces)) return false;
+    if (p->method != TF_METHOD_DGA) return true;
+    std::vector<int32_t> rows;
+    for (int32_t e = 0; e < p->n_edges; ++e)
+        if (d.h_row[e] >= 0) rows.push_back(d.h_row[e]);
+    return (int64_t)rows.size() == d.H.nrows && is_permutation(rows.data(), d.H.nrows);
+}
+
+// One operator of instance k to append: `rows` and `cmap` are the instance's
+// order of its rows and the places of its columns (null: its own numbering),
+// both without the instance's offsets; val: it carries values (else signs).
+RowCopy stack_part(const tf_csr& m, const int32_t* rows, const int32_t* cmap, int32_t ncmap, int32_t coff, bool val,
+                   CsrBuf& out) {
+    if (val && !m.val) throw std::runtime_error("operator without values");
+    if (!val && !m.sgn) throw std::runtime_error("incidence without signs");
+    RowCopy j;
+    j.m = &m;
+    j.rows = rows;
+    j.n = m.nrows;
+    j.cmap = cmap;
+    j.ncmap = ncmap;
+    j.coff = coff;
+    j.out = &out;
+    return j;
+}
+
+// Stacks n dga or n gfdtd problems. A gfdtd instance's free edges are padded
+// to a multiple of 64 with solver-only edges appended after its own edges: no
+// face touches them (empty C columns and Ct rows), their rows of A and E are
+// the diagonal 1, so their CG rows stay 0 (no right-hand side) and every
+// 64-row slice of the CG belongs to one instance.
+void stack_problems(const tf_problem* const* probs, int32_t n, Stack& m) {
+    const bool gf = probs[0]->method == TF_METHOD_GFDTD;
+    // sizes and offsets
+    m.eoff.assign(1, 0);
+    m.foff.assign(1, 0);
+    std::vector<int32_t> hoff(1, 0), boff(1, 0), pad(n, 0);
+    int64_t rows = 0, hrows = 0;
+    if (gf) m.row0.assign(1, 0);
+    for (int32_t k = 0; k < n; ++k) {
+        const tf_problem* p = probs[k];
+        if (!p) throw std::runtime_error("null problem in batch");
+        if (gf && p->method != TF_METHOD_GFDTD) throw std::runtime_error("a batch holds one method (dga or gfdtd)");
+        if (!gf && p->method != TF_METHOD_DGA) throw std::runtime_error("batches hold method dga problems");
+        const tf_dga_ops& d = p->dga;
+        if (!gf && d.frac.enabled) throw std::runtime_error("batches hold lossless dga problems only");
+        if (gf && d.Sig.nnz > 0) throw std::runtime_error("gfdtd batches hold lossless problems only");
+        if (!gf && (p->n_edges <= 0 || p->n_faces <= 0)) throw std::runtime_error("empty problem in batch");
+        if (!(p->dt > 0)) throw std::runtime_error("batch instance without a time step");
+        const int32_t E = p->n_edges, F = p->n_faces, nf = d.n_free;
+        if (d.C.nrows != F || d.Ct.nrows != E || d.N.nrows != F ||
+            (gf && (d.A.nrows != nf || d.RHS1.nrows != E || d.E.nrows != E || !d.free_edges)))
+            throw std::runtime_error("inconsistent operators");
+        if (gf) pad[k] = (kSlice - nf % kSlice) % kSlice;
+        const int64_t eo = (int64_t)m.eoff.back() + E + pad[k], fo = (int64_t)m.foff.back() + F;
+        hrows += gf ? 0 : d.H.nrows;
+        rows += gf ? nf + pad[k] : 0;
+        if (eo > INT32_MAX || fo > INT32_MAX || hrows > INT32_MAX) throw std::runtime_error("batch too large");
+        m.ecnt.push_back(E);
+        m.eoff.push_back((int32_t)eo);
+        m.foff.push_back((int32_t)fo);
+        hoff.push_back((int32_t)hrows);
+        boff.push_back(boff.back() + d.n_bnd);
+        if (gf) m.row0.push_back((int32_t)rows);
+    }
+    const int32_t E = m.eoff.back(), F = m.foff.back(), NF = (int32_t)rows;
+    // per edge, face and H row, one instance per task
+    const char* env = std::getenv("TETFIT_TET_ORDER");
+    const bool numbering = env && std::strcmp(env, "numbering") == 0;
+    m.use.assign(n, 0);
+    for (std::vector<int32_t>* v : {&m.ep, &m.erow, &m.bnd_edge}) v->resize(E);
+    for (std::vector<int32_t>* v : {&m.fp, &m.frow}) v->resize(F);
+    if (!gf) m.h_row.resize(E);
+    m.h_sel.resize(hrows);
+    m.edge_class.resize(E);
+    m.fixed_value.resize(E);
+    m.f_dt.resize(F);
+    m.h_dt.resize(hrows);
+    m.cg_dt.resize(NF);
+    m.free_edges.resize(NF);
+    par_chunks(n, 1, [&](int64_t k, int64_t) {
+        const tf_problem* p = probs[k];
+        const tf_dga_ops& d = p->dga;
+        const int32_t eo = m.eoff[k], fo = m.foff[k], En = p->n_edges, Fn = p->n_faces;
+        const bool use = !numbering && usable_ranks(p);
+        m.use[k] = use;
+        for (int32_t e = 0; e < En; ++e) {
+            const int32_t q = use ? d.edge_rank[e] : e;
+            m.ep[eo + e] = eo + q;
+            m.erow[eo + q] = e;
+            m.bnd_edge[eo + q] = d.bnd_edge && d.bnd_edge[e] >= 0 ? d.bnd_edge[e] + boff[k] : -1;
+            m.edge_class[eo + q] = d.edge_class[e];
+            m.fixed_value[eo + q] = d.fixed_value[e];
+        }
+        for (int32_t e = eo + En; e < m.eoff[k + 1]; ++e) {  // solver-only edges
+            m.ep[e] = e;
+            m.bnd_edge[e] = -1;
+            m.edge_class[e] = 1;
+            m.fixed_value[e] = 0;
+        }
+        for (int32_t f = 0; f < Fn; ++f) {
+            const int32_t q = use ? d.face_rank[f] : f;
+            m.fp[fo + f] = fo + q;
+            m.frow[fo + q] = f;
+        }
+        std::fill(m.f_dt.begin() + fo, m.f_dt.begin() + fo + Fn, p->dt);
+        if (gf) {
+            const int32_t ro = m.row0[k];
+            for (int32_t i = 0; i < d.n_free; ++i)
+                m.free_edges[ro + i] = eo + (use ? d.edge_rank[d.free_edges[i]] : d.free_edges[i]);
+            for (int32_t i = d.n_free; i < m.row0[k + 1] - ro; ++i) m.free_edges[ro + i] = eo + En + i - d.n_free;
+            std::fill(m.cg_dt.begin() + ro, m.cg_dt.begin() + m.row0[k + 1], p->dt);
+            return;
+        }
+        // H's rows follow their edges' places
+        int32_t r = hoff[k];
+        for (int32_t q = 0; q < En; ++q) {
+            const int32_t h = d.h_row[use ? m.erow[eo + q] : q];
+            m.h_row[eo + q] = h < 0 ? -1 : use ? r : hoff[k] + h;
+            if (use && h >= 0) m.h_sel[r++] = h;
+        }
+        std::fill(m.h_dt.begin() + hoff[k], m.h_dt.begin() + hoff[k + 1], p->dt);
+    });
+    for (int32_t k = 0; k < n; ++k) m.ranked = m.ranked || m.use[k];
+    // the operators
+    std::vector<RowCopy> jobs;
+    auto tail = [&](CsrBuf& out, int32_t k, bool unit, int32_t coff) {
+        RowCopy j;
+        j.n = pad[k];
+        j.unit = unit;
+        j.coff = coff;
+        j.out = &out;
+        jobs.push_back(j);
+    };
+    for (int32_t k = 0; k < n; ++k) {
+        const tf_dga_ops& d = probs[k]->dga;
+        const bool use = m.use[k];
+        const int32_t eo = m.eoff[k], fo = m.foff[k], En = probs[k]->n_edges, Fn = probs[k]->n_faces;
+        const int32_t* er = use ? m.erow.data() + eo : nullptr;
+        const int32_t* fr = use ? m.frow.data() + fo : nullptr;
+        const int32_t* ec = use ? d.edge_rank : nullptr;
+        const int32_t* fc = use ? d.face_rank : nullptr;
+        jobs.push_back(stack_part(d.C, fr, ec, En, eo, false, m.C));
+        jobs.push_back(stack_part(d.Ct, er, fc, Fn, fo, false, m.Ct));
+        jobs.push_back(stack_part(d.N, fr, fc, Fn, fo, true, m.N));
+        if (!gf) {
+            jobs.push_back(stack_part(d.H, use ? m.h_sel.data() + hoff[k] : nullptr, ec, En, eo, true, m.H));
+            continue;
+        }
+        const int32_t ro = m.row0[k];
+        jobs.push_back(stack_part(d.E, er, ec, En, eo, true, m.E));
+        jobs.push_back(stack_part(d.RHS1, er, ec, En, eo, true, m.RHS1));
+        jobs.push_back(stack_part(d.A, nullptr, nullptr, 0, ro, true, m.A));
+        tail(m.Ct, k, false, 0);
+        tail(m.E, k, true, eo + En);
+        tail(m.RHS1, k, false, 0);
+        tail(m.A, k, true, ro + d.n_free);
+    }
+    copy_rows(std::move(jobs));
+    tf_problem& p = m.p;
+    p.method = probs[0]->method;
+    p.n_edges = E;
+    p.n_faces = F;
+    p.dt = probs[0]->dt;
+    p.duration = probs[0]->duration;
+    for (int32_t k = 0; k < n; ++k) p.n_vols += probs[k]->n_vols;
+    tf_dga_ops& d = p.dga;
+    auto set = [](tf_csr& o, const CsrBuf& b, int32_t ncols) {
+        o = b.v;
+        o.ncols = ncols;
+    };
+    set(d.C, m.C, E);
+    set(d.Ct, m.Ct, F);
+    set(d.N, m.N, F);
+    if (gf) {
+        set(d.E, m.E, E);
+        set(d.RHS1, m.RHS1, E);
+        set(d.A, m.A, NF);
+        d.free_edges = m.free_edges.data();
+        d.n_free = NF;
+    } else {
+        set(d.H, m.H, E);
+        d.h_row = m.h_row.data();
+    }
+    d.bnd_edge = m.bnd_edge.data();
+    d.n_bnd = boff.back();
+    d.edge_class = m.edge_class.data();
+    d.fixed_value = m.fixed_value.data();
+}
+
+// stack: the instances of a batch, p their stacked problem (null: p is a
+// single simulation).
+std::unique_ptr<tf_ctx> make_ctx(const tf_problem* p, int32_t prec, const Stack* stack = nullptr) {
     if (p->method < 0 || p->method > 3) throw std::runtime_error("unknown method");
     if (prec != TF_PREC_FP64 && prec != TF_PREC_FP32) throw std::runtime_error("unknown precision");
     if (p->n_edges <= 0 || p->n_faces <= 0) throw std::runtime_error("empty problem");
@@ -3265,7 +3623,14 @@ std::unique_ptr<tf_ctx> make_ctx(const tf_problem* p, int32_t prec,
     } else {
         TetRelabel rl;
         const tf_problem* q = p;
-        if (relabel_tet(p, rl)) {
+        const std::vector<int32_t>* batch_rows = stack && !stack->row0.empty() ? &stack->row0 : nullptr;
+        if (stack) {
+            c->tet_relabel = stack->ranked;
+            if (stack->ranked) {
+                c->h_esid = stack->ep;
+                c->h_fsid = stack->fp;
+            }
+        } else if (relabel_tet(p, rl)) {
             q = &rl.p;
             c->tet_relabel = true;
             c->h_esid = rl.ep;
@@ -3284,146 +3649,6 @@ std::unique_ptr<tf_ctx> make_ctx(const tf_problem* p, int32_t prec,
     ensure_carr(c.get(), 1, 0);
     TF_HIP(hipStreamSynchronize(c->stream));
     return c;
-}
-
-// Block-diagonal concatenation of n dga problems: edge, face and H-row
-// indices of instance k are offset by the sizes of instances 0..k-1.
-struct MergedDga {
-    std::vector<int64_t> c_ptr, ct_ptr, h_ptr, n_ptr;
-    std::vector<int32_t> c_col, ct_col, h_col, n_col, h_row, bnd_edge;
-    std::vector<int8_t> c_sg, ct_sg, edge_class;
-    std::vector<double> h_val, n_val, fixed_value, h_dt, f_dt;
-    std::vector<int32_t> eoff, foff, erank, frank;
-    bool ranked = false;  // some instance carries locality ranks
-    tf_problem p{};
-};
-
-// Whether rank[0..n) is a permutation.
-bool is_permutation(const int32_t* rank, int32_t n) {
-    std::vector<uint8_t> seen(n, 0);
-    for (int32_t i = 0; i < n; ++i) {
-        if (rank[i] < 0 || rank[i] >= n || seen[rank[i]]) return false;
-        seen[rank[i]] = 1;
-    }
-    return true;
-}
-// Whether an instance of a batch is relabeled by its locality ranks: they are
-// permutations of its own edges and faces, and (dga) each row of H belongs to
-// one edge. Any other keeps its own numbering, which asks nothing of either.
-bool usable_ranks(const tf_problem* p) {
-    const tf_dga_ops& d = p->dga;
-    if (!d.edge_rank || !d.face_rank) return false;
-    if (!is_permutation(d.edge_rank, p->n_edges) || !is_permutation(d.face_rank, p->n_faces)) return false;
-    if (p->method != TF_METHOD_DGA) return true;
-    std::vector<int32_t> rows;
-    for (int32_t e = 0; e < p->n_edges; ++e)
-        if (d.h_row[e] >= 0) rows.push_back(d.h_row[e]);
-    return (int64_t)rows.size() == d.H.nrows && is_permutation(rows.data(), d.H.nrows);
-}
-
-// Appends an instance's locality ranks at its offsets (its own numbering when
-// it carries none to use), extra entries after its edges in place. The merged problem
-// is then relabeled inside each instance's block (relabel_tet), as a single
-// simulation is: in the instances' own numbering a slice's gathers touch about
-// twelve cache lines instead of four or five. Measured, 16 Kuhn cavities
-// n in [16, 24], FP32 (FP64): dga 46.8 -> 43.3 us a step (68.4 -> 66.6; sell_h
-// 19.2 -> 16.4), gfdtd 656 -> 633 (920 -> 890; cg_w 12.3 -> 11.4 a pass).
-void append_ranks(const tf_problem* p, int32_t eo, int32_t extra, int32_t fo, std::vector<int32_t>& er,
-                  std::vector<int32_t>& fr, bool& ranked) {
-    const tf_dga_ops& d = p->dga;
-    const bool have = usable_ranks(p);
-    ranked = ranked || have;
-    for (int32_t e = 0; e < p->n_edges + extra; ++e)
-        er.push_back(eo + (have && e < p->n_edges ? d.edge_rank[e] : e));
-    for (int32_t f = 0; f < p->n_faces; ++f) fr.push_back(fo + (have ? d.face_rank[f] : f));
-}
-
-void append_csr(const tf_csr& m, int32_t col_off, std::vector<int64_t>& ptr, std::vector<int32_t>& col,
-                std::vector<int8_t>* sg, std::vector<double>* val) {
-    if (ptr.empty()) ptr.push_back(0);
-    const int64_t base = ptr.back();
-    for (int32_t r = 0; r < m.nrows; ++r) ptr.push_back(base + m.rowptr[r + 1]);
-    for (int64_t q = 0; q < m.nnz; ++q) {
-        const int64_t c64 = (int64_t)m.col[q] + col_off;
-        if (c64 > INT32_MAX) throw std::runtime_error("batch too large for int32 indices");
-        col.push_back((int32_t)c64);
-    }
-    if (sg) {
-        if (!m.sgn) throw std::runtime_error("incidence without signs");
-        sg->insert(sg->end(), m.sgn, m.sgn + m.nnz);
-    }
-    if (val) {
-        if (!m.val) throw std::runtime_error("operator without values");
-        val->insert(val->end(), m.val, m.val + m.nnz);
-    }
-}
-
-tf_csr csr_view(int32_t nrows, int32_t ncols, const std::vector<int64_t>& ptr, const std::vector<int32_t>& col,
-                const std::vector<int8_t>* sg, const std::vector<double>* val) {
-    tf_csr o{};
-    o.nrows = nrows;
-    o.ncols = ncols;
-    o.nnz = ptr.empty() ? 0 : ptr.back();
-    o.rowptr = ptr.data();
-    o.col = col.data();
-    o.sgn = sg ? sg->data() : nullptr;
-    o.val = val ? val->data() : nullptr;
-    return o;
-}
-
-void merge_dga(const tf_problem* const* probs, int32_t n, MergedDga& m) {
-    m.eoff.assign(1, 0);
-    m.foff.assign(1, 0);
-    int32_t hoff = 0, boff = 0;
-    for (int32_t k = 0; k < n; ++k) {
-        const tf_problem* p = probs[k];
-        if (!p) throw std::runtime_error("null problem in batch");
-        if (p->method != TF_METHOD_DGA) throw std::runtime_error("batches hold method dga problems");
-        if (p->dga.frac.enabled) throw std::runtime_error("batches hold lossless dga problems only");
-        if (p->n_edges <= 0 || p->n_faces <= 0) throw std::runtime_error("empty problem in batch");
-        if (!(p->dt > 0)) throw std::runtime_error("batch instance without a time step");
-        const tf_dga_ops& d = p->dga;
-        const int32_t E = p->n_edges, F = p->n_faces, eo = m.eoff.back(), fo = m.foff.back();
-        if ((int64_t)eo + E > INT32_MAX || (int64_t)fo + F > INT32_MAX) throw std::runtime_error("batch too large");
-        if (d.C.nrows != F || d.Ct.nrows != E || d.N.nrows != F) throw std::runtime_error("inconsistent operators");
-        append_csr(d.C, eo, m.c_ptr, m.c_col, &m.c_sg, nullptr);
-        append_csr(d.Ct, fo, m.ct_ptr, m.ct_col, &m.ct_sg, nullptr);
-        append_csr(d.H, eo, m.h_ptr, m.h_col, nullptr, &m.h_val);
-        append_csr(d.N, fo, m.n_ptr, m.n_col, nullptr, &m.n_val);
-        for (int32_t e = 0; e < E; ++e) {
-            m.h_row.push_back(d.h_row[e] >= 0 ? d.h_row[e] + hoff : -1);
-            m.bnd_edge.push_back(d.bnd_edge && d.bnd_edge[e] >= 0 ? d.bnd_edge[e] + boff : -1);
-            m.edge_class.push_back(d.edge_class[e]);
-            m.fixed_value.push_back(d.fixed_value[e]);
-        }
-        append_ranks(p, eo, 0, fo, m.erank, m.frank, m.ranked);
-        m.h_dt.insert(m.h_dt.end(), (size_t)d.H.nrows, p->dt);
-        m.f_dt.insert(m.f_dt.end(), (size_t)F, p->dt);
-        hoff += d.H.nrows;
-        boff += d.n_bnd;
-        m.eoff.push_back(eo + E);
-        m.foff.push_back(fo + F);
-    }
-    const int32_t E = m.eoff.back(), F = m.foff.back();
-    tf_problem& p = m.p;
-    p.method = TF_METHOD_DGA;
-    p.n_edges = E;
-    p.n_faces = F;
-    p.dt = probs[0]->dt;
-    p.duration = probs[0]->duration;
-    for (int32_t k = 0; k < n; ++k) p.n_vols += probs[k]->n_vols;
-    tf_dga_ops& d = p.dga;
-    d.C = csr_view(F, E, m.c_ptr, m.c_col, &m.c_sg, nullptr);
-    d.Ct = csr_view(E, F, m.ct_ptr, m.ct_col, &m.ct_sg, nullptr);
-    d.H = csr_view(hoff, E, m.h_ptr, m.h_col, nullptr, &m.h_val);
-    d.N = csr_view(F, F, m.n_ptr, m.n_col, nullptr, &m.n_val);
-    d.h_row = m.h_row.data();
-    d.bnd_edge = m.bnd_edge.data();
-    d.n_bnd = boff;
-    d.edge_class = m.edge_class.data();
-    d.fixed_value = m.fixed_value.data();
-    d.edge_rank = m.ranked ? m.erank.data() : nullptr;
-    d.face_rank = m.ranked ? m.frank.data() : nullptr;
 }
 
 // Rebuilds the merged source and probe tables of a batch from its
@@ -3622,106 +3847,6 @@ void autotune(tf_ctx* c) {
     }
 }
 
-// Block-diagonal concatenation of n lossless gfdtd problems for a batched
-// CG (run_gfdtd_batch). Instance k's free edges are padded to a multiple of
-// 64 with solver-only edges appended after its own edges: no face touches
-// them (empty C columns and Ct rows), their rows of A and E are the diagonal
-// 1, so their CG rows stay 0 (no right-hand side) and every 64-row slice of
-// the CG belongs to one instance. row0[k] is instance k's first CG row.
-struct MergedGf {
-    std::vector<int64_t> c_ptr, ct_ptr, n_ptr, e_ptr, a_ptr, r1_ptr;
-    std::vector<int32_t> c_col, ct_col, n_col, e_col, a_col, r1_col, bnd_edge, free_edges;
-    std::vector<int8_t> c_sg, ct_sg, edge_class;
-    std::vector<double> n_val, e_val, a_val, r1_val, fixed_value, f_dt, cg_dt;
-    std::vector<int32_t> eoff, foff, ecnt, row0, erank, frank;
-    bool ranked = false;  // some instance carries locality ranks
-    tf_problem p{};
-};
-
-void merge_gfdtd(const tf_problem* const* probs, int32_t n, MergedGf& m) {
-    m.eoff.assign(1, 0);
-    m.foff.assign(1, 0);
-    m.row0.assign(1, 0);
-    int32_t boff = 0;
-    auto empty_rows = [](std::vector<int64_t>& ptr, int32_t k) {
-        if (ptr.empty()) ptr.push_back(0);
-        for (int32_t r = 0; r < k; ++r) ptr.push_back(ptr.back());
-    };
-    auto unit_rows = [](std::vector<int64_t>& ptr, std::vector<int32_t>& col, std::vector<double>& val,
-                        int32_t first_col, int32_t k) {
-        if (ptr.empty()) ptr.push_back(0);
-        for (int32_t r = 0; r < k; ++r) {
-            col.push_back(first_col + r);
-            val.push_back(1.0);
-            ptr.push_back((int64_t)col.size());
-        }
-    };
-    for (int32_t k = 0; k < n; ++k) {
-        const tf_problem* p = probs[k];
-        if (!p) throw std::runtime_error("null problem in batch");
-        if (p->method != TF_METHOD_GFDTD) throw std::runtime_error("a batch holds one method (dga or gfdtd)");
-        const tf_dga_ops& d = p->dga;
-        if (d.Sig.nnz > 0) throw std::runtime_error("gfdtd batches hold lossless problems only");
-        if (!(p->dt > 0)) throw std::runtime_error("batch instance without a time step");
-        const int32_t E = p->n_edges, F = p->n_faces, nf = d.n_free;
-        if (d.C.nrows != F || d.Ct.nrows != E || d.N.nrows != F || d.A.nrows != nf || d.RHS1.nrows != E ||
-            d.E.nrows != E || !d.free_edges)
-            throw std::runtime_error("inconsistent operators");
-        const int32_t pad = (kSlice - nf % kSlice) % kSlice;
-        const int64_t eo = m.eoff.back(), fo = m.foff.back(), ro = m.row0.back();
-        if (eo + E + pad > INT32_MAX || fo + F > INT32_MAX) throw std::runtime_error("batch too large");
-        append_csr(d.C, (int32_t)eo, m.c_ptr, m.c_col, &m.c_sg, nullptr);
-        append_csr(d.Ct, (int32_t)fo, m.ct_ptr, m.ct_col, &m.ct_sg, nullptr);
-        empty_rows(m.ct_ptr, pad);
-        append_csr(d.N, (int32_t)fo, m.n_ptr, m.n_col, nullptr, &m.n_val);
-        append_csr(d.E, (int32_t)eo, m.e_ptr, m.e_col, nullptr, &m.e_val);
-        unit_rows(m.e_ptr, m.e_col, m.e_val, (int32_t)(eo + E), pad);
-        append_csr(d.RHS1, (int32_t)eo, m.r1_ptr, m.r1_col, nullptr, &m.r1_val);
-        empty_rows(m.r1_ptr, pad);
-        append_csr(d.A, (int32_t)ro, m.a_ptr, m.a_col, nullptr, &m.a_val);
-        unit_rows(m.a_ptr, m.a_col, m.a_val, (int32_t)(ro + nf), pad);
-        for (int32_t i = 0; i < nf; ++i) m.free_edges.push_back((int32_t)(eo + d.free_edges[i]));
-        for (int32_t j = 0; j < pad; ++j) m.free_edges.push_back((int32_t)(eo + E + j));
-        for (int32_t e = 0; e < E + pad; ++e) {
-            const bool own = e < E;
-            m.bnd_edge.push_back(own && d.bnd_edge && d.bnd_edge[e] >= 0 ? d.bnd_edge[e] + boff : -1);
-            m.edge_class.push_back(own ? d.edge_class[e] : (int8_t)1);
-            m.fixed_value.push_back(own ? d.fixed_value[e] : 0.0);
-        }
-        append_ranks(p, (int32_t)eo, pad, (int32_t)fo, m.erank, m.frank, m.ranked);
-        m.f_dt.insert(m.f_dt.end(), (size_t)F, p->dt);
-        m.cg_dt.insert(m.cg_dt.end(), (size_t)(nf + pad), p->dt);
-        boff += d.n_bnd;
-        m.ecnt.push_back(E);
-        m.eoff.push_back((int32_t)(eo + E + pad));
-        m.foff.push_back((int32_t)(fo + F));
-        m.row0.push_back((int32_t)(ro + nf + pad));
-    }
-    const int32_t E = m.eoff.back(), F = m.foff.back(), NF = m.row0.back();
-    tf_problem& p = m.p;
-    p.method = TF_METHOD_GFDTD;
-    p.n_edges = E;
-    p.n_faces = F;
-    p.dt = probs[0]->dt;
-    p.duration = probs[0]->duration;
-    for (int32_t k = 0; k < n; ++k) p.n_vols += probs[k]->n_vols;
-    tf_dga_ops& d = p.dga;
-    d.C = csr_view(F, E, m.c_ptr, m.c_col, &m.c_sg, nullptr);
-    d.Ct = csr_view(E, F, m.ct_ptr, m.ct_col, &m.ct_sg, nullptr);
-    d.N = csr_view(F, F, m.n_ptr, m.n_col, nullptr, &m.n_val);
-    d.E = csr_view(E, E, m.e_ptr, m.e_col, nullptr, &m.e_val);
-    d.A = csr_view(NF, NF, m.a_ptr, m.a_col, nullptr, &m.a_val);
-    d.RHS1 = csr_view(E, E, m.r1_ptr, m.r1_col, nullptr, &m.r1_val);
-    d.free_edges = m.free_edges.data();
-    d.n_free = NF;
-    d.bnd_edge = m.bnd_edge.data();
-    d.n_bnd = boff;
-    d.edge_class = m.edge_class.data();
-    d.edge_rank = m.ranked ? m.erank.data() : nullptr;
-    d.face_rank = m.ranked ? m.frank.data() : nullptr;
-    d.fixed_value = m.fixed_value.data();
-}
-
 // CG workgroup table of a gfdtd batch: each instance's slices in chunks of
 // kBatchChunk (whole instances of up to 4 waves' worth of slices per
 // workgroup), the workgroups of one instance consecutive.
@@ -3912,9 +4037,9 @@ tf_status tf_create_batch(const tf_problem* const* probs, int32_t n, int32_t pre
         if (probs[0]->method == TF_METHOD_GFDTD) {
             // CG-solved instances: block-diagonal system, one Jacobi CG per
             // instance per step (run_gfdtd_batch)
-            MergedGf m;
-            merge_gfdtd(probs, n, m);
-            auto c = make_ctx(&m.p, prec, &m.row0);
+            Stack m;
+            stack_problems(probs, n, m);
+            auto c = make_ctx(&m.p, prec, &m);
             build_batch_table(c.get(), m.row0);
             // per CG row dt: the CG rows permute only inside each instance's
             // block (batch_row_order), so the merged order's values hold
@@ -3936,9 +4061,9 @@ tf_status tf_create_batch(const tf_problem* const* probs, int32_t n, int32_t pre
             *out = c.release();
             return;
         }
-        MergedDga m;
-        merge_dga(probs, n, m);
-        auto c = make_ctx(&m.p, prec);
+        Stack m;
+        stack_problems(probs, n, m);
+        auto c = make_ctx(&m.p, prec, &m);
         // the instances' operators are block-diagonal: banded slice order
         // (measured 2-3% faster on 256 instances of 8^3-32^3)
         for (Sell* s : {&c->sCt, &c->H, &c->N}) s->band = true;
@@ -3946,7 +4071,7 @@ tf_status tf_create_batch(const tf_problem* const* probs, int32_t n, int32_t pre
         bt->n = n;
         bt->eoff = m.eoff;
         bt->foff = m.foff;
-        for (int32_t k = 0; k < n; ++k) bt->ecnt.push_back(m.eoff[k + 1] - m.eoff[k]);
+        bt->ecnt = m.ecnt;
         bt->poff.assign(n + 1, 0);
         bt->src.resize(n);
         bt->terms.resize(n);
