@@ -53,6 +53,7 @@ constexpr int kSpmvCap = 8192;   // blocks of the other SELL kernels
 // lane walks about 0.3 us per batch of 8, so 128 entries cost a lane about as
 // much as the launch itself.
 constexpr int kLongRow = 128;
+constexpr int kSellChunk = 1024;  // slices a host thread fills at a time (upload_sell)
 
 // Carrier of Source::Compute in long double (Source.hpp:316-327); 0 for t<0.
 double carrier_value(const tf_source& s, double t) {
@@ -446,63 +447,43 @@ void upload_csr(Csr32& d, const tf_csr& c, bool values) {
     }
 }
 
+// The rows of a CSR matrix that go into a SELL one: rows[0..n) (null: all of
+// them), those of more than max_len entries as empty rows; windows: whether the
+// four-window column form may be used.
+struct SellRows {
+    const int32_t* rows = nullptr;
+    int32_t n = 0;
+    bool windows = true;
+    int64_t max_len = INT64_MAX;
+};
+
 // CSR -> SELL-64 (slices of 64 rows, column-major inside a slice, rows
-// padded with value 0 on their last column).
-std::vector<int64_t> sell_layout(const tf_csr& c) {
-    const int32_t nslices = (c.nrows + kSlice - 1) / kSlice;
+// padded with value 0 on their last column): where each slice starts.
+std::vector<int64_t> sell_layout(const tf_csr& c, const SellRows& from = SellRows{}) {
+    const int32_t n = from.rows ? from.n : c.nrows;
+    const int32_t nslices = (n + kSlice - 1) / kSlice;
     std::vector<int64_t> sptr(nslices + 1, 0);
     for (int32_t s = 0; s < nslices; ++s) {
         int64_t w = 0;
-        for (int32_t r = s * kSlice; r < std::min(c.nrows, (s + 1) * kSlice); ++r)
-            w = std::max<int64_t>(w, c.rowptr[r + 1] - c.rowptr[r]);
+        for (int32_t i = s * kSlice; i < std::min(n, (s + 1) * kSlice); ++i) {
+            const int32_t r = from.rows ? from.rows[i] : i;
+            const int64_t len = c.rowptr[r + 1] - c.rowptr[r];
+            if (len <= from.max_len) w = std::max(w, len);
+        }
         sptr[s + 1] = sptr[s] + w * kSlice;
     }
     return sptr;
 }
 
-// windows: whether the four-window column form may be used.
 template <class T>
-void upload_sell(Sell& d, const tf_csr& c, bool values, bool windows = true) {
-    d.nrows = c.nrows;
-    d.nnz = c.nnz;
-    d.nslices = (c.nrows + kSlice - 1) / kSlice;
-    const std::vector<int64_t> sptr = sell_layout(c);
+void upload_sell(Sell& d, const tf_csr& c, bool values, const SellRows& from = SellRows{}) {
+    const bool windows = from.windows;
+    d.nrows = from.rows ? from.n : c.nrows;
+    d.nslices = (d.nrows + kSlice - 1) / kSlice;
+    const std::vector<int64_t> sptr = sell_layout(c, from);
     d.entries = sptr[d.nslices];
     d.min_width = d.nslices ? INT64_MAX : 0;
     for (int32_t s = 0; s < d.nslices; ++s) d.min_width = std::min(d.min_width, (sptr[s + 1] - sptr[s]) / kSlice);
-    std::vector<int32_t> col(d.entries, 0);
-    std::vector<T> val(values ? d.entries : 0, (T)0);
-    std::vector<int8_t> sg(values ? 0 : d.entries, 0);
-    par_chunks(d.nslices, 4096, [&](int64_t lo, int64_t hi) {
-      for (int32_t s = (int32_t)lo; s < (int32_t)hi; ++s) {
-        const int64_t w = (sptr[s + 1] - sptr[s]) / kSlice;
-        // rows without entries (and lanes past the last row) pad with a column
-        // the slice already uses, so that padding does not widen its span
-        int32_t slice_col = 0;
-        for (int32_t r = s * kSlice; r < std::min(c.nrows, (s + 1) * kSlice); ++r)
-            if (c.rowptr[r + 1] > c.rowptr[r]) { slice_col = c.col[c.rowptr[r]]; break; }
-        for (int lane = 0; lane < kSlice; ++lane) {
-            const int32_t r = s * kSlice + lane;
-            int64_t b = 0, e = 0;
-            if (r < c.nrows) { b = c.rowptr[r]; e = c.rowptr[r + 1]; }
-            const int32_t padc = e > b ? c.col[e - 1] : slice_col;
-            for (int64_t k = 0; k < w; ++k) {
-                const int64_t o = sptr[s] + k * kSlice + lane;
-                if (b + k < e) {
-                    col[o] = c.col[b + k];
-                    if (values) val[o] = (T)c.val[b + k];
-                    else sg[o] = c.sgn[b + k];
-                } else {
-                    col[o] = padc;
-                }
-            }
-        }
-      }
-    });
-    upload(d.sptr, sptr);
-    upload(d.col, col);
-    if (values) upload(d.val, val);
-    else upload(d.sg, sg);
     // 16-bit column codes: one base per slice when every slice spans at most
     // 65,536 columns, else four windows of 16,384 columns per slice when
     // every slice's columns fit in four, else int32 columns.
@@ -516,29 +497,81 @@ void upload_sell(Sell& d, const tf_csr& c, bool values, bool windows = true) {
     const bool force32 = env_on("TETFIT_SELL_COL32");
     std::vector<int32_t> cb(std::max(d.nslices, 1), 0);
     bool fits = !force32 && !env_on("TETFIT_SELL_WIN");
+    RawVec<int32_t> col(d.entries);
+    RawVec<T> val(values ? d.entries : 0);
+    RawVec<int8_t> sg(values ? 0 : d.entries);
+    RawVec<uint16_t> c16;
+    if (fits) c16.assign(1, 0), c16.resize(std::max<int64_t>(d.entries, 1));
     std::atomic<bool> ok{fits};
-    par_chunks(d.nslices, 4096, [&](int64_t s0, int64_t s1) {
-        for (int64_t s = s0; s < s1 && ok; ++s) {
+    std::atomic<int64_t> nnz{0};
+    par_chunks(d.nslices, kSellChunk, [&](int64_t s0, int64_t s1) {
+        const SellRows f = from;
+        const tf_csr m = c;
+        const int32_t nrows = d.nrows;
+        int64_t kept = 0;
+        for (int64_t s = s0; s < s1; ++s) {
+            const int64_t w = (sptr[s + 1] - sptr[s]) / kSlice;
+            int32_t* const pc = col.data() + sptr[s];
+            T* const pv = values ? val.data() + sptr[s] : nullptr;
+            int8_t* const ps = values ? nullptr : sg.data() + sptr[s];
+            int64_t b[kSlice], n[kSlice];
+            // rows without entries (and lanes past the last row) pad with a column
+            // the slice already uses, so that padding does not widen its span
+            int32_t slice_col = -1;
+            for (int lane = 0; lane < kSlice; ++lane) {
+                const int64_t i = s * kSlice + lane;
+                b[lane] = n[lane] = 0;
+                if (i >= nrows) continue;
+                const int32_t r = f.rows ? f.rows[i] : (int32_t)i;
+                b[lane] = m.rowptr[r];
+                n[lane] = m.rowptr[r + 1] - m.rowptr[r];
+                if (n[lane] > f.max_len) n[lane] = 0;
+                if (n[lane] && slice_col < 0) slice_col = m.col[b[lane]];
+            }
+            slice_col = std::max(slice_col, 0);
             int32_t lo = INT32_MAX, hi = 0;
-            for (int64_t o = sptr[s]; o < sptr[s + 1]; ++o) { lo = std::min(lo, col[o]); hi = std::max(hi, col[o]); }
-            if (sptr[s + 1] == sptr[s]) lo = hi = 0;
-            cb[s] = lo;
+            for (int lane = 0; lane < kSlice; ++lane) {
+                const int32_t* const mc = m.col + b[lane];
+                int64_t k = 0;
+                for (; k < n[lane]; ++k) {
+                    const int32_t j = mc[k];
+                    lo = std::min(lo, j);
+                    hi = std::max(hi, j);
+                    pc[k * kSlice + lane] = j;
+                }
+                const int32_t padc = n[lane] ? mc[n[lane] - 1] : slice_col;
+                for (; k < w; ++k) pc[k * kSlice + lane] = padc;
+                if (pv) {
+                    for (k = 0; k < n[lane]; ++k) pv[k * kSlice + lane] = (T)m.val[b[lane] + k];
+                    for (; k < w; ++k) pv[k * kSlice + lane] = 0;
+                } else {
+                    for (k = 0; k < n[lane]; ++k) ps[k * kSlice + lane] = m.sgn[b[lane] + k];
+                    for (; k < w; ++k) ps[k * kSlice + lane] = 0;
+                }
+                kept += n[lane];
+            }
+            if (!w) continue;
             if ((int64_t)hi - lo > 65535) ok = false;
+            if (!ok) continue;
+            cb[s] = lo;
+            uint16_t* const p16 = c16.data() + sptr[s];
+            for (int64_t o = 0; o < w * kSlice; ++o) p16[o] = (uint16_t)(pc[o] - lo);
         }
+        nnz += kept;
     });
+    d.nnz = nnz;
+    upload(d.sptr, sptr);
+    upload(d.col, col);
+    if (values) upload(d.val, val);
+    else upload(d.sg, sg);
     fits = ok;
-    std::vector<uint16_t> c16;
-    if (fits) {
-        c16.assign(std::max<int64_t>(d.entries, 1), 0);
-        for (int32_t s = 0; s < d.nslices; ++s)
-            for (int64_t o = sptr[s]; o < sptr[s + 1]; ++o) c16[o] = (uint16_t)(col[o] - cb[s]);
-    } else if (!force32 && windows) {
+    if (!fits && !force32 && windows) {
         // windows: greedy over the slice's sorted columns, each window opening
         // at the smallest column not yet covered
         cb.assign(4 * std::max(d.nslices, 1), 0);
         std::vector<uint8_t> nwin(std::max(d.nslices, 1), 0);
         ok = true;
-        par_chunks(d.nslices, 4096, [&](int64_t lo, int64_t hi) {
+        par_chunks(d.nslices, kSellChunk, [&](int64_t lo, int64_t hi) {
             std::vector<int32_t> cs;
             for (int64_t s = lo; s < hi && ok; ++s) {
                 cs.assign(col.begin() + sptr[s], col.begin() + sptr[s + 1]);
@@ -555,9 +588,10 @@ void upload_sell(Sell& d, const tf_csr& c, bool values, bool windows = true) {
         });
         fits = ok;
         if (fits) {
-            c16.assign(std::max<int64_t>(d.entries, 1), 0);
+            c16.assign(1, 0);
+            c16.resize(std::max<int64_t>(d.entries, 1));
             ok = true;
-            par_chunks(d.nslices, 4096, [&](int64_t lo, int64_t hi) {
+            par_chunks(d.nslices, kSellChunk, [&](int64_t lo, int64_t hi) {
                 for (int64_t s = lo; s < hi; ++s)
                     for (int64_t o = sptr[s]; o < sptr[s + 1]; ++o) {
                         // the last opened window whose base is <= the column; the
@@ -652,8 +686,9 @@ struct RowCopy {
     bool unit = false;
     int64_t row0 = 0;  // copy_rows: first row in out
 };
-// All copies in one threaded pass each for the row lengths and the entries
-// (a thread costs about as much to start as 10,000 rows to copy). The parts of
+// All copies in one threaded pass each for the row lengths and the entries,
+// some 32,768 rows to a thread at a time (starting one costs about as much as
+// copying 10,000). The parts of
 // one `out` follow one another in the order given and agree on which of values
 // and signs they carry. Fills out->v.
 void copy_rows(std::vector<RowCopy> jobs) {
@@ -663,15 +698,17 @@ void copy_rows(std::vector<RowCopy> jobs) {
         int64_t lo, hi;
     };
     std::vector<Piece> pieces;
+    int64_t rows = 0;
     for (RowCopy& j : jobs) {
+        rows += j.n;
         auto& rp = j.out->rp;
         if (rp.empty()) rp.push_back(0);
         j.row0 = (int64_t)rp.size() - 1;
         rp.resize(j.row0 + j.n + 1);
         for (int64_t lo = 0; lo < j.n; lo += kPiece) pieces.push_back({&j, lo, std::min<int64_t>(j.n, lo + kPiece)});
     }
-    // pieces a thread takes at a time (a few: no threads)
-    const int64_t np = (int64_t)pieces.size(), per = np <= 4 ? std::max<int64_t>(np, 1) : std::min<int64_t>(4, np / 4);
+    const int64_t np = (int64_t)pieces.size();
+    const int64_t per = std::max<int64_t>(1, rows > 0 ? np * 32768 / rows : 1);
     par_chunks(np, per, [&](int64_t p0, int64_t p1) {
         for (int64_t q = p0; q < p1; ++q) {
             const RowCopy& j = *pieces[q].j;
@@ -1271,37 +1308,54 @@ void residual_operator(const tf_dga_ops& d, double dt, const std::vector<int32_t
     const bool lossy = d.Sig.nnz > 0;
     if (lossy && (d.Sig.nrows != d.E.nrows || d.Sig.nnz != d.E.nnz))
         throw std::runtime_error("SigMat must have E's pattern");
-    o.rp.assign(1, 0);
-    o.col.clear();
-    o.val.clear();
-    o.sg.clear();
-    std::vector<std::pair<int32_t, double>> arow;
-    std::vector<uint8_t> used;
-    for (size_t k = 0; k < fe.size(); ++k) {
-        const int32_t e = fe[k], a = perm[k];
-        arow.clear();
-        for (int64_t q = d.A.rowptr[a]; q < d.A.rowptr[a + 1]; ++q)
-            arow.push_back({d.free_edges[d.A.col[q]], d.A.val[q]});
-        used.assign(arow.size(), 0);
-        for (int64_t q = d.E.rowptr[e]; q < d.E.rowptr[e + 1]; ++q) {
-            double v = lossy ? d.E.val[q] - (0.5 * dt) * d.Sig.val[q] : d.E.val[q];
-            for (size_t t = 0; t < arow.size(); ++t)
-                if (!used[t] && arow[t].first == d.E.col[q]) {
-                    v -= arow[t].second;
-                    used[t] = 1;
-                    break;
+    // the rows of each chunk, then one after another
+    constexpr int64_t kRows = 16384;
+    struct Part {
+        std::vector<int64_t> len;
+        std::vector<int32_t> col;
+        std::vector<double> val;
+    };
+    const int64_t n = (int64_t)fe.size();
+    std::vector<Part> parts((n + kRows - 1) / kRows);
+    par_chunks(n, kRows, [&](int64_t lo, int64_t hi) {
+        Part& p = parts[lo / kRows];
+        std::vector<std::pair<int32_t, double>> arow;
+        std::vector<uint8_t> used;
+        for (int64_t k = lo; k < hi; ++k) {
+            const int32_t e = fe[k], a = perm[k];
+            const size_t before = p.col.size();
+            arow.clear();
+            for (int64_t q = d.A.rowptr[a]; q < d.A.rowptr[a + 1]; ++q)
+                arow.push_back({d.free_edges[d.A.col[q]], d.A.val[q]});
+            used.assign(arow.size(), 0);
+            for (int64_t q = d.E.rowptr[e]; q < d.E.rowptr[e + 1]; ++q) {
+                double v = lossy ? d.E.val[q] - (0.5 * dt) * d.Sig.val[q] : d.E.val[q];
+                for (size_t t = 0; t < arow.size(); ++t)
+                    if (!used[t] && arow[t].first == d.E.col[q]) {
+                        v -= arow[t].second;
+                        used[t] = 1;
+                        break;
+                    }
+                if (v != 0) {
+                    p.col.push_back(d.E.col[q]);
+                    p.val.push_back(v);
                 }
-            if (v != 0) {
-                o.col.push_back(d.E.col[q]);
-                o.val.push_back(v);
             }
+            for (size_t t = 0; t < arow.size(); ++t)
+                if (!used[t] && arow[t].second != 0) {
+                    p.col.push_back(arow[t].first);
+                    p.val.push_back(-arow[t].second);
+                }
+            p.len.push_back((int64_t)(p.col.size() - before));
         }
-        for (size_t t = 0; t < arow.size(); ++t)
-            if (!used[t] && arow[t].second != 0) {
-                o.col.push_back(arow[t].first);
-                o.val.push_back(-arow[t].second);
-            }
-        o.rp.push_back((int64_t)o.col.size());
+    });
+    o = CsrBuf{};
+    o.rp.assign(1, 0);
+    o.rp.reserve(n + 1);
+    for (const Part& p : parts) {
+        for (int64_t len : p.len) o.rp.push_back(o.rp.back() + len);
+        o.col.insert(o.col.end(), p.col.begin(), p.col.end());
+        o.val.insert(o.val.end(), p.val.begin(), p.val.end());
     }
     o.v = tf_csr{};
     o.v.nrows = (int32_t)fe.size();
@@ -1318,36 +1372,24 @@ template <class T>
 void upload_frac_k(Sell& d, tf_ctx::Long& l, const tf_csr& k) {
     std::vector<int32_t> row, ptr(1, 0), col;
     std::vector<T> val;
-    CsrBuf o;
-    o.rp.assign(1, 0);
-    o.rp.reserve((size_t)k.nrows + 1);
-    o.col.reserve(k.nnz);
-    o.val.reserve(k.nnz);
     for (int32_t r = 0; r < k.nrows; ++r) {
         const int64_t b = k.rowptr[r], e = k.rowptr[r + 1];
-        if (e - b > kLongRow) {
-            if ((int64_t)col.size() + (e - b) > INT32_MAX) throw std::runtime_error("fractional operator too large");
-            row.push_back(r);
-            col.insert(col.end(), k.col + b, k.col + e);
-            for (int64_t q = b; q < e; ++q) val.push_back((T)k.val[q]);
-            ptr.push_back((int32_t)col.size());
-        } else {
-            o.col.insert(o.col.end(), k.col + b, k.col + e);
-            o.val.insert(o.val.end(), k.val + b, k.val + e);
-        }
-        o.rp.push_back((int64_t)o.col.size());
+        if (e - b <= kLongRow) continue;
+        if ((int64_t)col.size() + (e - b) > INT32_MAX) throw std::runtime_error("fractional operator too large");
+        row.push_back(r);
+        col.insert(col.end(), k.col + b, k.col + e);
+        for (int64_t q = b; q < e; ++q) val.push_back((T)k.val[q]);
+        ptr.push_back((int32_t)col.size());
     }
-    o.v = k;
-    o.v.nnz = o.rp.back();
-    o.v.rowptr = o.rp.data();
-    o.v.col = o.col.data();
-    o.v.val = o.val.data();
     // windowed columns bring the wide-mesh kernels with their non-temporal
     // loads, which only an operator beyond the 256 MB Infinity Cache gains
     // from (24^3, 27 MB: sell_frac 15.5 us windowed, 14.3 us with int32 columns)
     const bool big = k.nnz * (int64_t)(sizeof(T) + 4) > ((int64_t)256 << 20);
     const char* win = std::getenv("TETFIT_SELL_WIN");
-    upload_sell<T>(d, o.v, true, big || (win && *win && std::strcmp(win, "0") != 0));
+    SellRows from;
+    from.windows = big || (win && *win && std::strcmp(win, "0") != 0);
+    from.max_len = kLongRow;
+    upload_sell<T>(d, k, true, from);
     l.n = (int32_t)row.size();
     if (!l.n) return;
     std::vector<uint64_t> mask(std::max(d.nslices, 1), 0);
@@ -1447,9 +1489,7 @@ void create_tet(tf_ctx* c, const tf_problem* p, const std::vector<int32_t>* batc
         for (int32_t r = 0; r < fr.Kf.nrows && c->f_plain; ++r)
             c->f_plain = fr.Kf.rowptr[r + 1] - fr.Kf.rowptr[r] <= kLongRow;
         if (c->f_plain) {
-            CsrBuf nb;
-            select_rows(fr.Kf, c->h_tf_a.data(), F, nullptr, 0, nb);
-            upload_sell<T>(c->fKf, nb.v, true);
+            upload_sell<T>(c->fKf, fr.Kf, true, SellRows{c->h_tf_a.data(), F});
         } else {
             upload_frac_k<T>(c->fKf, c->lf, fr.Kf);
             upload_sell<T>(c->fRf, fr.Rf, true);
@@ -1479,13 +1519,7 @@ void create_tet(tf_ctx* c, const tf_problem* p, const std::vector<int32_t>* batc
         } else {
             c->h_perm = sigma_order(d.H);
         }
-        if (c->tet_relabel) {
-            upload_sell<T>(c->H, d.H, true);
-        } else {
-            CsrBuf hs;
-            select_rows(d.H, c->h_perm.data(), d.H.nrows, nullptr, 0, hs);
-            upload_sell<T>(c->H, hs.v, true);
-        }
+        upload_sell<T>(c->H, d.H, true, SellRows{c->h_perm.data(), d.H.nrows});
         std::vector<int32_t> row_edge(d.H.nrows, -1);
         for (int32_t e = 0; e < E; ++e)
             if (d.h_row[e] >= 0) {
@@ -1513,34 +1547,26 @@ void create_tet(tf_ctx* c, const tf_problem* p, const std::vector<int32_t>* batc
         // the CG kernels stream A's (and G's) slices assuming width >= 1:
         // every free row holds its diagonal
         if (c->A.nslices > 0 && c->A.min_width < 1) throw std::runtime_error("A has a 64-row slice without entries");
-        c->hA_ptr = a.rp;
-        c->hA_col = a.col;
-        c->hA_val = a.val;
         c->hA_sptr = sell_layout(a.v);
         std::vector<int32_t> fe(d.n_free);
         for (int32_t k = 0; k < d.n_free; ++k) fe[k] = d.free_edges[perm[k]];
         if (p->method == TF_METHOD_FEM) {
             // fem residual: E and SigMat on the free rows (fem_w_kernel)
             c->fem = true;
-            CsrBuf m;
-            select_rows(d.E, fe.data(), d.n_free, nullptr, 0, m);
-            upload_sell<T>(c->Kf, m.v, true);
+            const SellRows rows{fe.data(), d.n_free};
+            upload_sell<T>(c->Kf, d.E, true, rows);
             c->k_dir_only = false;
             if (d.Sig.nnz > 0) {
-                select_rows(d.Sig, fe.data(), d.n_free, nullptr, 0, m);
+                upload_sell<T>(c->R1f, d.Sig, true, rows);
             } else {
-                m = CsrBuf{};
-                m.rp.assign(d.n_free + 1, 0);
-                m.v = tf_csr{};
-                m.v.nrows = d.n_free;
-                m.v.ncols = E;
-                m.v.rowptr = m.rp.data();
-                m.v.col = m.col.data();
-                m.v.val = m.val.data();
+                const std::vector<int64_t> rp(d.n_free + 1, 0);
+                tf_csr none{};
+                none.nrows = d.n_free;
+                none.ncols = E;
+                none.rowptr = rp.data();
+                upload_sell<T>(c->R1f, none, true);
             }
-            upload_sell<T>(c->R1f, m.v, true);
-            select_rows(d.Ct, fe.data(), d.n_free, nullptr, 0, m);
-            upload_sell<T>(c->Ctf, m.v, false);
+            upload_sell<T>(c->Ctf, d.Ct, false, rows);
             for (DevBuf* b : {&c->U_older, &c->fw, &c->fw2}) zero_field<T>(*b, E, c->stream);
         } else {
             CsrBuf m;
@@ -1551,10 +1577,9 @@ void create_tet(tf_ctx* c, const tf_problem* p, const std::vector<int32_t>* batc
             c->k_dir_only = true;
             for (int32_t col : m.col)
                 if (free_col[col]) c->k_dir_only = false;
-            select_rows(d.RHS1, fe.data(), d.n_free, nullptr, 0, m);
-            upload_sell<T>(c->R1f, m.v, true);
-            select_rows(d.Ct, fe.data(), d.n_free, nullptr, 0, m);
-            upload_sell<T>(c->Ctf, m.v, false);
+            const SellRows rows{fe.data(), d.n_free};
+            upload_sell<T>(c->R1f, d.RHS1, true, rows);
+            upload_sell<T>(c->Ctf, d.Ct, false, rows);
         }
         c->n_free = d.n_free;
         upload(c->free_edge, fe);
@@ -1579,6 +1604,9 @@ void create_tet(tf_ctx* c, const tf_problem* p, const std::vector<int32_t>* batc
             for (int64_t q = a.rp[i]; q < a.rp[i + 1]; ++q)
                 if (a.col[q] == i && a.val[q] != 0) pre[i] = (T)(1.0 / a.val[q]);
         upload(c->pre, pre);
+        c->hA_ptr = std::move(a.rp);
+        c->hA_col = std::move(a.col);
+        c->hA_val = std::move(a.val);
         const int64_t n = std::max<int32_t>(d.n_free, 1);
         for (DevBuf* b : {&c->x, &c->r, &c->z, &c->p0, &c->p1, &c->q, &c->r0}) zero_field<T>(*b, n, c->stream);
         for (DevBuf* b : {&c->rs0, &c->rs1}) zero_field<RS<T>>(*b, n, c->stream);
@@ -3465,7 +3493,7 @@ void stack_problems(const tf_problem* const* probs, int32_t n, Stack& m) {
         if (gf) m.row0.push_back((int32_t)rows);
     }
     const int32_t E = m.eoff.back(), F = m.foff.back(), NF = (int32_t)rows;
-    // per edge, face and H row, one instance per task
+    // per edge, face and H row
     const char* env = std::getenv("TETFIT_TET_ORDER");
     const bool numbering = env && std::strcmp(env, "numbering") == 0;
     m.use.assign(n, 0);
@@ -3479,7 +3507,7 @@ void stack_problems(const tf_problem* const* probs, int32_t n, Stack& m) {
     m.h_dt.resize(hrows);
     m.cg_dt.resize(NF);
     m.free_edges.resize(NF);
-    par_chunks(n, 1, [&](int64_t k, int64_t) {
+    auto place = [&](int64_t k) {
         const tf_problem* p = probs[k];
         const tf_dga_ops& d = p->dga;
         const int32_t eo = m.eoff[k], fo = m.foff[k], En = p->n_edges, Fn = p->n_faces;
@@ -3521,6 +3549,10 @@ void stack_problems(const tf_problem* const* probs, int32_t n, Stack& m) {
             if (use && h >= 0) m.h_sel[r++] = h;
         }
         std::fill(m.h_dt.begin() + hoff[k], m.h_dt.begin() + hoff[k + 1], p->dt);
+    };
+    const int64_t per = std::max<int64_t>(1, n * (int64_t)65536 / ((int64_t)E + F + 1));
+    par_chunks(n, per, [&](int64_t k0, int64_t k1) {
+        for (int64_t k = k0; k < k1; ++k) place(k);
     });
     for (int32_t k = 0; k < n; ++k) m.ranked = m.ranked || m.use[k];
     // the operators
