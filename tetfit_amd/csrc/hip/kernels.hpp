@@ -217,6 +217,17 @@ __host__ __device__ inline void fit_edge_slots(const FitGrid g, uint32_t s, int3
         f[0] = xf(i, j - 1, k); f[1] = xf(i, j, k); f[2] = yf(i - 1, j, k); f[3] = yf(i, j, k);
     }
 }
+// Whether the edge at position s has all four slots (it is off the boundary
+// planes across its direction).
+inline bool fit_edge_interior(const FitGrid g, uint32_t s) {
+    const uint32_t nx = g.nx, ny = g.ny, nz = g.nz;
+    const uint32_t nEx = nx * (ny + 1) * (nz + 1), nEy = (nx + 1) * ny * (nz + 1);
+    auto mid = [](uint32_t i, uint32_t n) { return i > 0 && i < n; };
+    if (s < nEx) return mid(s / nx % (ny + 1), ny) && mid(s / nx / (ny + 1), nz);
+    if (s < nEx + nEy) return mid((s - nEx) % (nx + 1), nx) && mid((s - nEx) / (nx + 1) / ny, nz);
+    const uint32_t r = s - nEx - nEy;
+    return mid(r % (nx + 1), nx) && mid(r / (nx + 1) % (ny + 1), ny);
+}
 __host__ __device__ inline void fit_face_slots(const FitGrid g, uint32_t s, int32_t e[4]) {
     const uint32_t nx = g.nx, ny = g.ny, nz = g.nz;
     const uint32_t nEx = nx * (ny + 1) * (nz + 1), nEy = (nx + 1) * ny * (nz + 1);

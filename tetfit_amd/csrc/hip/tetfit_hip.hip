@@ -1068,6 +1068,8 @@ bool fit_grid_positions(tf_ctx* c, const tf_fit_ops& f, std::vector<uint8_t>& eo
     for (int64_t q = 0; q < f.n_common; ++q) {
         const int32_t e = f.common_edges[q];
         if (f.ct_ptr[e + 1] - f.ct_ptr[e] != 4) return false;
+        // (the wrapped slots of a boundary edge can be other faces' positions)
+        if (!fit_edge_interior(g, (uint32_t)esid[e])) return false;
         int32_t slot[4];
         fit_edge_slots(g, (uint32_t)esid[e], slot);
         for (int k = 0; k < 4; ++k)
