@@ -466,6 +466,16 @@ struct FitPal {
 };
 constexpr int kPalMax = 512;
 
+// How a grid-order kernel finds an item's constants. kFitPal: palette;
+// kFitPlain: plain arrays; kFitPlainNt: plain arrays loaded non-temporally
+// (fit_non_temporal).
+enum FitMode { kFitPal, kFitPlain, kFitPlainNt };
+template <FitMode M, typename T>
+__device__ __forceinline__ T fit_coef(const T* p) {
+    if constexpr (M == kFitPlainNt) return __builtin_nontemporal_load(p);
+    else return *p;
+}
+
 // id[at[i]] = val[i] (faces that become probed or stop to be)
 __global__ void __launch_bounds__(kBlock) set_ids_kernel(int32_t n, const int32_t* __restrict__ at,
                                                          const uint16_t* __restrict__ val, uint16_t* __restrict__ id) {
@@ -488,13 +498,9 @@ __global__ void __launch_bounds__(kBlock) fit_src_kernel(FitSpecial sp, const do
 // goes to LDS meanwhile, and source values are prepared a step ahead. Larger
 // grids are bound by bytes: an fp64 item moves 26 (E) and 26 (H) with palettes,
 // against 42 and 50 with plain coefficients and B stored every step.
-// Plain coefficients are loaded non-temporally: read once a step, they would
-// push the fields out of the 256 MB Infinity Cache.
 // One step (both kernels, in a graph): 64^3 fp64 12.1 us, fp32 9.8 us; 161^3
-// random media fp64 141 us (E 87 us, H 55 us; 163 us with ordinary coefficient
-// loads, which cost H its cached fields). With codes read before the
-// neighbours, five-load source chains and one item per thread: 15.4, 12.0 and
-// 185 us.
+// random media fp64 137 us. With codes read before the neighbours, five-load
+// source chains and one item per thread: 15.4, 12.0 and 185 us.
 template <typename T>
 struct FitStep {
     FitGrid g;
@@ -516,9 +522,9 @@ struct FitStep {
 };
 
 // Palette into LDS (before the loads that follow are waited for).
-template <typename T, bool P>
+template <typename T, FitMode M>
 __device__ __forceinline__ void fit_pal_load(const FitStep<T>& a, FitPal<T>* __restrict__ lds) {
-    if constexpr (P)
+    if constexpr (M == kFitPal)
         for (int t = (int)threadIdx.x; t < a.n_pal; t += kBlock) lds[t] = a.pal[t];
 }
 
@@ -528,10 +534,10 @@ __device__ __forceinline__ void fit_pal_load(const FitStep<T>& a, FitPal<T>* __r
 // faces in the order 0, 2, 3, 1 of fit_edge_slots with signs +, -, +, - and the
 // direction's sign (checked when the context is created). Special items take
 // their source value from spv.
-template <typename T, bool P, int N>
+template <typename T, FitMode M, int N>
 __global__ void __launch_bounds__(kBlock) fit_e_grid_kernel(FitStep<T> a, const T* __restrict__ Fv, T* __restrict__ U,
                                                             const T* __restrict__ B) {
-    __shared__ FitPal<T> pal[P ? kPalMax : 1];
+    __shared__ FitPal<T> pal[M == kFitPal ? kPalMax : 1];
     __shared__ double red[kBlock / kWave];
     const int hb = (int)blockIdx.x;
     if (hb < a.sp_blocks) {
@@ -563,7 +569,7 @@ __global__ void __launch_bounds__(kBlock) fit_e_grid_kernel(FitStep<T> a, const 
     const uint32_t n = dir == 0 ? cnt[0] : dir == 1 ? cnt[1] : cnt[2];
     const uint32_t base = dir == 0 ? 0 : dir == 1 ? cnt[0] : cnt[0] + cnt[1];
     const double sg = a.sg[dir];
-    fit_pal_load<T, P>(a, pal);
+    fit_pal_load<T, M>(a, pal);
     uint32_t id[N];
     T u[N], v0[N], v1[N], v2[N], v3[N];
     FitPal<T> q[N];
@@ -604,13 +610,13 @@ __global__ void __launch_bounds__(kBlock) fit_e_grid_kernel(FitStep<T> a, const 
         v1[m] = Fv[in ? f1 : 0];
         v2[m] = Fv[in ? f2 : 0];
         v3[m] = Fv[in ? f3 : 0];
-        if constexpr (!P) q[m] = FitPal<T>{__builtin_nontemporal_load(a.c0 + s), __builtin_nontemporal_load(a.c1 + s)};
+        if constexpr (M != kFitPal) q[m] = FitPal<T>{fit_coef<M>(a.c0 + s), fit_coef<M>(a.c1 + s)};
     }
-    if constexpr (P) __syncthreads();
+    if constexpr (M == kFitPal) __syncthreads();
 #pragma unroll
     for (int m = 0; m < N; ++m) {
         const uint32_t r = first + m * kBlock + threadIdx.x;
-        if constexpr (P) q[m] = pal[id[m]];
+        if constexpr (M == kFitPal) q[m] = pal[id[m]];
         const double c = sg * ((((double)v0[m] - (double)v2[m]) + (double)v3[m]) - (double)v1[m]);
         if (r < n && id[m]) U[base + r] = (T)fit_e_new((double)q[m].c0, (double)u[m], (double)q[m].c1, c);
     }
@@ -623,10 +629,10 @@ __global__ void __launch_bounds__(kBlock) fit_e_grid_kernel(FitStep<T> a, const 
 // and on every face with store_b (the run's last step, energy samples). The
 // first workgroups take the U components of this step's sample and the next
 // step's source values.
-template <typename T, bool P, int N>
+template <typename T, FitMode M, int N>
 __global__ void __launch_bounds__(kBlock) fit_h_grid_kernel(FitStep<T> a, int store_b, const T* __restrict__ U,
                                                             T* __restrict__ Fv, T* __restrict__ B) {
-    __shared__ FitPal<T> pal[P ? kPalMax : 1];
+    __shared__ FitPal<T> pal[M == kFitPal ? kPalMax : 1];
     const int hb = (int)blockIdx.x;
     if (hb < a.src_blocks) {
         const int32_t i = hb * kBlock + threadIdx.x;
@@ -647,7 +653,7 @@ __global__ void __launch_bounds__(kBlock) fit_h_grid_kernel(FitStep<T> a, int st
     const uint32_t n = dir == 0 ? cnt[0] : dir == 1 ? cnt[1] : cnt[2];
     const uint32_t base = dir == 0 ? 0 : dir == 1 ? cnt[0] : cnt[0] + cnt[1];
     const double sg = a.sg[dir];
-    fit_pal_load<T, P>(a, pal);
+    fit_pal_load<T, M>(a, pal);
     uint32_t id[N];
     T fo[N], v0[N], v1[N], v2[N], v3[N];
     FitPal<T> q[N];
@@ -683,13 +689,13 @@ __global__ void __launch_bounds__(kBlock) fit_h_grid_kernel(FitStep<T> a, int st
         v1[m] = U[e1];
         v2[m] = U[e2];
         v3[m] = U[e3];
-        if constexpr (!P) q[m] = FitPal<T>{__builtin_nontemporal_load(a.c0 + s), __builtin_nontemporal_load(a.c1 + s)};
+        if constexpr (M != kFitPal) q[m] = FitPal<T>{fit_coef<M>(a.c0 + s), fit_coef<M>(a.c1 + s)};
     }
-    if constexpr (P) __syncthreads();
+    if constexpr (M == kFitPal) __syncthreads();
 #pragma unroll
     for (int m = 0; m < N; ++m) {
         const uint32_t r = first + m * kBlock + threadIdx.x;
-        if constexpr (P) q[m] = pal[id[m] >= a.flag ? id[m] - a.flag : id[m]];
+        if constexpr (M == kFitPal) q[m] = pal[id[m] >= a.flag ? id[m] - a.flag : id[m]];
         const double c = (((double)v0[m] - (double)v2[m]) + (double)v3[m]) - (double)v1[m];
         const double b = fit_b_new((double)q[m].c0, (double)fo[m], sg * c);
         if (r < n && id[m]) {

@@ -2043,9 +2043,49 @@ void fit_indexed_step(tf_ctx* c, const FitSpecial& sp, int sp_blocks, const doub
 // 4 bytes and the grid is large: 128^3 fp32 33.1 against 35.3 us, 161^3 fp64
 // 168 against 163, 48^3 fp32 8.7 against 8.3. Below about 17^3 the step is one
 // workgroup's latency: 16^3 fp64 6.6 us with one item, 6.7 with two.
+// $TETFIT_FIT_ITEMS (1, 2 or 4) overrides, to exercise each on small grids.
 template <class T>
 int fit_items(int64_t edges) {
+    if (const char* v = std::getenv("TETFIT_FIT_ITEMS")) {
+        const int n = std::atoi(v);
+        if (n == 1 || n == 2 || (n == 4 && sizeof(T) == 4)) return n;
+    }
     return edges < (1 << 16) ? 1 : sizeof(T) == 4 && edges >= (1 << 22) ? 4 : 2;
+}
+
+// Whether plain coefficients, read once a step, are loaded non-temporally:
+// when a step's arrays exceed the 256 MB Infinity Cache they would push the
+// fields out of it; below, they stay there themselves. Random media, a step
+// ordinary / non-temporal (E side plain, H palette): fp64 64^3 13.4 / 15.0 us,
+// 128^3 (226 MB) 67 / 72, 136^3 (272 MB) 92 / 84, 161^3 165 / 137; fp32 161^3
+// (242 MB) 71 / 76.
+// $TETFIT_FIT_NT (0 or 1) overrides, to exercise both on small grids.
+bool fit_non_temporal(const tf_ctx* c) {
+    if (const char* v = std::getenv("TETFIT_FIT_NT"))
+        if (*v) return std::strcmp(v, "0") != 0;
+    size_t b = c->U.bytes + c->Fv.bytes;
+    for (const DevBuf* d : {&c->fe_id, &c->fh_id, &c->fe_ca, &c->fe_cb, &c->fh_cm, &c->fh_cn}) b += d->bytes;
+    return b > (size_t)256 << 20;
+}
+// The kernels of one mode for `per` items per thread (4: fp32 only).
+template <class T>
+using FitEKernel = void (*)(FitStep<T>, const T*, T*, const T*);
+template <class T>
+using FitHKernel = void (*)(FitStep<T>, int, const T*, T*, T*);
+template <class T, FitMode M>
+std::pair<FitEKernel<T>, FitHKernel<T>> fit_kernels(int per) {
+    if constexpr (sizeof(T) == 4)
+        if (per == 4) return {fit_e_grid_kernel<T, M, 4>, fit_h_grid_kernel<T, M, 4>};
+    if (per == 1) return {fit_e_grid_kernel<T, M, 1>, fit_h_grid_kernel<T, M, 1>};
+    return {fit_e_grid_kernel<T, M, 2>, fit_h_grid_kernel<T, M, 2>};
+}
+template <class T>
+std::pair<FitEKernel<T>, FitHKernel<T>> fit_kernels(FitMode m, int per) {
+    switch (m) {
+        case kFitPal: return fit_kernels<T, kFitPal>(per);
+        case kFitPlainNt: return fit_kernels<T, kFitPlainNt>(per);
+        default: return fit_kernels<T, kFitPlain>(per);
+    }
 }
 
 template <class T>
@@ -2106,12 +2146,9 @@ void run_fit(tf_ctx* c, int64_t first, int64_t n, tf_stats* st) {
         const int per = fit_items<T>(c->E);
         const int e_grid = sp_blocks + e.probe_blocks + slab_grid(ecnt, per * kBlock);
         const int h_grid = sp_blocks + h.probe_blocks + slab_grid(fcnt, per * kBlock);
-        const auto ek = per == 1 ? (c->fe_pal.p ? fit_e_grid_kernel<T, true, 1> : fit_e_grid_kernel<T, false, 1>)
-                      : per == 2 ? (c->fe_pal.p ? fit_e_grid_kernel<T, true, 2> : fit_e_grid_kernel<T, false, 2>)
-                                 : (c->fe_pal.p ? fit_e_grid_kernel<T, true, 4> : fit_e_grid_kernel<T, false, 4>);
-        const auto hk = per == 1 ? (c->fh_pal.p ? fit_h_grid_kernel<T, true, 1> : fit_h_grid_kernel<T, false, 1>)
-                      : per == 2 ? (c->fh_pal.p ? fit_h_grid_kernel<T, true, 2> : fit_h_grid_kernel<T, false, 2>)
-                                 : (c->fh_pal.p ? fit_h_grid_kernel<T, true, 4> : fit_h_grid_kernel<T, false, 4>);
+        const FitMode plain = fit_non_temporal(c) ? kFitPlainNt : kFitPlain;
+        const auto ek = fit_kernels<T>(c->fe_pal.p ? kFitPal : plain, per).first;
+        const auto hk = fit_kernels<T>(c->fh_pal.p ? kFitPal : plain, per).second;
         // slot: row of the step before (its B is sampled by the E phase)
         auto step = [&](const double* cs, double* poy, const int64_t* slot, bool store_b) {
             e.poy_part = poy;
