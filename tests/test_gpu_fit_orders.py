@@ -80,3 +80,50 @@ def test_common_edge_on_the_boundary(workdir, monkeypatch, prec):
     assert not indexed and not np.array_equal(ref[0][e], state[0][e])
     for x, y in zip(got, ref):
         np.testing.assert_array_equal(x, y)
+
+
+def reordered(b, rng):
+    """The same updates in other words: for a third of the common edges and of
+    the faces the four entries are rotated by one and the sign turned round, for
+    another third the first and third entry change places (both '+')."""
+    o = b.fit_ops()
+    face, curl, dual = o["ct_face"].copy(), o["curl"].copy(), o["dual_curl"].copy()
+    edges = o["c_edge"].copy()
+
+    def change(rows, get, put, sign):
+        for r, how in zip(rows, rng.integers(0, 3, len(rows))):
+            q = get(r)
+            if how == 1:
+                put(r, np.roll(q, 1))
+                sign[r] *= -1
+            elif how == 2:
+                put(r, q[[2, 1, 0, 3]])
+
+    def put_face(e, q):
+        face[o["ct_ptr"][e]:o["ct_ptr"][e] + 4] = q
+
+    def put_edge(f, q):
+        edges[f] = q
+
+    change(o["common_edges"], lambda e: face[o["ct_ptr"][e]:o["ct_ptr"][e] + 4].copy(), put_face, dual)
+    change(o["tbc_faces"], lambda f: edges[f].copy(), put_edge, curl)
+    return Altered(b, ct_face=face, dual_curl=dual, c_edge=edges.reshape(-1), curl=curl)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("media", ["uniform", "random"])
+def test_entities_in_another_order(workdir, monkeypatch, media, prec):
+    """Orders and signs of their own keep the grid layout (a code per item),
+    with probes and sources; bitwise the index tables, which sum in the same
+    order."""
+    rng = np.random.default_rng(6)
+    if media == "uniform":
+        b = reordered(small_cavity(workdir), rng)
+    else:
+        b = reordered(Model(configs.fit_random_media(str(workdir), n=12, n_steps=400, n_probes=4, name="ord12")).build(1),
+                      rng)
+    state = [rng.standard_normal(m) for m in (b.n_edges, b.n_faces, b.n_faces)]
+    (grid, got), (indexed, ref) = both_layouts(b, monkeypatch, prec, state)
+    assert grid and not indexed
+    for x, y in zip(got, ref):
+        np.testing.assert_array_equal(x, y)

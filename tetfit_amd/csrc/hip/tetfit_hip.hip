@@ -246,6 +246,7 @@ struct tf_ctx {
     std::vector<uint16_t> h_fe_id, h_fh_id;
     int32_t fe_n = 0, fh_flag = 0;
     double fit_es[3] = {1, 1, 1}, fit_fs[3] = {1, 1, 1};
+    bool fit_coded = false;  // grid order with a code per entity (kFitCoded)
     int sg_probe_blocks = 0;
     std::vector<int32_t> fh_probed;  // device faces whose id carries fh_flag
     std::vector<double> h_ca_common, h_cb_common;
@@ -1027,12 +1028,12 @@ void ev_flush(tf_ctx* c) {
 
 // Grid order for a FIT problem that carries grid positions: used when every
 // common edge and tbc face has exactly its slots' entities (fit_edge_slots /
-// fit_face_slots) in the order 0, 2, 3, 1 and one sign per direction, as the
-// mesher numbers them (D:4643-5080). eon / fon: 1 for the entities at each
-// position that the main pass updates. False (the index-table layout is used)
-// otherwise, or if $TETFIT_FIT_INDEXED is set to a non-empty value other than
-// 0.
-bool fit_grid_positions(tf_ctx* c, const tf_fit_ops& f, std::vector<uint8_t>& eon, std::vector<uint8_t>& fon) {
+// fit_face_slots). False (the index-table layout is used) otherwise, or if
+// $TETFIT_FIT_INDEXED is set to a non-empty value other than 0. ecode / fcode:
+// per position the order and signs of its sum (kFitCoded; 0: not in the main
+// pass). All of them in the order 0, 2, 3, 1 with one sign per direction, as
+// the mesher numbers them (D:4643-5080), leave fit_coded unset.
+bool fit_grid_positions(tf_ctx* c, const tf_fit_ops& f, std::vector<uint16_t>& ecode, std::vector<uint16_t>& fcode) {
     const char* forced = std::getenv("TETFIT_FIT_INDEXED");
     if (forced && *forced && std::strcmp(forced, "0") != 0) return false;
     if (!f.edge_sid || !f.face_sid) return false;
@@ -1054,42 +1055,76 @@ bool fit_grid_positions(tf_ctx* c, const tf_fit_ops& f, std::vector<uint8_t>& eo
         for (int32_t v : esid) { if (v < 0 || v >= E || seen_e[v]) return false; seen_e[v] = 1; }
         for (int32_t v : fsid) { if (v < 0 || v >= F || seen_f[v]) return false; seen_f[v] = 1; }
     }
-    const int order[4] = {0, 2, 3, 1};
     // sign of each direction's sums: that of its first entity
     double es[3] = {0, 0, 0}, fs[3] = {0, 0, 0};
     const int64_t eoff[2] = {nx * (ny + 1) * (nz + 1), nx * (ny + 1) * (nz + 1) + (nx + 1) * ny * (nz + 1)};
     const int64_t foff[2] = {(nx + 1) * ny * nz, (nx + 1) * ny * nz + nx * (ny + 1) * nz};
-    auto same_sign = [](double& have, int d) {
-        if (d != 1 && d != -1) return false;
-        if (have == 0) have = d;
-        return have == d;
+    auto edge_dir = [&](int32_t e) { return (esid[e] >= eoff[0]) + (esid[e] >= eoff[1]); };
+    auto face_dir = [&](int32_t q) { return (fsid[q] >= foff[0]) + (fsid[q] >= foff[1]); };
+    for (int64_t q = 0; q < f.n_common && !(es[0] && es[1] && es[2]); ++q) {
+        double& s = es[edge_dir(f.common_edges[q])];
+        if (s == 0) s = f.dual_curl[f.common_edges[q]];
+    }
+    for (int64_t q = 0; q < f.n_tbc && !(fs[0] && fs[1] && fs[2]); ++q) {
+        double& s = fs[face_dir(f.tbc_faces[q])];
+        if (s == 0) s = f.curl[f.tbc_faces[q]];
+    }
+    std::atomic<bool> bad{false}, coded{false};
+    constexpr uint32_t kMesher = 0 | 2 << 2 | 3 << 4 | 1 << 6;
+    const int plus[4] = {1, -1, 1, -1}, minus[4] = {-1, 1, -1, 1};
+    const uint16_t mesher[2] = {(uint16_t)(kMesher << 8 | code4(minus)), (uint16_t)(kMesher << 8 | code4(plus))};
+    // the code of an entity whose sum runs over the positions `ref` with signs
+    // d, -d, d, -d; 0: they are not its slots
+    auto code_of = [&](const int32_t slot[4], const int64_t ref[4], int d, double dir_sign) -> uint16_t {
+        if (ref[0] == slot[0] && ref[1] == slot[2] && ref[2] == slot[3] && ref[3] == slot[1] && dir_sign == d &&
+            (d == 1 || d == -1))
+            return mesher[d > 0];
+        coded = true;
+        uint32_t m = 0;
+        for (int q = 0; q < 4; ++q) {
+            int hit = -1;
+            for (int k = 0; k < 4; ++k)
+                if (slot[k] == ref[q]) {
+                    if (hit >= 0) return 0;
+                    hit = k;
+                }
+            if (hit < 0) return 0;
+            m |= (uint32_t)hit << (2 * q);
+        }
+        const int sg[4] = {d, -d, d, -d};
+        return (uint16_t)(m << 8 | code4(sg));  // (m is never 0: a permutation)
     };
-    eon.assign(E, 0);
-    for (int64_t q = 0; q < f.n_common; ++q) {
-        const int32_t e = f.common_edges[q];
-        if (f.ct_ptr[e + 1] - f.ct_ptr[e] != 4) return false;
-        // (the wrapped slots of a boundary edge can be other faces' positions)
-        if (!fit_edge_interior(g, (uint32_t)esid[e])) return false;
-        int32_t slot[4];
-        fit_edge_slots(g, (uint32_t)esid[e], slot);
-        for (int k = 0; k < 4; ++k)
-            if (fsid[f.ct_face[f.ct_ptr[e] + k]] != slot[order[k]]) return false;
-        if (!same_sign(es[(esid[e] >= eoff[0]) + (esid[e] >= eoff[1])], f.dual_curl[e])) return false;
-        eon[esid[e]] = 1;
-    }
-    fon.assign(F, 0);
-    for (int64_t q = 0; q < f.n_tbc; ++q) {
-        const int32_t fi = f.tbc_faces[q];
-        int32_t slot[4];
-        fit_face_slots(g, (uint32_t)fsid[fi], slot);
-        for (int k = 0; k < 4; ++k)
-            if (esid[f.c_edge[4 * (int64_t)fi + k]] != slot[order[k]]) return false;
-        if (!same_sign(fs[(fsid[fi] >= foff[0]) + (fsid[fi] >= foff[1])], f.curl[fi])) return false;
-        fon[fsid[fi]] = 1;
-    }
+    ecode.assign(E, 0);
+    par_chunks(f.n_common, 65536, [&](int64_t lo, int64_t hi) {
+        for (int64_t q = lo; q < hi && !bad; ++q) {
+            const int32_t e = f.common_edges[q];
+            int32_t slot[4];
+            int64_t ref[4];
+            // (the wrapped slots of a boundary edge can be other faces' positions)
+            if (f.ct_ptr[e + 1] - f.ct_ptr[e] != 4 || !fit_edge_slots(g, (uint32_t)esid[e], slot)) {
+                bad = true;
+                return;
+            }
+            for (int k = 0; k < 4; ++k) ref[k] = fsid[f.ct_face[f.ct_ptr[e] + k]];
+            if (!(ecode[esid[e]] = code_of(slot, ref, f.dual_curl[e], es[edge_dir(e)]))) bad = true;
+        }
+    });
+    fcode.assign(F, 0);
+    par_chunks(f.n_tbc, 65536, [&](int64_t lo, int64_t hi) {
+        for (int64_t q = lo; q < hi && !bad; ++q) {
+            const int32_t fi = f.tbc_faces[q];
+            int32_t slot[4];
+            int64_t ref[4];
+            fit_face_slots(g, (uint32_t)fsid[fi], slot);
+            for (int k = 0; k < 4; ++k) ref[k] = esid[f.c_edge[4 * (int64_t)fi + k]];
+            if (!(fcode[fsid[fi]] = code_of(slot, ref, f.curl[fi], fs[face_dir(fi)]))) bad = true;
+        }
+    });
+    if (bad) return false;
+    c->fit_coded = coded;
     for (int k = 0; k < 3; ++k) {
-        c->fit_es[k] = es[k];
-        c->fit_fs[k] = fs[k];
+        c->fit_es[k] = c->fit_coded ? 1 : es[k];
+        c->fit_fs[k] = c->fit_coded ? 1 : fs[k];
     }
     c->grid = g;
     c->h_esid = std::move(esid);
@@ -1101,7 +1136,7 @@ bool fit_grid_positions(tf_ctx* c, const tf_fit_ops& f, std::vector<uint8_t>& eo
 // values): id per entity, 0 where on is 0. When there are more than kPalMax
 // the ids are 1 and pal stays empty (plain arrays).
 template <class T>
-void fit_palette(const std::vector<uint8_t>& on, const std::vector<T>& a, const std::vector<T>& b,
+void fit_palette(const std::vector<uint16_t>& on, const std::vector<T>& a, const std::vector<T>& b,
                  std::vector<uint16_t>& id, std::vector<FitPal<T>>& pal) {
     struct Key {
         T a, b;
@@ -1133,7 +1168,7 @@ void fit_palette(const std::vector<uint8_t>& on, const std::vector<T>& a, const 
             if (it == seen.end()) {
                 if (pal.size() >= (size_t)kPalMax) {
                     pal.clear();
-                    for (size_t q = 0; q < on.size(); ++q) id[q] = on[q];
+                            for (size_t q = 0; q < on.size(); ++q) id[q] = on[q] ? 1 : 0;
                     return;
                 }
                 it = seen.emplace(k, (uint16_t)pal.size()).first;
@@ -1148,7 +1183,7 @@ void fit_palette(const std::vector<uint8_t>& on, const std::vector<T>& a, const 
 
 // Marks the faces that the probes read as stored every step (FIT grid order).
 void fit_probe_faces(tf_ctx* c, const std::vector<int32_t>& faces) {
-    if (!c->fh_id.p) return;
+    if (!c->fh_id.p || c->fit_coded) return;
     std::vector<int32_t> at;
     std::vector<uint16_t> val;
     for (int32_t f : c->fh_probed) {
@@ -1183,8 +1218,8 @@ template <class T>
 void create_fit(tf_ctx* c, const tf_problem* p) {
     const tf_fit_ops& f = p->fit;
     const int32_t E = c->E, F = c->F;
-    std::vector<uint8_t> eon, fon;
-    c->fit_grid = fit_grid_positions(c, f, eon, fon);
+    std::vector<uint16_t> ecode, fcode;
+    c->fit_grid = fit_grid_positions(c, f, ecode, fcode);
     // per-entity arrays in device order
     auto by_edge = [&](auto v) {
         if (!c->fit_grid) return v;
@@ -1229,7 +1264,8 @@ void create_fit(tf_ctx* c, const tf_problem* p) {
     if (c->fit_grid) {
         const std::vector<T> a = by_edge(ca), b = by_edge(cb);
         std::vector<FitPal<T>> pal;
-        fit_palette(eon, a, b, c->h_fe_id, pal);
+        if (c->fit_coded) c->h_fe_id = ecode;
+        else fit_palette(ecode, a, b, c->h_fe_id, pal);
         c->fe_n = (int32_t)pal.size();
         if (!pal.empty()) {
             upload(c->fe_pal, pal);
@@ -1280,8 +1316,9 @@ void create_fit(tf_ctx* c, const tf_problem* p) {
     if (c->fit_grid) {
         const std::vector<T> a = by_face(cm), b = by_face(cn);
         std::vector<FitPal<T>> pal;
-        fit_palette(fon, a, b, c->h_fh_id, pal);
-        c->fh_flag = pal.empty() ? 2 : (int32_t)pal.size();
+        if (c->fit_coded) c->h_fh_id = fcode;
+        else fit_palette(fcode, a, b, c->h_fh_id, pal);
+        c->fh_flag = pal.empty() ? 2 : (int32_t)pal.size();  // (not used when fit_coded)
         if (!pal.empty()) {
             upload(c->fh_pal, pal);
         } else {
@@ -2052,18 +2089,17 @@ int fit_items(int64_t edges) {
     }
     return edges < (1 << 16) ? 1 : sizeof(T) == 4 && edges >= (1 << 22) ? 4 : 2;
 }
-
 // Whether plain coefficients, read once a step, are loaded non-temporally:
 // when a step's arrays exceed the 256 MB Infinity Cache they would push the
 // fields out of it; below, they stay there themselves. Random media, a step
 // ordinary / non-temporal (E side plain, H palette): fp64 64^3 13.4 / 15.0 us,
 // 128^3 (226 MB) 67 / 72, 136^3 (272 MB) 92 / 84, 161^3 165 / 137; fp32 161^3
-// (242 MB) 71 / 76.
+// (242 MB) 71 / 76. Coded: fp64 112^3 (253 MB) 62 / 67, 120^3 (311 MB) 83 / 80.
 // $TETFIT_FIT_NT (0 or 1) overrides, to exercise both on small grids.
 bool fit_non_temporal(const tf_ctx* c) {
     if (const char* v = std::getenv("TETFIT_FIT_NT"))
         if (*v) return std::strcmp(v, "0") != 0;
-    size_t b = c->U.bytes + c->Fv.bytes;
+    size_t b = c->U.bytes + c->Fv.bytes + (c->fit_coded ? c->B.bytes : 0);
     for (const DevBuf* d : {&c->fe_id, &c->fh_id, &c->fe_ca, &c->fe_cb, &c->fh_cm, &c->fh_cn}) b += d->bytes;
     return b > (size_t)256 << 20;
 }
@@ -2084,6 +2120,8 @@ std::pair<FitEKernel<T>, FitHKernel<T>> fit_kernels(FitMode m, int per) {
     switch (m) {
         case kFitPal: return fit_kernels<T, kFitPal>(per);
         case kFitPlainNt: return fit_kernels<T, kFitPlainNt>(per);
+        case kFitCoded: return fit_kernels<T, kFitCoded>(per);
+        case kFitCodedNt: return fit_kernels<T, kFitCodedNt>(per);
         default: return fit_kernels<T, kFitPlain>(per);
     }
 }
@@ -2146,7 +2184,8 @@ void run_fit(tf_ctx* c, int64_t first, int64_t n, tf_stats* st) {
         const int per = fit_items<T>(c->E);
         const int e_grid = sp_blocks + e.probe_blocks + slab_grid(ecnt, per * kBlock);
         const int h_grid = sp_blocks + h.probe_blocks + slab_grid(fcnt, per * kBlock);
-        const FitMode plain = fit_non_temporal(c) ? kFitPlainNt : kFitPlain;
+        const bool nt = fit_non_temporal(c);
+        const FitMode plain = c->fit_coded ? (nt ? kFitCodedNt : kFitCoded) : nt ? kFitPlainNt : kFitPlain;
         const auto ek = fit_kernels<T>(c->fe_pal.p ? kFitPal : plain, per).first;
         const auto hk = fit_kernels<T>(c->fh_pal.p ? kFitPal : plain, per).second;
         // slot: row of the step before (its B is sampled by the E phase)
