@@ -812,6 +812,8 @@ __device__ __forceinline__ CgRow<T> cg_row_next(const CgRow<T>& q, double alpha,
     return o;
 }
 constexpr int kOneMax = 1024;  // partials per array (workgroups of a solve) at most
+// Rows fit 4 MB, so 1024 workgroups hold every slice with one per wave.
+static_assert(kOneMax * (kBlock / kWave) * kSlice >= (4 << 20) / (int)(4 * sizeof(float)), "cg_one: a slice per wave");
 
 template <typename T, int NB>
 __global__ void __launch_bounds__(kBlock) cg_one_kernel(int32_t it, SellView<T> m, const CgRow<T>* __restrict__ q,
@@ -835,7 +837,7 @@ __global__ void __launch_bounds__(kBlock) cg_one_kernel(int32_t it, SellView<T> 
     const double rr0 = st->rr0, tol = st->tol, gam_prev = st->gam[(it - 1) & 1], alpha_prev = st->alpha[(it - 1) & 1];
     const int32_t maxiter = st->maxiter, given = st->rr0_given;
     const int lane = lane_id();
-    SliceRange sr = block_slices(m.nslices, m.band);
+    const SliceRange sr = block_slices(m.nslices, 0);
     T v[NB];
     CgRow<T> g[NB], own;
     T pown = 0, xown = 0;
@@ -893,7 +895,7 @@ __global__ void __launch_bounds__(kBlock) cg_one_kernel(int32_t it, SellView<T> 
         }
     }
     double ru = 0, wu = 0, rr = 0;
-    for (; sr.s < sr.end; sr.s += sr.step) {
+    if (sr.s < sr.end) {  // this wave's slice
         T acc = 0;
         for (int k0 = 0;;) {
 #pragma unroll
@@ -907,19 +909,15 @@ __global__ void __launch_bounds__(kBlock) cg_one_kernel(int32_t it, SellView<T> 
             load(sr.s, k0);
         }
         const int32_t i = sr.s * kSlice + lane;
-        const CgRow<T> o = own;
-        const T po = pown, xo = xown;
-        const int sn = sr.s + sr.step;
-        if (sn < sr.end) load(sn, 0);
         if (i < m.nrows) {
             T ui;
-            CgRow<T> n = cg_row_next(o, alpha, beta, it, ui);
+            CgRow<T> n = cg_row_next(own, alpha, beta, it, ui);
             if (it >= 0) {
                 // p and x of pass it (u_it = pre r_it)
-                const T uo = (T)((double)o.pre * (double)o.r);
-                const T pi = it == 0 ? uo : (T)__builtin_fma(beta, (double)po, (double)uo);
+                const T uo = (T)((double)own.pre * (double)own.r);
+                const T pi = it == 0 ? uo : (T)__builtin_fma(beta, (double)pown, (double)uo);
                 p[i] = pi;
-                x[i] = (T)__builtin_fma(alpha, (double)pi, (double)xo);
+                x[i] = (T)__builtin_fma(alpha, (double)pi, (double)xown);
             } else {
                 n.s = 0;
             }
