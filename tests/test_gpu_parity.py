@@ -243,7 +243,9 @@ def test_column_layouts_parity(workdir, method, layout, monkeypatch):
     codes over four column windows per slice (the layouts for meshes whose
     slices span more than 65,536 columns), gives the same fp64 parity; so do
     the wide-mesh kernels (non-temporal operator loads) on one-base 16-bit
-    columns, the combination of a large mesh numbered compactly."""
+    columns, the combination of a large mesh numbered compactly. gfdtd in the
+    two-kernel CG passes of large meshes."""
+    monkeypatch.setenv("TETFIT_CG_ONE", "0")
     env = {"col32": "TETFIT_SELL_COL32", "win": "TETFIT_SELL_WIN", "wide": "TETFIT_SELL_WIDE"}[layout]
     monkeypatch.setenv(env, "1")
     b = Model(configs.kuhn_cavity(str(workdir), n=5, method=method, n_steps=60, n_probes=4, block=2,
@@ -324,6 +326,7 @@ def test_slice_stream_bitwise(workdir, prec, precond, monkeypatch):
     gfdtd run (Jacobi fp64, learned fp32) gives bitwise equal fields and
     iteration counts either way."""
     from tetfit_amd.device import Simulation
+    monkeypatch.setenv("TETFIT_CG_ONE", "0")
     b = Model(configs.kuhn_cavity(str(workdir), n=10, method="gfdtd", n_steps=60, n_probes=4, block=2, seed=5,
                                   eps_range=(1.0, 80.0), log_eps=True, name="stream_bw")).build(1)
     out = {}
@@ -333,6 +336,7 @@ def test_slice_stream_bitwise(workdir, prec, precond, monkeypatch):
         monkeypatch.setenv(env, "1")
         print(f"case: slice stream {prec} {precond} {layout} E={b.n_edges}", flush=True)
         sim = Simulation(b, prec)
+        sim.set_profiling(True)
         info = sim.sell_info("a")
         assert info["col_bases"] == (4 if layout == "win" else 1)
         if precond == "learned":
@@ -341,6 +345,7 @@ def test_slice_stream_bitwise(workdir, prec, precond, monkeypatch):
             assert st["pc_state"] == 2
         else:
             st = sim.run()
+        assert ("cg_w_kernel" if precond == "jacobi" else "cg_pg_kernel") in sim.kernel_times()
         out[layout] = (st["cg_iters_total"],) + sim.state()
         sim.close()
     assert out["win"][0] == out["wide"][0]

@@ -14,16 +14,17 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("prec", ["fp64", "fp32"])
 @pytest.mark.parametrize("case", ["grid", "indexed", "relabeled", "numbering"])
 def test_state_round_trip(workdir, monkeypatch, case, prec):
-    """A grid large enough for the touched-page path (4 MB a field in fp64) and
-    a tet mesh, in both of their layouts."""
+    """A grid whose fields take the staging buffer's 2^20 values and a part of
+    them once more, and a tet mesh, in both of their layouts."""
     if case in ("grid", "indexed"):
         monkeypatch.setenv("TETFIT_FIT_INDEXED", "1" if case == "indexed" else "0")
-        b = Model(configs.fit_cavity(str(workdir), n=57, step=0.1, n_steps=4, n_probes=1, name="io_fit")).build(1)
+        b = Model(configs.fit_cavity(str(workdir), n=72, step=0.1, n_steps=4, n_probes=1, name="io_fit")).build(1)
     else:
         if case == "numbering":
             monkeypatch.setenv("TETFIT_TET_ORDER", "numbering")
         b = Model(configs.kuhn_cavity(str(workdir), n=5, method="dga", n_steps=4, n_probes=1, block=2,
                                       name="io_dga")).build(1)
+    assert case not in ("grid", "indexed") or (1 << 20) < min(b.n_edges, b.n_faces) < (2 << 20)
     rng = np.random.default_rng(3)
     put = [rng.standard_normal(k) for k in (b.n_edges, b.n_faces, b.n_faces)]
     sim = Simulation(b, prec, output=False)

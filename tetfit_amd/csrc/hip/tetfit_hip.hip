@@ -1678,15 +1678,25 @@ void create_tet(tf_ctx* c, const tf_problem* p, const std::vector<int32_t>* batc
     c->wide = c->wide || streamed > ((size_t)256 << 20);
     // $TETFIT_SELL_WIDE (non-empty, not 0) selects the wide-mesh kernels on
     // any mesh, to exercise them with one-base columns on small meshes
+    bool forced = false;
     if (const char* v = std::getenv("TETFIT_SELL_WIDE"))
-        if (*v && std::strcmp(v, "0") != 0) c->wide = c->wide_cg = true;
+        if (*v && std::strcmp(v, "0") != 0) c->wide = c->wide_cg = forced = true;
     // Resident share of an operator that is read over and over: next to the
     // vectors the passes use (kept by their ordinary loads) about 215 MB of the
     // Infinity Cache hold. A cyclic read of more than fits would keep none of
     // it (64^3 fp64 gfdtd, A 206 MB beside 102 MB of vectors: cg_w 71 us all
     // non-temporal, 73 us all cached, 60 us with half cached and the step 2.95 ->
     // 2.72 ms; dga 56^3 fp64 152 -> 144 us, 72^3 fp32 204 -> 198 us a step).
+    // $TETFIT_SELL_KEEP (0 to 8) sets the share; meshes forced into the
+    // wide-mesh kernels, whose operators would fit whole, keep none otherwise.
+    int fixed = forced ? 0 : -1;
+    if (const char* v = std::getenv("TETFIT_SELL_KEEP"))
+        if (*v) fixed = std::max(0, std::min(8, std::atoi(v)));
     auto share = [&](Sell& m, size_t& used) {
+        if (fixed >= 0) {
+            m.keep = fixed;
+            return;
+        }
         const size_t budget = (size_t)215 << 20, nb = bytes(m);
         if (!nb || used >= budget) return;
         m.keep = (int32_t)std::min<size_t>(8, 8 * (budget - used) / nb);
@@ -2576,8 +2586,11 @@ void cg_capture(tf_ctx* c, const CgSolve& cs, const CgView<T>& v, int k) {
 // Whether the Jacobi solves of a context run one launch per pass
 // (cg_one_kernel): its rows fit an XCD's 4 MB L2 (fp64 up to about 25^3 Kuhn
 // meshes, fp32 up to about 32^3; the kernel's comment has both sides).
+// $TETFIT_CG_ONE=0 keeps the two kernels, to exercise them on small meshes.
 template <class T>
 bool one_launch_passes(const tf_ctx* c) {
+    const char* v = std::getenv("TETFIT_CG_ONE");
+    if (v && std::strcmp(v, "0") == 0) return false;
     return c->n_free > 0 && (size_t)c->n_free * sizeof(CgRow<T>) <= ((size_t)4 << 20);
 }
 // Buffers of cg_one_kernel (partials: three arrays per pass parity).
@@ -2611,6 +2624,7 @@ void cg_passes(tf_ctx* c, CgSolve& cs, int n) {
     const int stop = std::min(cs.it + n, cs.init.maxiter + 1);
     if (cs.one) {
         const int nb = even_blocks(c->A, kOneMax);
+        if (c->A.nslices > nb * (kBlock / kWave)) throw std::logic_error("cg_one: a slice per wave");
         for (int it = cs.it == 0 ? -1 : cs.it; it < stop; ++it) {
             cg_one_launch<T>(c, it, nb, dst);
             tag(it, 0);
