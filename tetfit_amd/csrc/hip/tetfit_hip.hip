@@ -15,6 +15,7 @@
 #include <cstdlib>
 #include <cmath>
 #include <cstring>
+#include <exception>
 #include <future>
 #include <map>
 #include <memory>
@@ -361,6 +362,11 @@ struct tf_ctx {
     // sampling inside the steps (plan_samples): sample slot per step of the
     // run (row 0: the step before it) and what the kernels write to
     DevBuf slots, samp_ref;
+    struct Planned {
+        int64_t n;    // samples and the next output time once step k is planned
+        double next;
+    };
+    std::vector<Planned> planned;
     double next_print = 0, period = 0;
     bool out_enabled = false;
     bool initial_done = false;
@@ -2026,9 +2032,11 @@ int64_t run_graph_chunks(tf_ctx* c, int64_t first_k, int64_t m, int per_step, bo
 template <class Index>
 bool plan_samples(tf_ctx* c, int64_t n, Index index) {
     std::vector<int64_t> slot((size_t)n + 1, -1);
+    c->planned.resize(n);
     for (int64_t k = 0; k < n; ++k) {
         const std::pair<int64_t, double> it = index(k);
         if (want_sample(c, it.first, it.second)) slot[k + 1] = sample_reserve(c, it.second);
+        c->planned[k] = {c->n_samples, c->next_print};
     }
     if (c->n_probes == 0 || !(c->batch ? c->batch->every > 0 : c->out_enabled)) return false;
     const SampleRef ref{c->probes.as<ProbeDev>(), c->samples.as<double>(), c->n_probes};
@@ -2039,6 +2047,20 @@ bool plan_samples(tf_ctx* c, int64_t n, Index index) {
     TF_HIP(hipStreamSynchronize(c->stream));
     return true;
 }
+// Takes back the planned samples of the steps after `k` when a run ends with an
+// exception (a preconditioner that cannot be built, after some of its steps).
+struct PlanGuard {
+    tf_ctx* c;
+    bool on;
+    int64_t k = 0;
+    int before = std::uncaught_exceptions();
+    ~PlanGuard() {
+        if (!on || std::uncaught_exceptions() <= before || k >= (int64_t)c->planned.size()) return;
+        c->n_samples = c->planned[k].n;
+        c->next_print = c->planned[k].next;
+        c->sample_times.resize(c->n_samples);
+    }
+};
 // The sample of row `slot` of the table, by workgroups of another kernel.
 template <class T>
 SampleArgs<T> sample_args(tf_ctx* c, bool inside, const int64_t* slot) {
@@ -3211,6 +3233,7 @@ void run_gfdtd(tf_ctx* c, int64_t first, int64_t n, const tf_cg_opts* cg, tf_sta
     const bool inside = mine && plan_samples(c, n, [&](int64_t k) {
         return std::make_pair(first + k - 1, (double)(first + k) * c->dt - c->dt);
     });
+    PlanGuard plan{c, mine};
     auto pre = [&](int64_t k, GfPre& g, bool fresh, const CgState* guard) {
         const int64_t i = first + k;
         const double t = (double)i * c->dt;
@@ -3294,6 +3317,7 @@ void run_gfdtd(tf_ctx* c, int64_t first, int64_t n, const tf_cg_opts* cg, tf_sta
         // the solve of step k: the mode it needs now, its start redone if the
         // start already launched was for the other preconditioner
         const bool learned = want_learned && L.state == LearnedPc::kActive;
+        plan.k = k;
         CgSolve sol;
         sol.init = init;
         sol.learned = learned;
