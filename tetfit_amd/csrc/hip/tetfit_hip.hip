@@ -1100,8 +1100,10 @@ bool fit_grid_positions(tf_ctx* c, const tf_fit_ops& f, std::vector<uint16_t>& e
         const int sg[4] = {d, -d, d, -d};
         return (uint16_t)(m << 8 | code4(sg));  // (m is never 0: a permutation)
     };
+    // (on one thread where starting others costs more: a few 100,000 entities)
+    const int64_t chunk = E < (1 << 19) ? E : 65536;
     ecode.assign(E, 0);
-    par_chunks(f.n_common, 65536, [&](int64_t lo, int64_t hi) {
+    par_chunks(f.n_common, chunk, [&](int64_t lo, int64_t hi) {
         for (int64_t q = lo; q < hi && !bad; ++q) {
             const int32_t e = f.common_edges[q];
             int32_t slot[4];
@@ -1116,7 +1118,7 @@ bool fit_grid_positions(tf_ctx* c, const tf_fit_ops& f, std::vector<uint16_t>& e
         }
     });
     fcode.assign(F, 0);
-    par_chunks(f.n_tbc, 65536, [&](int64_t lo, int64_t hi) {
+    par_chunks(f.n_tbc, chunk, [&](int64_t lo, int64_t hi) {
         for (int64_t q = lo; q < hi && !bad; ++q) {
             const int32_t fi = f.tbc_faces[q];
             int32_t slot[4];
@@ -2106,12 +2108,14 @@ void fit_indexed_step(tf_ctx* c, const FitSpecial& sp, int sp_blocks, const doub
                  c->fh_cn.as<T>(), c->fh_e4.as<int4>(), c->U.as<T>(), c->Fv.as<T>(), c->B.as<T>(), c->dt);
 }
 
-// Items per thread of the grid-order kernels. Two (against one) took 12.1
-// instead of 12.4 us a step at 64^3 fp64, 22.5 instead of 24.7 at 90^3 and 163
-// instead of 185 at 161^3 random fp64; four gain only where an item's loads are
-// 4 bytes and the grid is large: 128^3 fp32 33.1 against 35.3 us, 161^3 fp64
-// 168 against 163, 48^3 fp32 8.7 against 8.3. Below about 17^3 the step is one
-// workgroup's latency: 16^3 fp64 6.6 us with one item, 6.7 with two.
+// Items per thread of the grid-order kernels. Small grids are a workgroup's
+// latency, which grows with its items; from about 2^19 edges on fewer, longer
+// workgroups win. A step with one / two, us: fp32 28^3 6.97 / 7.07, 40^3 7.76 /
+// 7.90, 56^3 (546,000 edges) 9.31 / 9.18, 64^3 10.5 / 10.0, 72^3 12.7 / 11.0;
+// fp64 36^3 7.68 / 7.91, 52^3 9.65 / 9.78, 72^3 15.0 / 14.2, 161^3 random 185 /
+// 163. Four gain only where an item's loads are 4 bytes and the grid is large:
+// 128^3 fp32 33.1 against 35.3 with two, 161^3 fp64 168 against 163, 48^3 fp32
+// 8.7 against 8.3.
 // $TETFIT_FIT_ITEMS (1, 2 or 4) overrides, to exercise each on small grids.
 template <class T>
 int fit_items(int64_t edges) {
@@ -2119,7 +2123,7 @@ int fit_items(int64_t edges) {
         const int n = std::atoi(v);
         if (n == 1 || n == 2 || (n == 4 && sizeof(T) == 4)) return n;
     }
-    return edges < (1 << 16) ? 1 : sizeof(T) == 4 && edges >= (1 << 22) ? 4 : 2;
+    return edges < (1 << 19) ? 1 : sizeof(T) == 4 && edges >= (1 << 22) ? 4 : 2;
 }
 // Whether plain coefficients, read once a step, are loaded non-temporally:
 // when a step's arrays exceed the 256 MB Infinity Cache they would push the
