@@ -1040,11 +1040,11 @@ __global__ void __launch_bounds__(kBlock) gf_inject_kernel(
 // the same order), and the other way round. The permutation and the conversion
 // run here, bound by the gather (161^3 fp64, 300 MB: 1 ms), so that the host
 // only receives the bytes.
-template <typename T>
+template <typename T, typename O>
 __global__ void __launch_bounds__(kBlock) state_gather_kernel(int64_t n, const int32_t* __restrict__ pos,
-                                                              const T* __restrict__ x, double* __restrict__ out) {
+                                                              const T* __restrict__ x, O* __restrict__ out) {
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (i < n) out[i] = (double)x[pos ? pos[i] : i];
+    if (i < n) out[i] = (O)x[pos ? pos[i] : i];
 }
 template <typename T>
 __global__ void __launch_bounds__(kBlock) state_scatter_kernel(int64_t n, const int32_t* __restrict__ pos,

@@ -3466,6 +3466,9 @@ tf_status guarded(F f) {
 // MB a chunk: 161^3 fp64, 101 MB a field, 10 ms into fresh memory, 33 ms when
 // the host permuted; half or an eighth of it 0-10% slower).
 constexpr int64_t kStage = 1 << 20;
+// An fp32 field of at most this many values crosses as fp32 and widens on the
+// host: half the bytes, and the host's pass stays in its cache.
+constexpr int64_t kSmallRead = 1 << 18;
 double* stage_buffer(tf_ctx* c, int64_t n) {
     const size_t need = (size_t)std::min(n, kStage) * sizeof(double);
     if (c->stage.bytes < need) c->stage.alloc(need);
@@ -3480,12 +3483,25 @@ void read_field(tf_ctx* c, const DevBuf& b, const int32_t* pos, int64_t off, int
         return;
     }
     double* st = stage_buffer(c, n);
+    if (!f64 && n <= kSmallRead) {
+        float* sf = b.as<float>() + off;
+        if (pos) {
+            sf = reinterpret_cast<float*>(st);
+            state_gather_kernel<<<blocks_for(n), kBlock, 0, c->stream>>>(n, pos + off, b.as<float>(), sf);
+            TF_HIP(hipGetLastError());
+        }
+        TF_HIP(hipStreamSynchronize(c->stream));
+        std::vector<float> h(n);
+        TF_HIP(hipMemcpy(h.data(), sf, n * sizeof(float), hipMemcpyDeviceToHost));
+        std::copy(h.begin(), h.end(), dst);
+        return;
+    }
     for (int64_t k = 0; k < n; k += kStage) {
         const int64_t m = std::min(kStage, n - k);
         const int32_t* p = pos ? pos + off + k : nullptr;
         const int64_t o = pos ? 0 : off + k;
-        if (f64) state_gather_kernel<double><<<blocks_for(m), kBlock, 0, c->stream>>>(m, p, b.as<double>() + o, st);
-        else state_gather_kernel<float><<<blocks_for(m), kBlock, 0, c->stream>>>(m, p, b.as<float>() + o, st);
+        if (f64) state_gather_kernel<<<blocks_for(m), kBlock, 0, c->stream>>>(m, p, b.as<double>() + o, st);
+        else state_gather_kernel<<<blocks_for(m), kBlock, 0, c->stream>>>(m, p, b.as<float>() + o, st);
         TF_HIP(hipGetLastError());
         // (a synchronous copy: on the context's own stream the runtime set up
         // its staging once more per context, 10 ms on the first read)
