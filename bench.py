@@ -230,16 +230,27 @@ def batch_workload(d, count=256, steps=2000, seed=4, workers=16, method="dga"):
 
 
 def fit_bytes(b, kernel, vb, grid_order=True):
-    """Algorithmic bytes per launch of the FIT kernels on a medium of few
-    distinct coefficients. Grid order: E phase reads U and the 2-byte id,
-    writes U, gathers F once; H phase reads F and the id, writes F, gathers U
-    once (B is stored on probed faces and at the end of a run only). Index
+    """Algorithmic bytes per launch of the FIT kernels. Grid order: E phase
+    reads U and the 2-byte id, writes U, gathers F once; H phase reads F and the
+    id, writes F, gathers U once (B is stored on probed faces and at the end of
+    a run only); a side with more than 511 distinct coefficient pairs (judged on
+    up to 2^20 of its entities) also reads its two coefficient arrays. Index
     tables: 17 bytes of faces or edges and signs and the two coefficients
     besides, and H reads and writes B each step."""
+    import numpy as np
     E, F = b.n_edges, b.n_faces
-    if kernel == "fit_e_kernel":
-        return E * (2 * vb + 2 if grid_order else 4 * vb + 17) + F * vb
-    return F * (2 * vb + 2 if grid_order else 5 * vb + 17) + E * vb
+    side_e = kernel == "fit_e_kernel"
+    if not grid_order:
+        return E * (4 * vb + 17) + F * vb if side_e else F * (5 * vb + 17) + E * vb
+    o = b.fit_ops()
+    at = o["common_edges"] if side_e else o["tbc_faces"]
+    at = at[::max(1, len(at) >> 20)]
+    if side_e:
+        pair = np.stack([o["upml"][at] ** 2 * o["M_h"][at] * o["M_q"][at], o["upml"][at] ** 3 * o["M_h"][at]])
+    else:
+        pair = np.stack([o["M_mu"][at] * o["fpml"][at], o["fpml"][at] * o["M_nu"][at]])
+    item = 2 * vb + 2 + (2 * vb if len(np.unique(pair, axis=1).T) > 511 else 0)
+    return E * item + F * vb if side_e else F * item + E * vb
 
 
 def run_chunks(sim, steps, chunk, label, precond="jacobi", learn_steps=200, stop_before_last=False, guess=0):

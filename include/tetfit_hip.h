@@ -189,7 +189,8 @@ tf_status tf_set_profiling(tf_ctx* ctx, int32_t on);
 
 /* fdtd and dga contexts step in HIP graphs when no launch depends on the host
  * (no energy output, no profiling; probe samples are taken by the steps' own
- * kernels): 64 steps of launches are captured once and replayed; on (default) or off (every step launched from the host).
+ * kernels): 64 steps of launches are captured once and replayed; on (default)
+ * or off (every step launched from the host).
  * Results are identical either way. No reference counterpart. */
 tf_status tf_set_graphs(tf_ctx* ctx, int32_t on);
 
@@ -207,14 +208,18 @@ tf_status tf_destroy(tf_ctx* ctx);
  * summed by one lane in entry order for each choice, so explicit fields are
  * identical; the CG's dot products are summed per workgroup, so a different
  * grid changes their rounding (gfdtd / fem fields agree to rounding). Choices are cached per (kernel, precision, rows, entries) in the
- * process and in the file named by $TETFIT_TUNE_CACHE if set. No reference
+ * process and in the file named by $TETFIT_TUNE_CACHE if set. Jacobi solves of
+ * a single system of at most 4 MB of CG rows (4 values per free edge) run one
+ * launch per pass, which has one shape; cg_w's choice then serves only the
+ * collection solves of the learned preconditioner. No reference
  * counterpart. tf_get_tuning reports the choice per kernel (order:
  * sell_ct, sell_h, sell_n, cg_w, cg_pg, cg_wu; blocks 0 = default). */
 tf_status tf_autotune(tf_ctx* ctx);
 tf_status tf_get_tuning(tf_ctx* ctx, int32_t* blocks, int32_t* unroll, int32_t* band, int32_t cap, int32_t* n);
 /* Sets the launch shape of the first n kernels in tf_get_tuning's order
  * (blocks 0 = default grid; unroll 4, 8 or 16; band 0 or 1, null = all 0),
- * e.g. to replay a choice. */
+ * e.g. to replay a choice. A kernel that the context does not run keeps its
+ * shape without effect. */
 tf_status tf_set_tuning(tf_ctx* ctx, const int32_t* blocks, const int32_t* unroll, const int32_t* band,
                         int32_t n);
 

@@ -793,8 +793,8 @@ __global__ void __launch_bounds__(kBlock) cg_w_kernel(int32_t it, SellView<T> m,
 // of gamma, delta and ||r||^2 of pass it + 1. it = -1 starts a solve: w_0 = A u_0
 // from r_0. The first batch of entries and quadruples is loaded before the
 // scalars are reduced. Iterates are those of cg_w / cg_upd.
-// 16^3 fp64: 7.9 us a pass against 6.5 + 4.7, the step 331 -> 265 us; 32^3 fp32
-// 11.6 against 7.6 + 6.5, 432 -> 364 us. A gathered row is four values instead
+// 16^3 fp64: 7.9 us a pass against 6.5 + 4.7, the step 352 -> 254 us; 32^3 fp32
+// 11.6 against 7.6 + 6.5, 429 -> 339 us. A gathered row is four values instead
 // of one, so it loses once the rows leave an XCD's 4 MB L2: 32^3 fp64 (7.1 MB)
 // 538 -> 625 us. Twelve entries a batch spill the gain (16^3 fp64 302 us).
 template <typename T>

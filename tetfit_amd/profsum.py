@@ -39,7 +39,8 @@ def _one(directory, suffix):
 
 
 def _short(name):
-    return name.split("(")[0].replace("void ", "")
+    # template arguments of an enum type print as casts: (ns::Enum)1
+    return re.sub(r"\((?:\w+::)*\w+\)(?=\d)", "", name).split("(")[0].replace("void ", "")
 
 
 def trace_stats(directory, min_us=5.0, match=None):
