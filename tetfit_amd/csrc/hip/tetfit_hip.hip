@@ -1078,14 +1078,15 @@ bool fit_grid_positions(tf_ctx* c, const tf_fit_ops& f, std::vector<uint16_t>& e
     std::atomic<bool> bad{false}, coded{false};
     constexpr uint32_t kMesher = 0 | 2 << 2 | 3 << 4 | 1 << 6;
     const int plus[4] = {1, -1, 1, -1}, minus[4] = {-1, 1, -1, 1};
-    const uint16_t mesher[2] = {(uint16_t)(kMesher << 8 | code4(minus)), (uint16_t)(kMesher << 8 | code4(plus))};
+    const std::array<uint16_t, 2> mesher{(uint16_t)(kMesher << 8 | code4(minus)), (uint16_t)(kMesher << 8 | code4(plus))};
     // the code of an entity whose sum runs over the positions `ref` with signs
-    // d, -d, d, -d; 0: they are not its slots
-    auto code_of = [&](const int32_t slot[4], const int64_t ref[4], int d, double dir_sign) -> uint16_t {
+    // d, -d, d, -d; 0: they are not its slots. other: not the mesher's order or
+    // not its direction's sign
+    auto code_of = [mesher](const int32_t slot[4], const int32_t ref[4], int d, double dir_sign, bool& other) -> uint16_t {
         if (ref[0] == slot[0] && ref[1] == slot[2] && ref[2] == slot[3] && ref[3] == slot[1] && dir_sign == d &&
             (d == 1 || d == -1))
             return mesher[d > 0];
-        coded = true;
+        other = true;
         uint32_t m = 0;
         for (int q = 0; q < 4; ++q) {
             int hit = -1;
@@ -1100,33 +1101,55 @@ bool fit_grid_positions(tf_ctx* c, const tf_fit_ops& f, std::vector<uint16_t>& e
         const int sg[4] = {d, -d, d, -d};
         return (uint16_t)(m << 8 | code4(sg));  // (m is never 0: a permutation)
     };
-    // (on one thread where starting others costs more: a few 100,000 entities)
-    const int64_t chunk = E < (1 << 19) ? E : 65536;
+    // (on one thread where starting others costs more: 40^3 2.7 ms against 1;
+    // the loops work on copies, which nothing they write can alias)
+    const int64_t chunk = E < (1 << 18) ? E : 65536;
     ecode.assign(E, 0);
     par_chunks(f.n_common, chunk, [&](int64_t lo, int64_t hi) {
-        for (int64_t q = lo; q < hi && !bad; ++q) {
-            const int32_t e = f.common_edges[q];
-            int32_t slot[4];
-            int64_t ref[4];
+        const FitGrid gl = g;
+        const tf_fit_ops o = f;
+        const int32_t *const es_at = esid.data(), *const fs_at = fsid.data();
+        uint16_t* const out = ecode.data();
+        const double sign[3] = {es[0], es[1], es[2]};
+        const int32_t o1 = (int32_t)eoff[0], o2 = (int32_t)eoff[1];
+        bool ok = true, other = false;
+        for (int64_t q = lo; q < hi && ok; ++q) {
+            const int32_t e = o.common_edges[q], at = es_at[e];
+            const int64_t b = o.ct_ptr[e];
+            int32_t slot[4], ref[4];
             // (the wrapped slots of a boundary edge can be other faces' positions)
-            if (f.ct_ptr[e + 1] - f.ct_ptr[e] != 4 || !fit_edge_slots(g, (uint32_t)esid[e], slot)) {
-                bad = true;
-                return;
+            if (o.ct_ptr[e + 1] - b != 4 || !fit_edge_slots(gl, (uint32_t)at, slot)) {
+                ok = false;
+                break;
             }
-            for (int k = 0; k < 4; ++k) ref[k] = fsid[f.ct_face[f.ct_ptr[e] + k]];
-            if (!(ecode[esid[e]] = code_of(slot, ref, f.dual_curl[e], es[edge_dir(e)]))) bad = true;
+            for (int k = 0; k < 4; ++k) ref[k] = fs_at[o.ct_face[b + k]];
+            const uint16_t code = code_of(slot, ref, o.dual_curl[e], sign[(at >= o1) + (at >= o2)], other);
+            out[at] = code;
+            ok = code != 0;
         }
+        if (!ok) bad = true;
+        if (other) coded = true;
     });
     fcode.assign(F, 0);
     par_chunks(f.n_tbc, chunk, [&](int64_t lo, int64_t hi) {
-        for (int64_t q = lo; q < hi && !bad; ++q) {
-            const int32_t fi = f.tbc_faces[q];
-            int32_t slot[4];
-            int64_t ref[4];
-            fit_face_slots(g, (uint32_t)fsid[fi], slot);
-            for (int k = 0; k < 4; ++k) ref[k] = esid[f.c_edge[4 * (int64_t)fi + k]];
-            if (!(fcode[fsid[fi]] = code_of(slot, ref, f.curl[fi], fs[face_dir(fi)]))) bad = true;
+        const FitGrid gl = g;
+        const tf_fit_ops o = f;
+        const int32_t *const es_at = esid.data(), *const fs_at = fsid.data();
+        uint16_t* const out = fcode.data();
+        const double sign[3] = {fs[0], fs[1], fs[2]};
+        const int32_t o1 = (int32_t)foff[0], o2 = (int32_t)foff[1];
+        bool ok = !bad, other = false;
+        for (int64_t q = lo; q < hi && ok; ++q) {
+            const int32_t fi = o.tbc_faces[q], at = fs_at[fi];
+            int32_t slot[4], ref[4];
+            fit_face_slots(gl, (uint32_t)at, slot);
+            for (int k = 0; k < 4; ++k) ref[k] = es_at[o.c_edge[4 * (int64_t)fi + k]];
+            const uint16_t code = code_of(slot, ref, o.curl[fi], sign[(at >= o1) + (at >= o2)], other);
+            out[at] = code;
+            ok = code != 0;
         }
+        if (!ok) bad = true;
+        if (other) coded = true;
     });
     if (bad) return false;
     c->fit_coded = coded;
